@@ -5,13 +5,27 @@
 //
 // Exact sequential semantics in parallel: seed s only reads and writes the
 // (2 ncut + 1)^3 cells around its cell, so two seeds whose cubes do not
-// intersect commute.  Each round marks, per 8^3 block, the earliest
-// unprocessed live seed; a seed whose neighbourhood of blocks holds no
-// earlier unprocessed live seed runs in this round.  Rounds repeat until
-// every seed up to npart_new is processed or dead.  Per-seed arithmetic is
-// FP64 on the float32 positions scaled by nx, as in the reference.
+// intersect commute.  Each round marks, per small block of cells, the
+// earliest unprocessed live seed; a seed runs in this round when no earlier
+// unprocessed live seed lies in the blocks within 2 ncut cells of it.
+// Rounds repeat until every seed up to npart_new is processed or dead.
+// Per-seed arithmetic is FP64 on the float32 positions scaled by nx, as in
+// the reference.
+//
+// A round has few ready seeds (tens on a 128^3 catalogue), and the largest
+// of them holds almost all of its work, so a round is a chain of launches
+// that each spread one step over the GPU: gather (one workgroup per seed),
+// centre search (64 candidates per workgroup), growth (one workgroup per
+// seed, keys sorted in LDS).  One workgroup per seed for everything took
+// 5.2 ms a round, 353 ms for the 66 rounds of the 128^3 catalogue: FP64
+// square roots and divisions of every candidate pair on one CU, then a
+// bitonic sort of all gathered particles in global memory.  The staged
+// rounds take 7.8 ms with the transfers; what is left is the chain of six
+// short launches per round.
+#include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <numeric>
 #include <vector>
 
 #include "sod_common.h"
@@ -20,27 +34,70 @@ int psod_fill_i32(psod_ctx *c, int32_t *p, int64_t n, int32_t v);
 
 namespace {
 
-constexpr int GT = 256;
-constexpr int64_t GCAP = 1 << 18;  // gathered particles per workgroup slice
+constexpr int64_t GCAP = 1 << 18;  // gathered particles per seed, at most
+// particles gathered in one round, at most: a ready seed that does not fit
+// waits for the next round (one seed always fits)
+constexpr int64_t GPOOL = (int64_t)1 << 25;
+constexpr int64_t GWIN = 1 << 16;  // seeds looked at per round
+constexpr int GROUNDS = 8;         // rounds queued before the host looks (even)
 
 struct GreedyCfg {
-  int32_t nx, ncut, nbins, nb;
+  int32_t nx, ncut, nbins;
+  int32_t bsh, nb;  // marking blocks of 2^bsh cells per side, nb per axis
   double seuil, seuil2, mmin, lr0, lr1, rmaxf;
   int64_t nsel;
 };
 
-struct GEntry {   // one gathered particle
-  double x, y, z;  // scaled position relative to the seed cell origin
-  int32_t slot, idx;
-  int32_t off;     // Chebyshev offset of its cell from the seed cell
-  int32_t rank;    // candidate order: walk rank of its cell (3^3) or -1
+// Progress of the rounds, on the device.  Entries [2] alternate between
+// rounds: a round of parity p resets its own entries in k_mark and reads
+// the window start that the round before left in first[1 - p].
+struct GState {
+  unsigned long long fail;       // smallest (seed order << 8 | code), or ~0
+  unsigned long long cursor[2];  // pool entries handed out
+  int32_t first[2];              // first unprocessed seed order
+  int32_t nready[2], nunits[2];
+  int32_t total, nrec;           // ready seeds so far, records so far
+};
+enum { GF_NSEL = 1, GF_GCAP = 2, GF_UNCLOSED = 3 };
+
+// One ready seed of a round: its pool entries [off, off + n1), of which the
+// first nnear / ncand entries of the near / candidate lists are set; its
+// centre-search units [unit0, unit0 + ceil(ncand / 64)); n1 = 0: nothing to
+// do this round.
+struct GInfo {
+  int64_t off;
+  int32_t n1, nnear, ncand, unit0;
+  unsigned long long best;  // largest lower bound of S, as double bits
+};
+
+// Pool arrays, one entry per gathered particle
+struct GPoolPtrs {
+  float4 *p;       // block-relative position, particle index
+  int32_t *slot;   // its place in cell order
+  int32_t *cell;   // offset of its cell from the seed cell, 10 bits per axis
+  float4 *near;    // within 2 cells: position relative to the seed cell,
+                   // place in p
+  int32_t *cand;   // within 1 cell: place in near
+  double *upper;   // per candidate: bound of its S
+  uint64_t *d2;    // squared distance from the centre (double bits)
+  uint64_t *key;   // sort area: d2 bits and place in p
+  uint32_t *ord;
 };
 
 struct GRec {
-  int64_t ipart, seed, centre, iamas, masse, masse2, npart_sel;
+  int64_t ipart, seed, centre, iamas, masse, masse2;
   double amass, xc, yc, zc, rayon, overdens, overdens2;
-  int32_t accepted, status;
+  int32_t accepted, pad;
 };
+
+__device__ inline int32_t pack_off(int di, int dj, int dk) {
+  return (di + 511) | ((dj + 511) << 10) | ((dk + 511) << 20);
+}
+__device__ inline void unpack_off(int32_t v, int *o) {
+  o[0] = (v & 1023) - 511;
+  o[1] = ((v >> 10) & 1023) - 511;
+  o[2] = (v >> 20) - 511;
+}
 
 __global__ void k_inverse_perm(const int32_t *__restrict__ perm, int64_t n,
                                int32_t *__restrict__ slot_of) {
@@ -54,351 +111,803 @@ __global__ void k_set_u8(uint8_t *__restrict__ p, int64_t n, uint8_t v) {
     p[i] = v;
 }
 
-// per block: smallest order of an unprocessed live seed in [lo, hi)
-__global__ void k_mark_blocks(GreedyCfg c, const int32_t *__restrict__ seeds,
-                              const int32_t *__restrict__ slot_of,
-                              const float *__restrict__ pos,
-                              const uint8_t *__restrict__ alive,
-                              const uint8_t *__restrict__ done, int64_t lo,
-                              int64_t hi, int32_t *__restrict__ bmin) {
+__device__ inline void seed_cell(const float *pos, int32_t s, int32_t nx,
+                                 int32_t *cs) {
+  for (int d = 0; d < 3; d++) {
+    float f;
+    split_coord(pos[3 * (int64_t)s + d], nx, &cs[d], &f);
+  }
+}
+
+// per block: smallest order of an unprocessed live seed of the window
+__global__ void __launch_bounds__(256)
+k_mark(GreedyCfg c, const int32_t *__restrict__ isort,
+       const int32_t *__restrict__ slot_of, const float *__restrict__ pos,
+       const uint8_t *__restrict__ alive, const uint8_t *__restrict__ done,
+       int32_t npart_new, int par, GState *__restrict__ S,
+       int32_t *__restrict__ bmin) {
+  const int32_t lo = S->first[1 - par];
+  const int32_t hi = (int32_t)min((int64_t)npart_new, lo + GWIN);
   const int64_t o = lo + (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (o >= hi || done[o]) return;
-  const int32_t s = seeds[o];
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    S->total += S->nready[1 - par];
+    S->first[par] = hi;
+    S->nready[par] = 0;
+    S->nunits[par] = 0;
+    S->cursor[par] = 0;
+  }
+  if (o >= hi || done[o] || S->fail != ~0ull) return;
+  const int32_t s = isort[o] - 1;
   if (!alive[slot_of[s]]) return;
   int32_t b[3];
-  for (int d = 0; d < 3; d++) {
-    int32_t cc;
-    float f;
-    split_coord(pos[3 * (int64_t)s + d], c.nx, &cc, &f);
-    b[d] = cc >> 3;
-  }
-  atomicMin(&bmin[(b[2] * c.nb + b[1]) * c.nb + b[0]], (int32_t)(o - lo));
+  seed_cell(pos, s, c.nx, b);
+  for (int d = 0; d < 3; d++) b[d] >>= c.bsh;
+  atomicMin(&bmin[(b[2] * c.nb + b[1]) * c.nb + b[0]], (int32_t)o);
 }
 
-// ready seeds: live, unprocessed, and no earlier unprocessed live seed in
-// the blocks a (2ncut+1)^3 cube around either seed can reach
-__global__ void k_ready(GreedyCfg c, const int32_t *__restrict__ seeds,
-                        const int32_t *__restrict__ slot_of,
-                        const float *__restrict__ pos,
-                        const uint8_t *__restrict__ alive,
-                        uint8_t *__restrict__ done, int64_t lo, int64_t hi,
-                        const int32_t *__restrict__ bmin,
-                        int32_t *__restrict__ ready,
-                        int32_t *__restrict__ nready) {
+// Ready seeds: live, unprocessed, and no earlier unprocessed live seed in
+// the blocks within 2 ncut cells (cubes intersect only if the seed cells
+// are at most 2 ncut apart).  Also the first unprocessed seed, the start of
+// the next round's window (seeds that run in this round count as
+// unprocessed until the next).
+__global__ void __launch_bounds__(256)
+k_ready(GreedyCfg c, const int32_t *__restrict__ isort,
+        const int32_t *__restrict__ slot_of, const float *__restrict__ pos,
+        const uint8_t *__restrict__ alive, uint8_t *__restrict__ done,
+        int32_t npart_new, int par, GState *__restrict__ S,
+        const int32_t *__restrict__ bmin, int32_t *__restrict__ ready) {
+  const int32_t lo = S->first[1 - par];
+  const int32_t hi = (int32_t)min((int64_t)npart_new, lo + GWIN);
   const int64_t o = lo + (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (o >= hi || done[o]) return;
-  const int32_t s = seeds[o];
-  if (!alive[slot_of[s]]) {  // captured earlier: nothing to do (:1628)
-    done[o] = 1;
-    return;
-  }
-  int32_t b[3];
-  for (int d = 0; d < 3; d++) {
-    int32_t cc;
-    float f;
-    split_coord(pos[3 * (int64_t)s + d], c.nx, &cc, &f);
-    b[d] = cc >> 3;
-  }
-  // cubes intersect only if the seed cells are <= 2 ncut apart
-  const int reach = (2 * c.ncut + 7) / 8 + 1;
-  const int span = min(2 * reach + 1, c.nb);
-  const int32_t me = (int32_t)(o - lo);
-  for (int i = 0; i < span; i++)
-    for (int j = 0; j < span; j++)
-      for (int k = 0; k < span; k++) {
-        const int32_t bx = wrapi(b[0] - reach + i, c.nb);
-        const int32_t by = wrapi(b[1] - reach + j, c.nb);
-        const int32_t bz = wrapi(b[2] - reach + k, c.nb);
-        if (bmin[(bz * c.nb + by) * c.nb + bx] < me) return;
+  if (S->fail != ~0ull) return;
+  int32_t open = INT32_MAX;
+  bool go = false;
+  if (o < hi && !done[o]) {
+    const int32_t s = isort[o] - 1;
+    if (!alive[slot_of[s]]) {  // captured earlier: nothing to do (:1628)
+      done[o] = 1;
+    } else {
+      open = (int32_t)o;
+      go = true;
+      int32_t cs[3], b0[3], nb[3];
+      seed_cell(pos, s, c.nx, cs);
+      for (int d = 0; d < 3; d++) {
+        b0[d] = (cs[d] - 2 * c.ncut) >> c.bsh;
+        nb[d] = min(((cs[d] + 2 * c.ncut) >> c.bsh) - b0[d] + 1, c.nb);
       }
-  ready[atomicAdd(nready, 1)] = me;  // relative to the window start lo
+      for (int i = 0; i < nb[2] && go; i++)
+        for (int j = 0; j < nb[1] && go; j++) {
+          const int32_t row = (wrapi(b0[2] + i, c.nb) * c.nb +
+                               wrapi(b0[1] + j, c.nb)) * c.nb;
+          for (int k = 0; k < nb[0]; k++)
+            go = go && bmin[row + wrapi(b0[0] + k, c.nb)] >= open;
+        }
+    }
+  }
+  const int l = threadIdx.x & 63;
+  const uint64_t mo = __ballot(open != INT32_MAX);
+  if (mo && l == __ffsll((unsigned long long)mo) - 1)
+    atomicMin(&S->first[par], open);  // orders ascend with the lane
+  const uint64_t m = __ballot(go);
+  int32_t base = 0;
+  if (l == 0 && m) base = atomicAdd(&S->nready[par], (int32_t)__popcll(m));
+  base = __shfl(base, 0, 64);
+  if (go)
+    ready[base + __popcll(m & (l == 0 ? 0ull : (~0ull >> (64 - l))))] = open;
 }
 
-struct GShared {
-  int32_t cnt, ncand;
-  int64_t red_l[GT / 64];
-  double red_d[GT / 64];
-  int64_t bk[GT / 64];
-  double bs[GT / 64];
-  int32_t item;
+constexpr int GA_T = 1024;  // threads of a gather workgroup
+
+// exclusive prefix of v over the GA_T threads; *tot the sum
+__device__ inline int32_t ga_scan(int32_t v, int32_t *wsum, int32_t *tot) {
+  const int w = threadIdx.x >> 6;
+  const int32_t inc = wave_incl_scan(v);
+  __syncthreads();
+  if ((threadIdx.x & 63) == 63) wsum[w] = inc;
+  __syncthreads();
+  int32_t off = 0, t = 0;
+  for (int i = 0; i < GA_T / 64; i++) {
+    if (i < w) off += wsum[i];
+    t += wsum[i];
+  }
+  *tot = t;
+  return off + inc - v;
+}
+
+// S1: live particles of the (2ncut+1)^3 cells of each ready seed in walk
+// order, x outermost (main file:1658-1716): the gathered list keeps the
+// reference's order, which decides exact ties.  One workgroup per seed: the
+// cells' ranges GA_T at a time, their records in flat order (a lane per
+// record: a thread per cell walked a dense cell's thousands of records
+// alone), ranks from ballots.
+__global__ void __launch_bounds__(GA_T)
+k_greedy_gather(GreedyCfg c, const int32_t *__restrict__ isort,
+                const int32_t *__restrict__ cell_start,
+                const float4 *__restrict__ rec, const float *__restrict__ pos,
+                const uint8_t *__restrict__ alive, uint8_t *__restrict__ done,
+                int par, GState *__restrict__ S,
+                const int32_t *__restrict__ ready, GInfo *__restrict__ info,
+                int2 *__restrict__ units, GPoolPtrs G, int64_t pcap) {
+  __shared__ int32_t pre[GA_T + 1], st[GA_T], wsum[GA_T / 64];
+  __shared__ int32_t wc[GA_T / 64][3];
+  __shared__ long long soff;
+  const int32_t nr = S->nready[par];
+  const int side = 2 * c.ncut + 1;
+  const int32_t ncell = side * side * side;
+  const int l = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const uint64_t below = l == 0 ? 0ull : (~0ull >> (64 - l));
+  for (int32_t it = blockIdx.x; it < nr; it += gridDim.x) {
+    const int32_t o = ready[it];
+    int32_t cs[3];
+    seed_cell(pos, isort[o] - 1, c.nx, cs);
+    // pool entries: every particle of the cells, a power of two (the sort's
+    // padding)
+    int64_t all = 0;
+    for (int32_t base = 0; base < ncell; base += GA_T) {
+      const int32_t q = base + threadIdx.x;
+      int32_t n = 0, a = 0;
+      if (q < ncell) {
+        int di, dj, dk;
+        int32_t lc[3];
+        walk_off(q, c.ncut, &di, &dj, &dk);
+        const int32_t key = key_at(c.nx, cs, di, dj, dk, lc);
+        a = cell_start[key];
+        n = cell_start[key + 1] - a;
+      }
+      int32_t tot;
+      const int32_t ex = ga_scan(n, wsum, &tot);
+      pre[threadIdx.x] = ex;  // kept when there is one batch of cells
+      st[threadIdx.x] = a;
+      if (threadIdx.x == 0) pre[GA_T] = tot;
+      all += tot;
+    }
+    int64_t cap = 64;
+    while (cap < all && cap < GCAP) cap <<= 1;
+    if (threadIdx.x == 0) {
+      const long long off = (long long)atomicAdd(&S->cursor[par],
+                                                 (unsigned long long)cap);
+      soff = off + cap <= pcap ? off : -1;
+    }
+    __syncthreads();
+    const int64_t off = soff;
+    GInfo gi;
+    gi.off = off;
+    gi.n1 = gi.nnear = gi.ncand = gi.unit0 = 0;
+    gi.best = 0;
+    if (off < 0) {  // the pool is full: next round
+      if (threadIdx.x == 0) info[it] = gi;
+      __syncthreads();
+      continue;
+    }
+    int64_t n1 = 0;
+    int32_t nnear = 0, ncand = 0;
+    for (int32_t base = 0; base < ncell; base += GA_T) {
+      if (ncell > GA_T) {
+        const int32_t q = base + threadIdx.x;
+        int32_t n = 0, a = 0;
+        if (q < ncell) {
+          int di, dj, dk;
+          int32_t lc[3];
+          walk_off(q, c.ncut, &di, &dj, &dk);
+          const int32_t key = key_at(c.nx, cs, di, dj, dk, lc);
+          a = cell_start[key];
+          n = cell_start[key + 1] - a;
+        }
+        int32_t tot;
+        const int32_t ex = ga_scan(n, wsum, &tot);
+        pre[threadIdx.x] = ex;
+        st[threadIdx.x] = a;
+        if (threadIdx.x == 0) pre[GA_T] = tot;
+      }
+      __syncthreads();
+      const int32_t tot = pre[GA_T];
+      for (int32_t j0 = 0; j0 < tot; j0 += GA_T) {
+        const int32_t j = j0 + threadIdx.x;
+        bool live = false, near = false, cand = false;
+        int di = 0, dj = 0, dk = 0;
+        int32_t k = 0;
+        if (j < tot) {
+          int lo = 0, hi = GA_T;  // last cell with pre <= j (empty cells: the
+          while (hi - lo > 1) {   // last of equal entries holds j)
+            const int mid = (lo + hi) >> 1;
+            if (pre[mid] <= j) lo = mid; else hi = mid;
+          }
+          k = st[lo] + (j - pre[lo]);
+          live = alive[k] != 0;
+          walk_off(base + lo, c.ncut, &di, &dj, &dk);
+          const int cheb = max(abs(di), max(abs(dj), abs(dk)));
+          near = live && cheb <= 2;
+          cand = live && cheb <= 1;
+        }
+        const uint64_t ml = __ballot(live), mn = __ballot(near),
+                       mc = __ballot(cand);
+        if (l == 0) {
+          wc[w][0] = __popcll(ml);
+          wc[w][1] = __popcll(mn);
+          wc[w][2] = __popcll(mc);
+        }
+        __syncthreads();
+        int32_t t0 = 0, t1 = 0, t2 = 0, e0 = 0, e1 = 0, e2 = 0;
+        for (int i = 0; i < GA_T / 64; i++) {
+          if (i == w) {
+            e0 = t0;
+            e1 = t1;
+            e2 = t2;
+          }
+          t0 += wc[i][0];
+          t1 += wc[i][1];
+          t2 += wc[i][2];
+        }
+        if (live) {
+          const int64_t e = n1 + e0 + __popcll(ml & below);
+          if (e < cap && e < c.nsel) {
+            const float4 r = rec[k];
+            G.p[off + e] = r;
+            G.slot[off + e] = k;
+            G.cell[off + e] = pack_off(di, dj, dk);
+            if (near) {
+              const int32_t en = nnear + e1 + __popcll(mn & below);
+              G.near[off + en] = make_float4(
+                  rel1(r.x, (cs[0] + di) & 7, di, 0.f),
+                  rel1(r.y, (cs[1] + dj) & 7, dj, 0.f),
+                  rel1(r.z, (cs[2] + dk) & 7, dk, 0.f),
+                  __int_as_float((int32_t)e));
+              if (cand) G.cand[off + ncand + e2 + __popcll(mc & below)] = en;
+            }
+          }
+        }
+        n1 += t0;
+        nnear += t1;
+        ncand += t2;
+        __syncthreads();
+      }
+    }
+    if (threadIdx.x == 0) {
+      if (n1 > c.nsel || n1 > GCAP) {  // "Increase Nsel" (main file:1681)
+        const int code = n1 > c.nsel ? GF_NSEL : GF_GCAP;
+        atomicMin(&S->fail, ((unsigned long long)o << 8) | code);
+      } else if (!((double)n1 >= c.mmin)) {
+        done[o] = 1;  // Mtotsel >= Mmin with unit masses (main file:1759)
+      } else {
+        gi.n1 = (int32_t)n1;
+        gi.nnear = nnear;
+        gi.ncand = ncand;
+        const int32_t ng = (ncand + 63) >> 6;
+        gi.unit0 = atomicAdd(&S->nunits[par], ng);
+        for (int32_t g = 0; g < ng; g++)
+          units[gi.unit0 + g] = make_int2(it, g);
+      }
+      info[it] = gi;
+    }
+    __syncthreads();
+  }
+}
+
+// Centre search (main file:1799-1875) in two launches.  The first bounds
+// every candidate's S in FP32: relative coordinates and their differences
+// are good to 4e-7 cells, so a term 1/sqrt(d2 + 2^-12) is good to 2.3e-5
+// and d2 to 3e-6; sums of 64 FP32 terms add at most 4e-6 and are folded in
+// FP64.  S lies between (1 - 1e-4) times the terms of d2 <= 1 - 1e-5 and
+// (1 + 1e-4) times the terms of d2 <= 1 + 1e-5.  The second launch
+// evaluates in FP64 only the candidates whose upper bound reaches the
+// largest lower bound (no other can hold or tie the maximum): a few of
+// thousands, in place of an FP64 square root and division per pair.
+// One workgroup takes 64 candidates, its 8 waves a share of the
+// neighbours each.
+constexpr int GC_T = 512;
+
+__global__ void __launch_bounds__(GC_T)
+k_greedy_bound(int par, GState *__restrict__ S, GInfo *__restrict__ info,
+               const int2 *__restrict__ units, GPoolPtrs G) {
+  __shared__ float4 tile[GC_T];
+  __shared__ double red[GC_T / 64][64][2];
+  const int l = threadIdx.x & 63,
+            w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int32_t nu = S->nunits[par];
+  for (int32_t u = blockIdx.x; u < nu; u += gridDim.x) {
+    const int2 un = units[u];
+    const GInfo gi = info[un.x];
+    const int32_t cd = un.y * 64 + l;
+    float4 p = make_float4(1e30f, 1e30f, 1e30f, 0.f);
+    if (cd < gi.ncand) p = G.near[gi.off + G.cand[gi.off + cd]];
+    double lo = 0.0, up = 0.0;
+    for (int32_t b = 0; b < gi.nnear; b += GC_T) {
+      __syncthreads();
+      const int32_t j = b + (int32_t)threadIdx.x;
+      // entries past the end lie beyond every cutoff
+      tile[threadIdx.x] = j < gi.nnear ? G.near[gi.off + j]
+                                       : make_float4(-1e30f, 0.f, 0.f, 0.f);
+      __syncthreads();
+      float sl = 0.f, su = 0.f;
+#pragma unroll 8
+      for (int i = 0; i < 64; i++) {
+        const float4 q = tile[64 * w + i];
+        const float dx = q.x - p.x, dy = q.y - p.y, dz = q.z - p.z;
+        const float d2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
+        const float t = __builtin_amdgcn_rsqf(d2 + 1.0f / 4096.0f);
+        sl += d2 <= 1.0f - 1e-5f ? t : 0.f;
+        su += d2 <= 1.0f + 1e-5f ? t : 0.f;
+      }
+      lo += (double)sl;
+      up += (double)su;
+    }
+    red[w][l][0] = lo;
+    red[w][l][1] = up;
+    __syncthreads();
+    if (w == 0) {
+      for (int i = 1; i < GC_T / 64; i++) {
+        lo += red[i][l][0];
+        up += red[i][l][1];
+      }
+      if (cd < gi.ncand) G.upper[gi.off + cd] = up * (1.0 + 1e-4);
+      unsigned long long v =
+          cd < gi.ncand ? (unsigned long long)__double_as_longlong(
+                              lo * (1.0 - 1e-4))
+                        : 0ull;
+      for (int sh = 32; sh > 0; sh >>= 1) {
+        const unsigned long long x = __shfl_xor(v, sh, 64);
+        v = x > v ? x : v;
+      }
+      if (l == 0) atomicMax(&info[un.x].best, v);
+    }
+    __syncthreads();
+  }
+}
+
+// position of pool entry e relative to the box origin (FP64)
+__device__ inline void entry_pos(const GPoolPtrs &G, int64_t e,
+                                 const int32_t *cs, double *x, int *off) {
+  const float4 r = G.p[e];
+  unpack_off(G.cell[e], off);
+  const double u[3] = {(double)r.x, (double)r.y, (double)r.z};
+  for (int d = 0; d < 3; d++)
+    x[d] = (double)cs[d] + (double)off[d] +
+           (u[d] - (double)((cs[d] + off[d]) & 7));
+}
+
+// FP64 S of the candidates left, one wave each, terms in parallel and their
+// sum in gather order (the reference's); first strict maximum in walk
+// order.  ures[u] = best (S bits, key) of unit u, key = walk rank of the
+// candidate's cell << 32 | particle index.  Also clears the marks for the
+// next round.
+__global__ void __launch_bounds__(256)
+k_greedy_centre(GreedyCfg c, const int32_t *__restrict__ isort,
+                const float *__restrict__ pos, int par,
+                const GState *__restrict__ S, const int32_t *__restrict__ ready,
+                const GInfo *__restrict__ info, const int2 *__restrict__ units,
+                GPoolPtrs G, uint64_t *__restrict__ ures,
+                int32_t *__restrict__ bmin, int32_t nbk) {
+  __shared__ uint64_t mask;
+  __shared__ double term[4][64];
+  __shared__ double ws[4];
+  __shared__ int64_t wk[4];
+  for (int32_t i = blockIdx.x * 256 + threadIdx.x; i < nbk;
+       i += gridDim.x * 256)
+    bmin[i] = INT32_MAX;
+  const int l = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const uint64_t below = l == 0 ? 0ull : (~0ull >> (64 - l));
+  const double taille = (double)c.nx;
+  const int32_t nu = S->nunits[par];
+  for (int32_t u = blockIdx.x; u < nu; u += gridDim.x) {
+    const int2 un = units[u];
+    const GInfo gi = info[un.x];
+    if (w == 0) {
+      const int32_t cd = un.y * 64 + l;
+      const bool left =
+          cd < gi.ncand &&
+          G.upper[gi.off + cd] >= __longlong_as_double((long long)gi.best);
+      const uint64_t m = __ballot(left);
+      if (l == 0) mask = m;
+    }
+    __syncthreads();
+    uint64_t todo = mask;
+    for (int i = 0; i < w && todo; i++) todo &= todo - 1;
+    double bs = 0.0;
+    int64_t bk = INT64_MAX;
+    int32_t cs[3];
+    if (todo) seed_cell(pos, isort[ready[un.x]] - 1, c.nx, cs);
+    while (todo) {  // survivors w, w + 4, ... of the unit
+      const int32_t cd = un.y * 64 + __ffsll((unsigned long long)todo) - 1;
+      const int64_t ce = gi.off + __float_as_int(
+          G.near[gi.off + G.cand[gi.off + cd]].w);
+      double pc[3];
+      int po[3];
+      entry_pos(G, ce, cs, pc, po);
+      double acc = 0.0;
+      for (int32_t b = 0; b < gi.nnear; b += 64) {
+        bool in = false;
+        double t = 0.0;
+        if (b + l < gi.nnear) {
+          double q[3], dd[3];
+          int qo[3];
+          entry_pos(G, gi.off + __float_as_int(G.near[gi.off + b + l].w), cs, q,
+                    qo);
+          for (int d = 0; d < 3; d++) {
+            dd[d] = fabs(q[d] - pc[d]);
+            dd[d] = fmin(dd[d], taille - dd[d]);
+          }
+          const double d2 = __dadd_rn(__dadd_rn(__dmul_rn(dd[0], dd[0]),
+                                                __dmul_rn(dd[1], dd[1])),
+                                      __dmul_rn(dd[2], dd[2]));
+          in = d2 <= 1.0;
+          if (in) t = 1.0 / sqrt(d2 + (1.0 / 64.0) * (1.0 / 64.0));
+        }
+        const uint64_t mi = __ballot(in);
+        if (in) term[w][__popcll(mi & below)] = t;
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        const int n = __popcll(mi);
+#pragma unroll 8
+        for (int i = 0; i < n; i++) acc += term[w][i];
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+      }
+      const int64_t rank = (po[0] + 1) * 9 + (po[1] + 1) * 3 + (po[2] + 1);
+      const int64_t key =
+          (rank << 32) | (uint32_t)__float_as_int(G.p[ce].w);
+      if (acc > bs || (acc == bs && key < bk)) {
+        bs = acc;
+        bk = key;
+      }
+      for (int i = 0; i < 4 && todo; i++) todo &= todo - 1;
+    }
+    if (l == 0) {
+      ws[w] = bs;
+      wk[w] = bk;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      for (int i = 1; i < 4; i++)
+        if (ws[i] > bs || (ws[i] == bs && wk[i] < bk)) {
+          bs = ws[i];
+          bk = wk[i];
+        }
+      ures[2 * (int64_t)u] = (uint64_t)__double_as_longlong(bs);
+      ures[2 * (int64_t)u + 1] = (uint64_t)bk;
+    }
+    __syncthreads();
+  }
+}
+
+// Growth, one workgroup per seed.  The particles that can be ranked up to
+// the crossing are sorted by (d2, gather order) in LDS: all of them when
+// they are at most GS_CAP, otherwise those of the radial bins (uniform in
+// r^3 up to ncut) up to the first one inside which a crossing is sure; only
+// seeds with more than GS_CAP of those sort in global memory (steps within
+// GS_CAP keys still in LDS).
+constexpr int GG_T = 512, GS_CAP = 8192, GS_BINS = 4096;
+
+struct GrowLds {
+  uint64_t key[GS_CAP];
+  uint32_t ord[GS_CAP];
+  int32_t hist[GS_BINS];
+  int64_t red_l[GG_T / 64];
+  double red_d[GG_T / 64];
+  int32_t n;
 };
 
-__device__ inline int64_t gmin(int64_t v, GShared &S) {
+__device__ inline int64_t gg_min(int64_t v, GrowLds &S) {
   for (int o = 32; o > 0; o >>= 1) v = min(v, (int64_t)__shfl_xor(v, o, 64));
   __syncthreads();
   if ((threadIdx.x & 63) == 0) S.red_l[threadIdx.x >> 6] = v;
   __syncthreads();
   int64_t r = S.red_l[0];
-  for (int i = 1; i < GT / 64; i++) r = min(r, S.red_l[i]);
+  for (int i = 1; i < GG_T / 64; i++) r = min(r, S.red_l[i]);
   __syncthreads();
   return r;
 }
 
-// one workgroup per ready seed, persistent over the ready list
-__global__ void __launch_bounds__(GT)
-k_greedy_seed(GreedyCfg c, const int32_t *__restrict__ seeds,
-              const int32_t *__restrict__ cell_start,
-              const float4 *__restrict__ rec, const float *__restrict__ pos,
-              const int64_t *__restrict__ ids, uint8_t *__restrict__ alive,
-              uint8_t *__restrict__ done, int64_t lo, int64_t hi,
-              const int32_t *__restrict__ ready,
-              const int32_t *__restrict__ nready,
-              int32_t *__restrict__ queue, GEntry *__restrict__ ent_all,
-              double *__restrict__ d2_all, int32_t *__restrict__ ord_all,
-              int64_t *__restrict__ structure, GRec *__restrict__ recs,
-              double *__restrict__ radb, int32_t *__restrict__ massb,
-              int32_t *__restrict__ fail) {
-  __shared__ GShared S;
-  GEntry *ent = ent_all + (int64_t)blockIdx.x * GCAP;
-  double *d2 = d2_all + (int64_t)blockIdx.x * GCAP;
-  int32_t *ord = ord_all + (int64_t)blockIdx.x * GCAP;
-  const int32_t nr = *nready;
-  const double taille = (double)c.nx;
-  for (;;) {
-    if (threadIdx.x == 0) S.item = atomicAdd(queue, 1);
-    __syncthreads();
-    const int32_t it = S.item;
-    __syncthreads();
-    if (it >= nr) break;
-    const int64_t o = lo + ready[it];
-    if (o < lo || o >= hi) continue;  // never: ready holds window offsets
-    const int32_t s = seeds[o];
-    GRec R;
-    memset(&R, 0, sizeof(R));
-    R.ipart = o + 1;
-    R.seed = s;
-    int32_t cs[3];
-    for (int d = 0; d < 3; d++) {
-      float f;
-      split_coord(pos[3 * (int64_t)s + d], c.nx, &cs[d], &f);
+// one step of the bitonic network on keys in LDS: pairs (i, i + j) of the
+// nk keys, whose place in the whole sequence starts at g0
+__device__ inline void gg_step(GrowLds &S, int32_t nk, int64_t g0, int64_t k,
+                               int32_t j) {
+  for (int32_t t = threadIdx.x; t < nk / 2; t += GG_T) {
+    const int32_t i = ((t & ~(j - 1)) << 1) | (t & (j - 1)), p = i + j;
+    const uint64_t a = S.key[i], b = S.key[p];
+    const uint32_t oa = S.ord[i], ob = S.ord[p];
+    const bool gt = a > b || (a == b && oa > ob);
+    if (gt == (((g0 + i) & k) == 0)) {
+      S.key[i] = b;
+      S.key[p] = a;
+      S.ord[i] = ob;
+      S.ord[p] = oa;
     }
-    // S1: live particles of the (2ncut+1)^3 cells, walk x outermost
-    // (main file:1658-1716)
-    if (threadIdx.x == 0) S.cnt = 0;
-    __syncthreads();
-    const int side = 2 * c.ncut + 1;
-    const int32_t ncell = side * side * side;
-    // cells are visited in walk order by one thread each, so that the
-    // gathered list keeps the reference's order (needed for exact ties)
-    for (int32_t base = 0; base < ncell; base += GT) {
-      const int32_t q = base + threadIdx.x;
-      int32_t a = 0, b = 0, lc[3] = {0, 0, 0};
-      int di = 0, dj = 0, dk = 0;
-      int32_t nlive = 0;
-      if (q < ncell) {
-        walk_off(q, c.ncut, &di, &dj, &dk);
-        const int32_t key = key_at(c.nx, cs, di, dj, dk, lc);
-        a = cell_start[key];
-        b = cell_start[key + 1];
-        for (int32_t k = a; k < b; k++) nlive += alive[k];
-      }
-      // exclusive prefix over this batch of cells
-      int32_t inc = wave_incl_scan(nlive);
-      const int w = threadIdx.x >> 6;
-      if ((threadIdx.x & 63) == 63) S.red_l[w] = inc;
-      __syncthreads();
-      int32_t off = S.cnt, tot = 0;
-      for (int i = 0; i < GT / 64; i++) {
-        if (i < w) off += (int32_t)S.red_l[i];
-        tot += (int32_t)S.red_l[i];
-      }
-      off += inc - nlive;
-      if (q < ncell) {
-        int32_t e = off;
-        for (int32_t k = a; k < b; k++) {
-          if (!alive[k]) continue;
-          if (e < GCAP && e < c.nsel) {
-            const float4 r = rec[k];
-            GEntry g;
-            g.x = (double)cs[0] + (double)di + ((double)r.x - (double)lc[0]);
-            g.y = (double)cs[1] + (double)dj + ((double)r.y - (double)lc[1]);
-            g.z = (double)cs[2] + (double)dk + ((double)r.z - (double)lc[2]);
-            g.slot = k;
-            g.idx = __float_as_int(r.w);
-            g.off = max(abs(di), max(abs(dj), abs(dk)));
-            g.rank = g.off <= 1 ? (di + 1) * 9 + (dj + 1) * 3 + (dk + 1) : -1;
-            ent[e] = g;
-          }
-          e++;
-        }
-      }
-      __syncthreads();
-      if (threadIdx.x == 0) S.cnt += tot;
-      __syncthreads();
+  }
+  __syncthreads();
+}
+
+// sorts n keys ascending by (key, ord): keys already in LDS when n <= GS_CAP,
+// else in gk / go (space for the next power of two)
+__device__ inline void gg_sort(GrowLds &S, uint64_t *gk, uint32_t *go,
+                               int32_t n) {
+  int32_t np = 64;
+  while (np < n) np <<= 1;
+  if (n <= GS_CAP) {
+    for (int32_t t = n + threadIdx.x; t < np; t += GG_T) {
+      S.key[t] = ~0ull;
+      S.ord[t] = ~0u;
     }
-    const int32_t n1 = S.cnt;
-    if (n1 > c.nsel || n1 > GCAP) {  // "Increase Nsel" (main file:1681)
-      if (threadIdx.x == 0) {
-        R.status = n1 > c.nsel ? PSOD_E_CAPACITY : -PSOD_E_CAPACITY;
-        recs[o] = R;
-        atomicMin(&fail[0], (int32_t)o);
-      }
-      __syncthreads();
-      continue;
-    }
-    __threadfence_block();
-    __syncthreads();
-    // Mtotsel >= Mmin with unit masses (main file:1759)
-    if (!((double)n1 >= c.mmin)) {
-      if (threadIdx.x == 0) done[o] = 1;
-      continue;
-    }
-    // centre search over the 3^3 candidates against S2 (offset <= 2),
-    // first strict maximum in walk order (main file:1799-1875)
-    double bs = 0.0;
-    int64_t bk = INT64_MAX;
-    for (int32_t t = threadIdx.x; t < n1; t += GT) {
-      const GEntry p = ent[t];
-      if (p.rank < 0) continue;
-      double acc = 0.0;
-      for (int32_t u = 0; u < n1; u++) {
-        const GEntry q = ent[u];
-        if (q.off > 2) continue;
-        double dx = fabs(q.x - p.x);
-        dx = fmin(dx, taille - dx);
-        double dy = fabs(q.y - p.y);
-        dy = fmin(dy, taille - dy);
-        double dz = fabs(q.z - p.z);
-        dz = fmin(dz, taille - dz);
-        const double dd = __dadd_rn(__dadd_rn(__dmul_rn(dx, dx),
-                                              __dmul_rn(dy, dy)),
-                                    __dmul_rn(dz, dz));
-        if (dd <= 1.0) acc += 1.0 / sqrt(dd + (1.0 / 64.0) * (1.0 / 64.0));
-      }
-      const int64_t key = ((int64_t)p.rank << 32) | (uint32_t)p.idx;
-      if (acc > bs || (acc == bs && key < bk)) { bs = acc; bk = key; }
-    }
-    for (int sh = 32; sh > 0; sh >>= 1) {
-      const double s2 = __shfl_xor(bs, sh, 64);
-      const int64_t k2 = __shfl_xor(bk, sh, 64);
-      if (s2 > bs || (s2 == bs && k2 < bk)) { bs = s2; bk = k2; }
-    }
-    if ((threadIdx.x & 63) == 0) {
-      S.bs[threadIdx.x >> 6] = bs;
-      S.bk[threadIdx.x >> 6] = bk;
-    }
-    __syncthreads();
-    bs = S.bs[0];
-    bk = S.bk[0];
-    for (int i = 1; i < GT / 64; i++)
-      if (S.bs[i] > bs || (S.bs[i] == bs && S.bk[i] < bk)) {
-        bs = S.bs[i];
-        bk = S.bk[i];
-      }
-    __syncthreads();
-    const int32_t centre = (int32_t)(bk & 0xFFFFFFFF);
-    double xc[3];
-    centre_scaled(pos, centre, c.nx, xc);
-    // distances (main file:2002-2020) and sort by (d2, gather order)
-    for (int32_t t = threadIdx.x; t < n1; t += GT) {
-      const GEntry p = ent[t];
-      double dx = fabs((double)(pos[3 * (int64_t)p.idx] * (float)c.nx) - xc[0]);
-      dx = fmin(dx, taille - dx);
-      double dy = fabs((double)(pos[3 * (int64_t)p.idx + 1] * (float)c.nx) - xc[1]);
-      dy = fmin(dy, taille - dy);
-      double dz = fabs((double)(pos[3 * (int64_t)p.idx + 2] * (float)c.nx) - xc[2]);
-      dz = fmin(dz, taille - dz);
-      d2[t] = __dadd_rn(__dadd_rn(__dmul_rn(dx, dx), __dmul_rn(dy, dy)),
-                        __dmul_rn(dz, dz));
-      ord[t] = t;
-    }
-    int32_t np = 1;
-    while (np < n1) np <<= 1;
-    for (int32_t t = n1 + threadIdx.x; t < np; t += GT) {
-      d2[t] = INFINITY;
-      ord[t] = INT32_MAX;
-    }
-    __threadfence_block();
     __syncthreads();
     for (int32_t k = 2; k <= np; k <<= 1)
-      for (int32_t j = k >> 1; j > 0; j >>= 1) {
-        for (int32_t i = threadIdx.x; i < np; i += GT) {
-          const int32_t p = i ^ j;
-          if (p > i) {
-            const double a = d2[i], b = d2[p];
-            const int32_t ia = ord[i], ib = ord[p];
-            const bool gt = a > b || (a == b && ia > ib);
-            if (gt == ((i & k) == 0)) {
-              d2[i] = b; d2[p] = a; ord[i] = ib; ord[p] = ia;
-            }
+      for (int32_t j = k >> 1; j > 0; j >>= 1) gg_step(S, np, 0, k, j);
+    return;
+  }
+  for (int32_t t = n + threadIdx.x; t < np; t += GG_T) {
+    gk[t] = ~0ull;
+    go[t] = ~0u;
+  }
+  __threadfence_block();
+  __syncthreads();
+  // stages k <= GS_CAP and the steps j < GS_CAP of later stages, block by
+  // block in LDS
+  for (int64_t k = GS_CAP; k <= np; k <<= 1) {
+    for (int32_t j = (int32_t)(k >> 1); j >= GS_CAP; j >>= 1) {
+      for (int32_t t = threadIdx.x; t < np / 2; t += GG_T) {
+        const int32_t i = ((t & ~(j - 1)) << 1) | (t & (j - 1)), p = i + j;
+        const uint64_t a = gk[i], b = gk[p];
+        const uint32_t oa = go[i], ob = go[p];
+        const bool gt = a > b || (a == b && oa > ob);
+        if (gt == ((i & k) == 0)) {
+          gk[i] = b;
+          gk[p] = a;
+          go[i] = ob;
+          go[p] = oa;
+        }
+      }
+      __threadfence_block();
+      __syncthreads();
+    }
+    for (int32_t g0 = 0; g0 < np; g0 += GS_CAP) {
+      for (int32_t t = threadIdx.x; t < GS_CAP; t += GG_T) {
+        S.key[t] = gk[g0 + t];
+        S.ord[t] = go[g0 + t];
+      }
+      __syncthreads();
+      if (k == GS_CAP)
+        for (int32_t k2 = 2; k2 < GS_CAP; k2 <<= 1)
+          for (int32_t j = k2 >> 1; j > 0; j >>= 1)
+            gg_step(S, GS_CAP, g0, k2, j);
+      for (int32_t j = GS_CAP >> 1; j > 0; j >>= 1)
+        gg_step(S, GS_CAP, g0, k, j);
+      for (int32_t t = threadIdx.x; t < GS_CAP; t += GG_T) {
+        gk[g0 + t] = S.key[t];
+        go[g0 + t] = S.ord[t];
+      }
+      __threadfence_block();
+      __syncthreads();
+    }
+  }
+}
+
+__global__ void __launch_bounds__(GG_T)
+k_greedy_grow(GreedyCfg c, const int32_t *__restrict__ isort,
+              const float *__restrict__ pos, const int64_t *__restrict__ ids,
+              uint8_t *__restrict__ alive, uint8_t *__restrict__ done, int par,
+              GState *__restrict__ St, const int32_t *__restrict__ ready,
+              const GInfo *__restrict__ info, const uint64_t *__restrict__ ures,
+              GPoolPtrs G, int64_t *__restrict__ structure,
+              GRec *__restrict__ recs, double *__restrict__ radb,
+              int32_t *__restrict__ massb) {
+  __shared__ GrowLds S;
+  const int l = threadIdx.x & 63;
+  const uint64_t below = l == 0 ? 0ull : (~0ull >> (64 - l));
+  const double taille = (double)c.nx;
+  const int32_t nr = St->nready[par];
+  for (int32_t it = blockIdx.x; it < nr; it += gridDim.x) {
+    const GInfo gi = info[it];
+    if (gi.n1 == 0) continue;
+    const int32_t o = ready[it];
+    const int32_t n1 = gi.n1;
+    uint64_t *d2 = G.d2 + gi.off, *gk = G.key + gi.off;
+    uint32_t *go = G.ord + gi.off;
+    // the best candidate over the seed's units (S > 0: as integers)
+    uint64_t bs = 0;
+    int64_t bk = INT64_MAX;
+    for (int32_t g = threadIdx.x; g < (gi.ncand + 63) >> 6; g += GG_T) {
+      const uint64_t s = ures[2 * (int64_t)(gi.unit0 + g)];
+      const int64_t k = (int64_t)ures[2 * (int64_t)(gi.unit0 + g) + 1];
+      if (s > bs || (s == bs && k < bk)) {
+        bs = s;
+        bk = k;
+      }
+    }
+    const int64_t top = -gg_min(-(int64_t)bs, S);
+    const int64_t kbest = gg_min((int64_t)bs == top ? bk : INT64_MAX, S);
+    const int32_t centre = (int32_t)(kbest & 0xFFFFFFFF);
+    double xc[3];
+    centre_scaled(pos, centre, c.nx, xc);
+    // distances (main file:2002-2020)
+    const bool lds = n1 <= GS_CAP;
+    const double nc = (double)c.ncut, bscale = GS_BINS / (nc * nc * nc);
+    auto bin = [&](uint64_t bits) {
+      const double x = __longlong_as_double((long long)bits);
+      const double b = x * sqrt(x) * bscale;  // grows with x
+      return b < (double)GS_BINS ? (int32_t)b : GS_BINS;
+    };
+    if (!lds)
+      for (int32_t t = threadIdx.x; t < GS_BINS; t += GG_T) S.hist[t] = 0;
+    __syncthreads();
+    for (int32_t t = threadIdx.x; t < n1; t += GG_T) {
+      const int64_t j = __float_as_int(G.p[gi.off + t].w);
+      double dd[3];
+      for (int a = 0; a < 3; a++) {
+        dd[a] = fabs((double)(pos[3 * j + a] * (float)c.nx) - xc[a]);
+        dd[a] = fmin(dd[a], taille - dd[a]);
+      }
+      const uint64_t v = (uint64_t)__double_as_longlong(
+          __dadd_rn(__dadd_rn(__dmul_rn(dd[0], dd[0]), __dmul_rn(dd[1], dd[1])),
+                    __dmul_rn(dd[2], dd[2])));
+      if (lds) {
+        S.key[t] = v;
+        S.ord[t] = (uint32_t)t;
+      } else {
+        d2[t] = v;
+        const int32_t b = bin(v);
+        if (b < GS_BINS) atomicAdd(&S.hist[b], 1);
+      }
+    }
+    __threadfence_block();
+    __syncthreads();
+    // The last bin to sort: the first one whose particles must lie below the
+    // threshold, O(k) <= (particles up to the bin) / volume(its lower edge),
+    // and whose first particle is at least the 10th.
+    int32_t blast = GS_BINS;
+    if (!lds) {
+      // inclusive scan of the bins, GS_BINS / GG_T per thread
+      constexpr int V = GS_BINS / GG_T;
+      int32_t v[V], s = 0;
+      for (int i = 0; i < V; i++) s += v[i] = S.hist[threadIdx.x * V + i];
+      const int32_t inc = wave_incl_scan(s);
+      if ((threadIdx.x & 63) == 63) S.red_l[threadIdx.x >> 6] = inc;
+      __syncthreads();
+      int32_t cum = inc - s;
+      for (int i = 0; i < (int)(threadIdx.x >> 6); i++)
+        cum += (int32_t)S.red_l[i];
+      int64_t first = GS_BINS;
+      for (int i = 0; i < V; i++) {
+        const int32_t b = threadIdx.x * V + i;
+        const double vol = 2.0 / 3.0 * TWOPI_REF * ((double)b / bscale);
+        if (v[i] > 0 && cum >= 9 && first == GS_BINS &&
+            (double)(cum + v[i]) <= c.seuil * vol * (1.0 - 1e-9))
+          first = b;
+        cum += v[i];
+      }
+      blast = (int32_t)gg_min(first, S);
+    }
+    int32_t ns = n1;  // keys sorted
+    const uint64_t *SK = S.key;
+    const uint32_t *SO = S.ord;
+    int64_t stop = INT64_MAX;
+    for (;;) {
+      if (lds) {
+        gg_sort(S, gk, go, n1);
+      } else {
+        // collect the bins up to blast (all keys: blast = GS_BINS)
+        if (threadIdx.x == 0) S.n = 0;
+        __syncthreads();
+        int32_t cnt = 0;
+        for (int32_t t = threadIdx.x; t < n1; t += GG_T)
+          cnt += bin(d2[t]) <= blast;
+        cnt = wave_sum(cnt);
+        if (l == 0 && cnt) atomicAdd(&S.n, cnt);
+        __syncthreads();
+        ns = S.n;
+        __syncthreads();
+        if (threadIdx.x == 0) S.n = 0;
+        __syncthreads();
+        const bool in = ns <= GS_CAP;
+        for (int32_t t0 = 0; t0 < n1; t0 += GG_T) {  // uniform trip count
+          const int32_t t = t0 + (int32_t)threadIdx.x;
+          const bool take = t < n1 && bin(d2[t]) <= blast;
+          const uint64_t m = __ballot(take);  // one counter update per wave
+          int32_t e = 0;
+          if (l == 0 && m) e = atomicAdd(&S.n, (int32_t)__popcll(m));
+          e = __shfl(e, 0, 64) + __popcll(m & below);
+          if (take && in) {
+            S.key[e] = d2[t];
+            S.ord[e] = (uint32_t)t;
+          } else if (take) {
+            gk[e] = d2[t];
+            go[e] = (uint32_t)t;
           }
         }
         __threadfence_block();
         __syncthreads();
+        gg_sort(S, gk, go, ns);
+        SK = in ? S.key : gk;
+        SO = in ? S.ord : go;
       }
-    // growth (main file:2040-2051): stop at the first i >= 10 with
-    // O(i) <= seuil, i == npart_sel or r_i >= ncut
-    int64_t stop = INT64_MAX;
-    for (int64_t i = 10 + threadIdx.x; i <= n1; i += GT) {
-      const double r = sqrt(d2[i - 1]);
-      if (od_k(i, 1.0, r) <= c.seuil || i >= n1 || r >= (double)c.ncut)
-        stop = min(stop, i);
+      // growth (main file:2040-2051): stop at the first i >= 10 with
+      // O(i) <= seuil, i == npart_sel or r_i >= ncut
+      stop = INT64_MAX;
+      for (int64_t i = 10 + threadIdx.x; i <= ns; i += GG_T) {
+        const double r = sqrt(__longlong_as_double((long long)SK[i - 1]));
+        if (od_k(i, 1.0, r) <= c.seuil || i >= n1 || r >= nc)
+          stop = min(stop, i);
+      }
+      stop = gg_min(stop, S);
+      if (stop != INT64_MAX || ns == n1) break;
+      blast = GS_BINS;  // not in those bins: every key
     }
-    stop = gmin(stop, S);
-    if (stop == INT64_MAX || od_k(stop, 1.0, sqrt(d2[stop - 1])) > c.seuil) {
+    auto rad = [&](int64_t i) {
+      return sqrt(__longlong_as_double((long long)SK[i]));
+    };
+    if (stop == INT64_MAX || od_k(stop, 1.0, rad(stop - 1)) > c.seuil) {
       // "Increase selection radius" (main file:2072-2089)
-      if (threadIdx.x == 0) {
-        R.status = PSOD_E_UNCLOSED;
-        R.npart_sel = n1;
-        recs[o] = R;
-        atomicMin(&fail[0], (int32_t)o);
-      }
+      if (threadIdx.x == 0)
+        atomicMin(&St->fail, ((unsigned long long)o << 8) | GF_UNCLOSED);
       __syncthreads();
       continue;
     }
     // second threshold: last i in [2, stop] above seuil2 (:2062-2069)
     int64_t m2 = 0;
-    for (int64_t i = 2 + threadIdx.x; i <= stop; i += GT)
-      if (od_k(i, 1.0, sqrt(d2[i - 1])) > c.seuil2) m2 = max(m2, i);
-    m2 = -gmin(-m2, S);
+    for (int64_t i = 2 + threadIdx.x; i <= stop; i += GG_T)
+      if (od_k(i, 1.0, rad(i - 1)) > c.seuil2) m2 = max(m2, i);
+    m2 = -gg_min(-m2, S);
     const int64_t masse = stop - 1;
-    const double rayon = sqrt(d2[masse - 1]);
+    const double rayon = rad(masse - 1);
     const double volume = 2.0 / 3.0 * TWOPI_REF * (rayon * rayon * rayon);
     const double amass = (double)masse;
-    // profile (main file:2103-2115)
-    for (int j = threadIdx.x; j < c.nbins; j += GT) {
+    if (threadIdx.x == 0) S.n = atomicAdd(&St->nrec, 1);
+    __syncthreads();
+    const int64_t row = S.n;
+    // profile (main file:2103-2115): counts of r < r_j.  Every particle
+    // closer than the last one sorted is sorted; a radius beyond it counts
+    // the unsorted ones too.
+    const double rlast = rad(ns - 1);
+    for (int j = threadIdx.x; j < c.nbins; j += GG_T) {
       // the last radius is rayon * rmax_frac exactly
       const double rj =
           j == c.nbins - 1 ? rayon * c.rmaxf
                            : rayon * exp(c.lr0 + (double)j * (c.lr1 - c.lr0) /
                                                      ((double)c.nbins - 1.0));
-      int32_t lo2 = 0, hi2 = n1;
-      while (lo2 < hi2) {
-        const int32_t mid = (lo2 + hi2) >> 1;
-        if (sqrt(d2[mid]) < rj) lo2 = mid + 1; else hi2 = mid;
+      int32_t lo2 = 0, hi2 = ns;
+      if (ns == n1 || rj <= rlast) {
+        while (lo2 < hi2) {
+          const int32_t mid = (lo2 + hi2) >> 1;
+          if (rad(mid) < rj) lo2 = mid + 1; else hi2 = mid;
+        }
+      } else {
+        for (int32_t t = 0; t < n1; t++)
+          lo2 += sqrt(__longlong_as_double((long long)d2[t])) < rj;
       }
-      radb[o * c.nbins + j] = rj;
-      massb[o * c.nbins + j] = lo2;
+      radb[row * c.nbins + j] = rj;
+      massb[row * c.nbins + j] = lo2;
     }
     const bool acc = amass >= c.mmin && xc[0] <= taille && xc[0] > 0.0 &&
                      xc[1] <= taille && xc[1] > 0.0 && xc[2] <= taille &&
                      xc[2] > 0.0;
     const int64_t iamas = ids ? ids[centre] : (int64_t)centre;
     // exclusion of the first masse particles, accepted or not
-    for (int64_t t = threadIdx.x; t < masse; t += GT) {
-      const GEntry p = ent[ord[t]];
-      alive[p.slot] = 0;
-      structure[p.idx] = acc ? iamas : 0;
+    for (int64_t t = threadIdx.x; t < masse; t += GG_T) {
+      const int64_t e = gi.off + SO[t];
+      alive[G.slot[e]] = 0;
+      structure[__float_as_int(G.p[e].w)] = acc ? iamas : 0;
     }
     if (threadIdx.x == 0) {
+      GRec R;
+      R.ipart = (int64_t)o + 1;
+      R.seed = isort[o] - 1;
       R.centre = centre;
       R.iamas = iamas;
       R.masse = masse;
       R.masse2 = m2;
-      R.npart_sel = n1;
       R.amass = amass;
       R.xc = xc[0];
       R.yc = xc[1];
       R.zc = xc[2];
       R.rayon = rayon;
       R.overdens = volume > 0.0 ? amass / volume : 0.0;
+      R.overdens2 = 0.0;
       if (m2 > 0) {
-        const double r2 = sqrt(d2[m2 - 1]);
+        const double r2 = rad(m2 - 1);
         R.overdens2 = r2 > 1e-30 ? od_k(m2, 1.0, r2) : 0.0;
       }
       R.accepted = acc ? 1 : 0;
-      R.status = 1;  // a processed seed
-      recs[o] = R;
+      R.pad = 0;
+      recs[row] = R;
       done[o] = 1;
     }
     __syncthreads();
@@ -442,7 +951,9 @@ extern "C" int psod_host_spherover(psod_ctx *ctx, int64_t npart,
   c.nx = p->nx;
   c.ncut = p->ncut;
   c.nbins = p->nbins;
-  c.nb = p->nx / 8;
+  // marking blocks of 4^3 cells, of 8^3 where a seed's reach spans many
+  c.bsh = p->ncut <= 8 ? 2 : 3;
+  c.nb = p->nx >> c.bsh;
   c.seuil = p->seuil;
   c.seuil2 = p->seuil2;
   c.mmin = p->mmin;
@@ -453,13 +964,15 @@ extern "C" int psod_host_spherover(psod_ctx *ctx, int64_t npart,
   hipStream_t st = ctx->stream;
   const int64_t ncellt = (int64_t)p->nx * p->nx * p->nx;
   const int64_t nn = npart_new > 0 ? npart_new : 1;
+  // every record removes at least 9 particles (its count starts at 10)
+  const int64_t rcap = std::min<int64_t>(nn, npart / 9 + 1);
   float *dpos = (float *)psod_scratch(ctx, S_HOST_A, (size_t)npart * 12);
   int32_t *cs = (int32_t *)psod_scratch(ctx, S_HOST_B, (size_t)(ncellt + 1) * 4);
   int32_t *perm = (int32_t *)psod_scratch(ctx, S_HOST_C, (size_t)npart * 4);
   float *drec = (float *)psod_scratch(ctx, S_HOST_D, (size_t)npart * 16);
   char *A = (char *)psod_scratch(ctx, S_GREEDY,
                                  (size_t)npart * (4 + 1 + 8 + 8 + 1) +
-                                     (size_t)nn * (4 + 1 + 4) + 4096);
+                                     (size_t)nn * (4 + 1) + 4096);
   if (!dpos || !cs || !perm || !drec || !A) return PSOD_E_NOMEM;
   int32_t *slot_of = (int32_t *)A;
   int64_t *dstruct = (int64_t *)(A + (((size_t)npart * 4 + 255) & ~(size_t)255));
@@ -468,23 +981,40 @@ extern "C" int psod_host_spherover(psod_ctx *ctx, int64_t npart,
   uint8_t *alive_o = alive_s + npart;
   int32_t *dseeds = (int32_t *)(((uintptr_t)(alive_o + npart) + 255) & ~(uintptr_t)255);
   uint8_t *done = (uint8_t *)(dseeds + nn);
-  int32_t *ready = (int32_t *)(((uintptr_t)(done + nn) + 255) & ~(uintptr_t)255);
-  const int32_t NG = ctx->num_cus * 2;
   const int32_t nbk = c.nb * c.nb * c.nb;
+  // the pool holds a round's gathered particles: at most every ready seed's
+  // cells, and one seed's whole slice
+  int64_t pcap = GCAP;
+  while (pcap < GPOOL && pcap < 16 * npart) pcap <<= 1;
+  const int64_t ucap = pcap / 64 + GWIN;
+  constexpr size_t PER = 16 + 4 + 4 + 16 + 4 + 8 + 8 + 8 + 4;
   char *B = (char *)psod_scratch(
       ctx, S_GREEDY2,
-      (size_t)NG * GCAP * (sizeof(GEntry) + 8 + 4) + (size_t)nbk * 4 + 1024);
-  GRec *recs = (GRec *)psod_scratch(ctx, S_GREEDY3,
-                                    (size_t)nn * (sizeof(GRec) +
-                                                  (size_t)p->nbins * 12) + 256);
-  if (!B || !recs) return PSOD_E_NOMEM;
-  GEntry *ent = (GEntry *)B;
-  double *d2 = (double *)(ent + (size_t)NG * GCAP);
-  int32_t *ord = (int32_t *)(d2 + (size_t)NG * GCAP);
-  int32_t *bmin = ord + (size_t)NG * GCAP;
-  int32_t *ctr = bmin + nbk;  // [0] nready, [1] queue, [2] fail
-  double *radb = (double *)(recs + nn);
-  int32_t *massb = (int32_t *)(radb + (size_t)nn * p->nbins);
+      (size_t)pcap * PER + (size_t)ucap * (16 + 8) +
+          (size_t)GWIN * (sizeof(GInfo) + 4) + (size_t)nbk * 4 + 8192);
+  char *R = (char *)psod_scratch(ctx, S_GREEDY3,
+                                 (size_t)rcap * (sizeof(GRec) +
+                                                 (size_t)p->nbins * 12) + 512);
+  if (!B || !R) return PSOD_E_NOMEM;
+  GPoolPtrs G;
+  GState *S = (GState *)B;
+  G.p = (float4 *)(B + 256);
+  G.near = G.p + pcap;
+  G.upper = (double *)(G.near + pcap);
+  G.d2 = (uint64_t *)(G.upper + pcap);
+  G.key = G.d2 + pcap;
+  uint64_t *ures = G.key + pcap;
+  int2 *units = (int2 *)(ures + 2 * ucap);
+  GInfo *info = (GInfo *)(units + ucap);
+  G.slot = (int32_t *)(info + GWIN);
+  G.cell = G.slot + pcap;
+  G.cand = G.cell + pcap;
+  G.ord = (uint32_t *)(G.cand + pcap);
+  int32_t *ready = (int32_t *)(G.ord + pcap);
+  int32_t *bmin = ready + GWIN;
+  GRec *recs = (GRec *)R;
+  double *radb = (double *)(recs + rcap);
+  int32_t *massb = (int32_t *)(radb + (size_t)rcap * p->nbins);
 
   PSOD_HIP(hipMemcpyAsync(dpos, pos, (size_t)npart * 12, hipMemcpyHostToDevice, st));
   PSOD_TRY(psod_cell_sort(ctx, npart, dpos, nullptr, p->nx, cs, perm, drec,
@@ -492,71 +1022,78 @@ extern "C" int psod_host_spherover(psod_ctx *ctx, int64_t npart,
   if (ids)
     PSOD_HIP(hipMemcpyAsync(dids, ids, (size_t)npart * 8, hipMemcpyHostToDevice, st));
   k_inverse_perm<<<grid_for(npart, 256), 256, 0, st>>>(perm, npart, slot_of);
+  PSOD_LAUNCH_CHECK();
   k_set_u8<<<grid_for(npart, 256, 4096), 256, 0, st>>>(alive_s, npart, 1);
+  PSOD_LAUNCH_CHECK();
   PSOD_HIP(hipMemsetAsync(dstruct, 0, (size_t)npart * 8, st));
   PSOD_HIP(hipMemsetAsync(done, 0, (size_t)nn, st));
-  PSOD_HIP(hipMemsetAsync(recs, 0, (size_t)nn * sizeof(GRec), st));
-  // seeds: isort is 1-based particle indices
-  std::vector<int32_t> hs(nn);
-  for (int64_t o = 0; o < npart_new; o++) hs[o] = isort[o] - 1;
-  PSOD_HIP(hipMemcpyAsync(dseeds, hs.data(), (size_t)npart_new * 4,
-                          hipMemcpyHostToDevice, st));
-  PSOD_TRY(psod_fill_i32(ctx, ctr + 2, 1, INT32_MAX));
+  // isort: 1-based particle indices
+  if (npart_new > 0)
+    PSOD_HIP(hipMemcpyAsync(dseeds, isort, (size_t)npart_new * 4,
+                            hipMemcpyHostToDevice, st));
+  PSOD_TRY(psod_fill_i32(ctx, bmin, nbk, INT32_MAX));
+  GState hs;
+  memset(&hs, 0, sizeof(hs));
+  hs.fail = ~0ull;
+  PSOD_HIP(hipMemcpyAsync(S, &hs, sizeof(hs), hipMemcpyHostToDevice, st));
   PSOD_HIP(hipStreamSynchronize(st));
-  // rounds over a sliding window of seeds
-  const int64_t WIN = 1 << 16;
-  std::vector<uint8_t> hdone;
-  int64_t lo = 0;
-  int rounds = 0;
-  while (lo < npart_new) {
-    const int64_t hi = std::min<int64_t>(npart_new, lo + WIN);
-    PSOD_TRY(psod_fill_i32(ctx, bmin, nbk, INT32_MAX));
-    PSOD_TRY(psod_fill_i32(ctx, ctr, 2, 0));
-    const unsigned gw = grid_for(hi - lo, 256);
-    k_mark_blocks<<<gw, 256, 0, st>>>(c, dseeds, slot_of, dpos, alive_s, done,
-                                      lo, hi, bmin);
-    k_ready<<<gw, 256, 0, st>>>(c, dseeds, slot_of, dpos, alive_s, done, lo,
-                                hi, bmin, ready, ctr);
-    int32_t nready = 0;
-    PSOD_HIP(hipMemcpyAsync(&nready, ctr, 4, hipMemcpyDeviceToHost, st));
-    PSOD_HIP(hipStreamSynchronize(st));
-    if (nready > 0) {
-      k_greedy_seed<<<(unsigned)std::min(nready, NG), GT, 0, st>>>(
-          c, dseeds, cs, (const float4 *)drec, dpos, ids ? dids : nullptr,
-          alive_s, done, lo, hi, ready, ctr, ctr + 1, ent, d2, ord, dstruct,
-          recs, radb, massb, ctr + 2);
+  // Rounds over a sliding window of seeds, GROUNDS of them queued at a time:
+  // the window, the counts and the work lists stay on the device.
+  const int32_t nnew = (int32_t)npart_new;
+  int32_t lo = 0;
+  int64_t ran = 0;  // ready seeds so far
+  while (lo < nnew && hs.fail == ~0ull) {
+    const int32_t lo0 = lo;
+    for (int r = 0; r < GROUNDS; r++) {
+      const int par = r & 1;
+      // the window starts at lo0 or later
+      const unsigned gw = grid_for(std::min<int64_t>(GWIN, nnew - lo0), 256);
+      k_mark<<<gw, 256, 0, st>>>(c, dseeds, slot_of, dpos, alive_s, done, nnew,
+                                 par, S, bmin);
+      PSOD_LAUNCH_CHECK();
+      k_ready<<<gw, 256, 0, st>>>(c, dseeds, slot_of, dpos, alive_s, done,
+                                  nnew, par, S, bmin, ready);
+      PSOD_LAUNCH_CHECK();
+      k_greedy_gather<<<(unsigned)ctx->num_cus, GA_T, 0, st>>>(
+          c, dseeds, cs, (const float4 *)drec, dpos, alive_s, done, par, S,
+          ready, info, units, G, pcap);
+      PSOD_LAUNCH_CHECK();
+      k_greedy_bound<<<(unsigned)ctx->num_cus * 4, GC_T, 0, st>>>(
+          par, S, info, units, G);
+      PSOD_LAUNCH_CHECK();
+      k_greedy_centre<<<(unsigned)ctx->num_cus * 4, 256, 0, st>>>(
+          c, dseeds, dpos, par, S, ready, info, units, G, ures, bmin, nbk);
+      PSOD_LAUNCH_CHECK();
+      k_greedy_grow<<<(unsigned)ctx->num_cus, GG_T, 0, st>>>(
+          c, dseeds, dpos, ids ? dids : nullptr, alive_s, done, par, S, ready,
+          info, ures, G, dstruct, recs, radb, massb);
       PSOD_LAUNCH_CHECK();
     }
-    int32_t fail = INT32_MAX;
-    PSOD_HIP(hipMemcpyAsync(&fail, ctr + 2, 4, hipMemcpyDeviceToHost, st));
-    hdone.resize((size_t)(hi - lo));
-    PSOD_HIP(hipMemcpyAsync(hdone.data(), done + lo, (size_t)(hi - lo),
-                            hipMemcpyDeviceToHost, st));
+    PSOD_HIP(hipMemcpyAsync(&hs, S, sizeof(hs), hipMemcpyDeviceToHost, st));
     PSOD_HIP(hipStreamSynchronize(st));
-    rounds++;
-    if (fail != INT32_MAX) break;
-    int64_t adv = 0;
-    while (adv < hi - lo && hdone[(size_t)adv]) adv++;
-    lo += adv;
-    if ((adv == 0 && nready == 0) || rounds > npart_new + 2)
+    lo = hs.first[(GROUNDS - 1) & 1];
+    const int64_t r1 = (int64_t)hs.total + hs.nready[(GROUNDS - 1) & 1];
+    if (hs.fail == ~0ull && lo == lo0 && r1 == ran)
       return psod_set_error(PSOD_E_DEVICE, "spherover: no progress");
+    ran = r1;
   }
-  int32_t fail = INT32_MAX;
-  PSOD_HIP(hipMemcpyAsync(&fail, ctr + 2, 4, hipMemcpyDeviceToHost, st));
-  PSOD_HIP(hipStreamSynchronize(st));
-  // records in seed order, up to the first failing seed
-  std::vector<GRec> hr((size_t)nn);
-  std::vector<double> hrb((size_t)nn * p->nbins);
-  std::vector<int32_t> hmb((size_t)nn * p->nbins);
-  PSOD_HIP(hipMemcpyAsync(hr.data(), recs, (size_t)nn * sizeof(GRec),
-                          hipMemcpyDeviceToHost, st));
-  PSOD_HIP(hipMemcpyAsync(hrb.data(), radb, hrb.size() * 8,
-                          hipMemcpyDeviceToHost, st));
-  PSOD_HIP(hipMemcpyAsync(hmb.data(), massb, hmb.size() * 4,
-                          hipMemcpyDeviceToHost, st));
+  // records, in seed order up to the first failing seed
+  const int64_t nr = hs.nrec;
+  std::vector<GRec> hr((size_t)nr);
+  std::vector<double> hrb((size_t)nr * p->nbins);
+  std::vector<int32_t> hmb((size_t)nr * p->nbins);
+  if (nr > 0) {
+    PSOD_HIP(hipMemcpyAsync(hr.data(), recs, (size_t)nr * sizeof(GRec),
+                            hipMemcpyDeviceToHost, st));
+    PSOD_HIP(hipMemcpyAsync(hrb.data(), radb, hrb.size() * 8,
+                            hipMemcpyDeviceToHost, st));
+    PSOD_HIP(hipMemcpyAsync(hmb.data(), massb, hmb.size() * 4,
+                            hipMemcpyDeviceToHost, st));
+  }
   if (alive) {
     k_alive_orig<<<grid_for(npart, 256), 256, 0, st>>>(alive_s, perm, npart,
                                                        alive_o);
+    PSOD_LAUNCH_CHECK();
     PSOD_HIP(hipMemcpyAsync(alive, alive_o, (size_t)npart,
                             hipMemcpyDeviceToHost, st));
   }
@@ -564,11 +1101,17 @@ extern "C" int psod_host_spherover(psod_ctx *ctx, int64_t npart,
     PSOD_HIP(hipMemcpyAsync(structure, dstruct, (size_t)npart * 8,
                             hipMemcpyDeviceToHost, st));
   PSOD_HIP(hipStreamSynchronize(st));
-  const int64_t upto = fail == INT32_MAX ? npart_new : (int64_t)fail;
+  const int64_t upto = hs.fail == ~0ull ? npart_new : (int64_t)(hs.fail >> 8);
+  std::vector<int32_t> order((size_t)nr);
+  std::iota(order.begin(), order.end(), 0);
+  std::sort(order.begin(), order.end(), [&](int32_t a, int32_t b) {
+    return hr[(size_t)a].ipart < hr[(size_t)b].ipart;
+  });
   int64_t k = 0;
-  for (int64_t o = 0; o < upto; o++) {
+  for (int64_t i = 0; i < nr; i++) {
+    const int64_t o = order[(size_t)i];
     const GRec &g = hr[(size_t)o];
-    if (g.status != 1) continue;
+    if (g.ipart > upto) break;
     if (k >= maxrec) return psod_set_error(PSOD_E_CAPACITY,
                                            "spherover: more than %lld records",
                                            (long long)maxrec);
@@ -592,20 +1135,19 @@ extern "C" int psod_host_spherover(psod_ctx *ctx, int64_t npart,
     k++;
   }
   *nrec = k;
-  if (fail != INT32_MAX) {
-    const GRec &g = hr[(size_t)fail];
-    if (g.status == -PSOD_E_CAPACITY)
+  if (hs.fail != ~0ull) {
+    const long long seed1 = (long long)(hs.fail >> 8) + 1;
+    const int code = (int)(hs.fail & 255);
+    if (code == GF_GCAP)
       return psod_set_error(PSOD_E_CAPACITY,
                             "spherover: seed %lld gathers more than %lld "
-                            "particles (device slice)",
-                            (long long)(fail + 1), (long long)GCAP);
-    return psod_set_error(g.status,
-                          g.status == PSOD_E_CAPACITY
-                              ? "spherover: Nsel exceeded at seed %lld"
-                              : "spherover: sphere of seed %lld not closed "
-                                "within ncut",
-                          (long long)(fail + 1));
+                            "particles (device slice)", seed1, (long long)GCAP);
+    if (code == GF_NSEL)
+      return psod_set_error(PSOD_E_CAPACITY,
+                            "spherover: Nsel exceeded at seed %lld", seed1);
+    return psod_set_error(PSOD_E_UNCLOSED,
+                          "spherover: sphere of seed %lld not closed within "
+                          "ncut", seed1);
   }
-  (void)rounds;
   return PSOD_OK;
 }
