@@ -205,12 +205,16 @@ __device__ inline T wave_sum(T v) {
   return v;
 }
 
+// Inclusive sum over the lanes; every lane of the wave must be active.  Row
+// shifts by 1, 2, 4, 8 scan each row of 16 lanes, broadcasts of lanes 15
+// and 31 carry the rows (register moves, no LDS round trips).
 __device__ inline int32_t wave_incl_scan(int32_t v) {
-  const int l = __lane_id();
-  for (int o = 1; o < 64; o <<= 1) {
-    int32_t t = __shfl_up(v, o, 64);
-    if (l >= o) v += t;
-  }
+  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);
   return v;
 }
 
