@@ -664,50 +664,20 @@ extern "C" int psod_label_counts(psod_ctx *ctx, int64_t npart,
 // with the particle index as a stable payload = decreasing rho, ties by
 // index; npart_new = #(rho > threshold) + 1 (main file:1029-1032).
 // ---------------------------------------------------------------------------
-__global__ void k_density_keys(const float *__restrict__ rho, int64_t n,
-                               float thr, uint64_t *__restrict__ keys,
-                               uint32_t *__restrict__ vals,
-                               unsigned long long *__restrict__ nabove) {
-  unsigned long long cnt = 0;
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-       i += (int64_t)gridDim.x * blockDim.x) {
-    const float r = rho[i];
-    keys[i] = (uint64_t)(0xFFFFFFFFu - __float_as_uint(fmaxf(r, 0.0f)));
-    vals[i] = (uint32_t)i;
-    cnt += (r > thr) ? 1 : 0;
-  }
-  cnt = wave_sum(cnt);
-  if ((threadIdx.x & 63) == 0 && cnt) atomicAdd(nabove, cnt);
-}
-
-__global__ void k_isort_out(const uint32_t *__restrict__ vals, int64_t n,
-                            int32_t *__restrict__ isort) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) isort[i] = (int32_t)vals[i] + 1;
-}
-
 extern "C" int psod_density_order(psod_ctx *ctx, int64_t npart,
                                   const float *d_rho, double threshold,
                                   int32_t *d_isort, int64_t *npart_new) {
   PSOD_TRY(psod_use_device(ctx));
   if (npart <= 0 || !d_rho || !d_isort || !npart_new)
     return psod_set_error(PSOD_E_ARG, "psod_density_order: bad arguments");
-  uint64_t *keys = (uint64_t *)psod_scratch(ctx, S_KEYS, (size_t)npart * 8);
-  uint32_t *vals = (uint32_t *)psod_scratch(ctx, S_VALS, (size_t)npart * 4);
   unsigned long long *cnt =
       (unsigned long long *)psod_scratch(ctx, S_MISC, 256);
-  if (!keys || !vals || !cnt) return PSOD_E_NOMEM;
+  if (!cnt) return PSOD_E_NOMEM;
   PSOD_TRY(psod_fill_u64(ctx, (uint64_t *)cnt, 1, 0));
   // float threshold: rho > thr in float equals rho > threshold for the
   // thresholds used (exactly representable, e.g. 100)
-  k_density_keys<<<grid_for(npart, 256, (int64_t)ctx->num_cus * 32), 256, 0,
-                   ctx->stream>>>(d_rho, npart, (float)threshold, keys, vals,
-                                  cnt);
-  PSOD_LAUNCH_CHECK();
-  PSOD_TRY(psod_radix_sort_u64(ctx, npart, keys, vals, 32));
-  k_isort_out<<<grid_for(npart, 256), 256, 0, ctx->stream>>>(vals, npart,
-                                                             d_isort);
-  PSOD_LAUNCH_CHECK();
+  PSOD_TRY(psod_order_by_density(ctx, npart, d_rho, (float)threshold, cnt,
+                                 d_isort));
   unsigned long long h = 0;
   PSOD_HIP(hipMemcpyAsync(&h, cnt, 8, hipMemcpyDeviceToHost, ctx->stream));
   PSOD_HIP(hipStreamSynchronize(ctx->stream));

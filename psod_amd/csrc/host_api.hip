@@ -185,7 +185,6 @@ extern "C" int psod_host_cicm1(psod_ctx *ctx, int64_t npart, const float *pos,
 // ---------------------------------------------------------------------------
 __global__ void k_pdens_keys(const double *__restrict__ rho, int64_t n,
                              double lim, uint64_t *__restrict__ keys,
-                             uint32_t *__restrict__ vals,
                              unsigned long long *__restrict__ nbelow) {
   unsigned long long cnt = 0;
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
@@ -194,17 +193,10 @@ __global__ void k_pdens_keys(const double *__restrict__ rho, int64_t n,
     // rho > 0 for every particle (its own mass is deposited); a
     // non-positive or NaN value sorts last
     keys[i] = pd > 0.0 ? (uint64_t)__double_as_longlong(pd) : ~0ull;
-    vals[i] = (uint32_t)i;
     cnt += (pd > 0.0 && pd < lim) ? 1 : 0;
   }
   cnt = wave_sum(cnt);
   if ((threadIdx.x & 63) == 0 && cnt) atomicAdd(nbelow, cnt);
-}
-
-__global__ void k_isort1(const uint32_t *__restrict__ vals, int64_t n,
-                         int32_t *__restrict__ isort) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) isort[i] = (int32_t)vals[i] + 1;
 }
 
 extern "C" int psod_density_order_f64(psod_ctx *ctx, int64_t npart,
@@ -215,18 +207,15 @@ extern "C" int psod_density_order_f64(psod_ctx *ctx, int64_t npart,
       !npart_new || !(threshold > 0.0))
     return psod_set_error(PSOD_E_ARG, "psod_density_order_f64: bad arguments");
   uint64_t *keys = (uint64_t *)psod_scratch(ctx, S_KEYS, (size_t)npart * 8);
-  uint32_t *vals = (uint32_t *)psod_scratch(ctx, S_VALS, (size_t)npart * 4);
   unsigned long long *cnt =
       (unsigned long long *)psod_scratch(ctx, S_MISC, 256);
-  if (!keys || !vals || !cnt) return PSOD_E_NOMEM;
+  if (!keys || !cnt) return PSOD_E_NOMEM;
   hipStream_t st = ctx->stream;
   PSOD_TRY(psod_fill_u64(ctx, (uint64_t *)cnt, 1, 0));
   k_pdens_keys<<<grid_for(npart, 256, (int64_t)ctx->num_cus * 32), 256, 0,
-                 st>>>(d_rho, npart, 1.0 / threshold, keys, vals, cnt);
+                 st>>>(d_rho, npart, 1.0 / threshold, keys, cnt);
   PSOD_LAUNCH_CHECK();
-  PSOD_TRY(psod_radix_sort_u64(ctx, npart, keys, vals, 64));
-  k_isort1<<<grid_for(npart, 256), 256, 0, st>>>(vals, npart, d_isort);
-  PSOD_LAUNCH_CHECK();
+  PSOD_TRY(psod_radix_sort_u64(ctx, npart, keys, (uint32_t *)d_isort, true));
   unsigned long long h = 0;
   PSOD_HIP(hipMemcpyAsync(&h, cnt, 8, hipMemcpyDeviceToHost, st));
   PSOD_HIP(hipStreamSynchronize(st));

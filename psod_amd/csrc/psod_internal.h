@@ -188,11 +188,16 @@ int psod_scan_i32(psod_ctx *ctx, const int32_t *in, int32_t *out, int64_t n,
                   int32_t *total);
 
 // radix sort of 64-bit keys with 32-bit values, ascending, stable.  With
-// d_n not NULL only the first min(n, *d_n) elements are sorted (a count
-// known on the device only; n is then the capacity).
+// `order` the values read are ignored and the sorted ones are the 1-based
+// places of the keys (the keys themselves are then not kept).
 int psod_radix_sort_u64(psod_ctx *ctx, int64_t n, uint64_t *keys,
-                        uint32_t *vals, int key_bits,
-                        const int32_t *d_n = nullptr);
+                        uint32_t *vals, bool order = false);
+
+// 1-based particle indices by decreasing density, ties by index, into isort
+// (n > 0); adds the densities above thr to *nabove.
+int psod_order_by_density(psod_ctx *ctx, int64_t n, const float *rho,
+                          float thr, unsigned long long *nabove,
+                          int32_t *isort);
 
 // ---------------------------------------------------------------------------
 // wave64 helpers

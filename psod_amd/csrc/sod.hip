@@ -1397,28 +1397,92 @@ k_task_items(const int4 *__restrict__ tasks,
   if ((threadIdx.x & 63) == 0 && ns) atomicAdd(&cstat[1], ns);
 }
 
-// Sort keys of the items: the ratio of the item's bound to its halo's best
+// Work lists are taken in decreasing order of a cost, which decides only
+// when a piece of work starts, never a result: an order of 256 classes
+// (8 per factor of two) does, in one counting pass.  Full sorts of 48- and
+// 32-bit keys were 6 and 4 radix passes, 16 of them a pass and about 0.5 ms
+// of launches at 256^3.  The key kernels write each element's class (0:
+// largest) and count the classes in hist[0..255]; k_class_scatter places
+// the elements (any order within a class).  hist[256..511]: places taken.
+__device__ inline uint32_t cost_class(double v) {
+  const int32_t b = (int32_t)(__float_as_uint(fmaxf((float)v, 1.0f)) >> 20) -
+                    (127 << 3);
+  return (uint32_t)(255 - min(b, 255));
+}
+
+// adds this thread's class (if on) to the launch's counts; all 256 threads
+__device__ inline void count_class(bool on, uint32_t cls,
+                                   int32_t *__restrict__ hist) {
+  __shared__ int32_t h[256];
+  h[threadIdx.x] = 0;
+  __syncthreads();
+  if (on) atomicAdd(&h[cls], 1);
+  __syncthreads();
+  if (h[threadIdx.x]) atomicAdd(&hist[threadIdx.x], h[threadIdx.x]);
+}
+
+constexpr int ORD_V = 16;
+__global__ void __launch_bounds__(256)
+k_class_scatter(const uint8_t *__restrict__ cls,
+                const int32_t *__restrict__ in, int32_t n,
+                const int32_t *__restrict__ dn, int32_t *__restrict__ hist,
+                int32_t *__restrict__ out) {
+  __shared__ int32_t cnt[256], base[256], wsum[4];
+  if (dn) n = min(n, *dn);
+  const int32_t t0 = blockIdx.x * 256 * ORD_V;
+  if (t0 >= n) return;  // uniform
+  const int l = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int32_t tot = hist[threadIdx.x], inc = wave_incl_scan(tot);
+  if (l == 63) wsum[w] = inc;
+  cnt[threadIdx.x] = 0;
+  __syncthreads();
+  int32_t e = inc - tot;
+  for (int i = 0; i < w; i++) e += wsum[i];
+  int32_t k[ORD_V], r[ORD_V], v[ORD_V];
+#pragma unroll
+  for (int j = 0; j < ORD_V; j++) {
+    const int32_t i = t0 + j * 256 + (int32_t)threadIdx.x;
+    if (i < n) {
+      k[j] = cls[i];
+      v[j] = in[i];
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < ORD_V; j++)
+    if (t0 + j * 256 + (int32_t)threadIdx.x < n) r[j] = atomicAdd(&cnt[k[j]], 1);
+  __syncthreads();
+  const int32_t c = cnt[threadIdx.x];
+  base[threadIdx.x] = c > 0 ? e + atomicAdd(&hist[256 + threadIdx.x], c) : 0;
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < ORD_V; j++)
+    if (t0 + j * 256 + (int32_t)threadIdx.x < n) out[base[k[j]] + r[j]] = v[j];
+}
+
+// Classes of the items: the ratio of the item's bound to its halo's best
 // after the pilots, largest first (the groups most likely to raise the best
-// run first; those after them meet a higher best).
-__global__ void k_item_keys(const int32_t *__restrict__ items,
-                            const int32_t *__restrict__ nitems,
-                            const int4 *__restrict__ tasks,
-                            const int32_t *__restrict__ ntask_total,
-                            int32_t tcap,
-                            const unsigned long long *__restrict__ cub,
-                            const unsigned long long *__restrict__ hbest,
-                            uint64_t *__restrict__ keys,
-                            uint32_t *__restrict__ vals) {
+// run first; those after them meet a higher best).  64 classes per unit of
+// the ratio, up to 5.
+__global__ void __launch_bounds__(256)
+k_item_keys(const int32_t *__restrict__ items,
+            const int32_t *__restrict__ nitems, const int4 *__restrict__ tasks,
+            int32_t tcap, const unsigned long long *__restrict__ cub,
+            const unsigned long long *__restrict__ hbest,
+            uint8_t *__restrict__ cls, int32_t *__restrict__ hist) {
   const int32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= *nitems) return;
-  const int32_t it = items[i];
-  const int32_t t = it >> 3, g = it & 7;
-  const double ub = (double)cub[((int64_t)tcap * 27 + t) * 8 + g];
-  const double b = (double)hbest[tasks[t].x];
-  const double r = b > 0.0 ? ub / b : 1e9;
-  const double q = fmin(r, 255.0) * 16777216.0;  // 2^24 per unit of ratio
-  keys[i] = 0xFFFFFFFFull - (uint64_t)q;
-  vals[i] = (uint32_t)it;
+  const int32_t n = *nitems;
+  if ((int32_t)(blockIdx.x * blockDim.x) >= n) return;  // uniform
+  uint32_t k = 0;
+  if (i < n) {
+    const int32_t it = items[i];
+    const int32_t t = it >> 3, g = it & 7;
+    const double ub = (double)cub[((int64_t)tcap * 27 + t) * 8 + g];
+    const double b = (double)hbest[tasks[t].x];
+    const double r = b > 0.0 ? ub / b : 5.0;
+    k = 255u - (uint32_t)fmax(0.0, fmin((r - 1.0) * 64.0, 255.0));
+    cls[i] = (uint8_t)k;
+  }
+  count_class(i < n, k, hist);
 }
 
 // Exact phase, one wave per item (task t, candidates 8g..8g+15).  Lane l
@@ -4013,52 +4077,71 @@ __global__ void k_retry_reset(int32_t *__restrict__ c, int32_t nitem,
   if (blockIdx.x == 0 && threadIdx.x == 0) *need = 0ull;
 }
 
-// Sort keys of the large halos, most costly first.  For the centre search
-// the cost is the particles near the seed (members plus those of the 5^3
-// cells).  For the growth it is the particles of the cube of the planned
-// reach, summed over the 8^3 blocks that the cube overlaps: a small halo
-// beside a giant one walks the giant's particles too.
-__global__ void k_large_keys(SodCfg c, const HaloPlan *__restrict__ plan,
-                             const int32_t *__restrict__ large, int32_t n,
-                             const int32_t *__restrict__ dn,
-                             const int32_t *__restrict__ cell_start,
-                             int growth,
-                             uint64_t *__restrict__ keys,
-                             uint32_t *__restrict__ vals) {
-  const int32_t e = blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= n || (dn && e >= *dn)) return;
-  const int32_t h = large[e];
-  const HaloPlan pl = plan[h];
-  int64_t cost = (int64_t)max(pl.nmem, 0) + pl.n5;
-  if (growth) {
-    const int32_t nb = c.nx >> 3, W = max(pl.w0, 2);
-    int32_t lo[3], hi[3];
-    for (int d = 0; d < 3; d++) {
-      lo[d] = floor8(pl.cs[d] - W);
-      hi[d] = min(floor8(pl.cs[d] + W), lo[d] + nb - 1);  // at most nx cells
+// Classes of the large halos by cost: of the centre search (members and
+// particles around the seed), or of the growth: the particles of the 8^3
+// blocks that the planned cube overlaps, at most 16 per axis, every s-th
+// one scaled by s^3: a small halo beside a giant one walks the giant's
+// particles too.  One wave per halo over the blocks (one thread per halo:
+// 0.6 ms per call beside a 6e6-particle central halo).
+constexpr int KL_WG = 16;  // halos of a workgroup (growth)
+__global__ void __launch_bounds__(256)
+k_large_keys(SodCfg c, const HaloPlan *__restrict__ plan,
+             const int32_t *__restrict__ large, int32_t n,
+             const int32_t *__restrict__ dn,
+             const int32_t *__restrict__ cell_start, int growth,
+             uint8_t *__restrict__ cls, int32_t *__restrict__ hist) {
+  __shared__ uint32_t wcls[KL_WG];
+  if (dn) n = min(n, *dn);
+  const int per = growth ? KL_WG : 256;  // halos of a workgroup
+  const int32_t e0 = (int32_t)blockIdx.x * per, e = e0 + (int32_t)threadIdx.x;
+  if (e0 >= n) return;  // uniform
+  const bool on = (int)threadIdx.x < per && e < n;
+  uint32_t mine = 0;
+  if (!growth) {
+    if (on) {
+      const HaloPlan pl = plan[large[e]];
+      mine = cost_class((double)max(pl.nmem, 0) + (double)pl.n5);
     }
-    // every s-th block per axis (all of them up to 16 per axis), scaled by
-    // s^3: the key only orders the halos
-    const int32_t s = (hi[0] - lo[0] + 16) / 16;
-    cost = 0;
-    for (int32_t bz = lo[2]; bz <= hi[2]; bz += s)
-      for (int32_t by = lo[1]; by <= hi[1]; by += s)
-        for (int32_t bx = lo[0]; bx <= hi[0]; bx += s) {
-          const int64_t b = ((int64_t)wrapi(bz, nb) * nb + wrapi(by, nb)) * nb +
-                            wrapi(bx, nb);
-          cost += cell_start[(b + 1) * BS3] - cell_start[b * BS3];
-        }
-    cost *= (int64_t)s * s * s;
-    // A cube already holding more particles than a sphere of radius
-    // W / rmax_frac at the first threshold would is likely to be outgrown
-    // and walked again at twice the reach (about 4x the particles): such a
-    // halo is costed at both walks, so that it starts among the first.
-    const double rw = (double)W / c.rmax_frac;
-    if ((double)cost * c.mpart > c.delta[0] * (4.0 / 3.0 * M_PI) * rw * rw * rw)
-      cost *= 5;
+  } else {
+    const int l = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int32_t nb = c.nx >> 3;
+    for (int32_t i = w; i < KL_WG && e0 + i < n; i += 4) {
+      const HaloPlan pl = plan[large[e0 + i]];
+      const int32_t W = max(pl.w0, 2);
+      int32_t lo[3], k[3];
+      // the most blocks any axis overlaps decides the stride
+      int32_t most = 0;
+      for (int d = 0; d < 3; d++) {
+        lo[d] = floor8(pl.cs[d] - W);
+        k[d] = min(floor8(pl.cs[d] + W) - lo[d] + 1, nb);  // at most nx cells
+        most = max(most, k[d]);
+      }
+      const int32_t s = (most + 15) / 16;
+      for (int d = 0; d < 3; d++) k[d] = (k[d] + s - 1) / s;
+      int32_t sum = 0;
+      for (int32_t q = l; q < k[0] * k[1] * k[2]; q += 64) {
+        const int32_t bx = wrapi(lo[0] + s * (q % k[0]), nb),
+                      by = wrapi(lo[1] + s * (q / k[0] % k[1]), nb),
+                      bz = wrapi(lo[2] + s * (q / (k[0] * k[1])), nb);
+        const int64_t b = ((int64_t)bz * nb + by) * nb + bx;
+        sum += cell_start[(b + 1) * BS3] - cell_start[b * BS3];
+      }
+      sum = wave_sum(sum);
+      double cost = (double)sum * s * s * s;
+      // A cube already holding more particles than a sphere of radius
+      // W / rmax_frac at the first threshold would is likely to be outgrown
+      // and walked again at twice the reach (about 4x the particles): such a
+      // halo is costed at both walks, so that it starts among the first.
+      const double rw = (double)W / c.rmax_frac;
+      if (cost * c.mpart > c.delta[0] * (4.0 / 3.0 * M_PI) * rw * rw * rw)
+        cost *= 5.0;
+      if (l == 0) wcls[i] = cost_class(cost);
+    }
+    __syncthreads();
+    if (on) mine = wcls[threadIdx.x];
   }
-  keys[e] = (uint64_t)(0x7FFFFFFFFFFFll - min(cost, (int64_t)0x7FFFFFFFFFFFll));
-  vals[e] = (uint32_t)h;
+  if (on) cls[e] = (uint8_t)mine;
+  count_class(on, mine, hist);
 }
 
 // Clamps the task count of a captured pass to the buffers' capacity and
@@ -4213,21 +4296,24 @@ static int centre_search(psod_ctx *ctx, const SodCfg &c,
     PSOD_HIP(hipMemcpyAsync(&ni, nitems, 4, hipMemcpyDeviceToHost, st));
     PSOD_HIP(hipStreamSynchronize(st));
   }
+  const int32_t *list = items;
   if (ni > 1) {
-    uint64_t *keys = (uint64_t *)psod_scratch(ctx, S_KEYS, (size_t)ni * 8);
-    uint32_t *vals = (uint32_t *)psod_scratch(ctx, S_VALS, (size_t)ni * 4);
-    if (!keys || !vals) return PSOD_E_NOMEM;
-    k_item_keys<<<grid_for(ni, 256), 256, 0, st>>>(items, nitems, tasks, ntot,
-                                                   tcap, cub, hbest, keys,
-                                                   vals);
+    int32_t *hist = (int32_t *)psod_scratch(ctx, S_KEYS, (size_t)ni + 2048);
+    int32_t *ord = (int32_t *)psod_scratch(ctx, S_VALS, (size_t)ni * 4);
+    if (!hist || !ord) return PSOD_E_NOMEM;
+    uint8_t *cls = (uint8_t *)(hist + 512);
+    PSOD_TRY(psod_fill_i32(ctx, hist, 512, 0));
+    k_item_keys<<<grid_for(ni, 256), 256, 0, st>>>(items, nitems, tasks, tcap,
+                                                   cub, hbest, cls, hist);
     PSOD_LAUNCH_CHECK();
-    PSOD_TRY(psod_radix_sort_u64(ctx, ni, keys, vals, 32, dn ? nitems : nullptr));
-    PSOD_HIP(hipMemcpyAsync(items, vals, (size_t)ni * 4,
-                            hipMemcpyDeviceToDevice, st));
+    k_class_scatter<<<grid_for(ni, 256 * ORD_V), 256, 0, st>>>(
+        cls, items, ni, nitems, hist, ord);
+    PSOD_LAUNCH_CHECK();
+    list = ord;
   }
   k_centre_group<<<resident((const void *)k_centre_group), 256, 0, st>>>(
       c, cat->cell_start, (const float4 *)cat->rec, plan, large, tasks, ntot,
-      tcap, items, nitems, hbest, cub, ires, cstat, wq + 2);
+      tcap, list, nitems, hbest, cub, ires, cstat, wq + 2);
   PSOD_LAUNCH_CHECK();
   k_centre_reduce<<<grid_for(nlarge, 4), 256, 0, st>>>(plan, large, nlarge, dn,
                                                        tres, ires);
@@ -4432,14 +4518,18 @@ static int sod_fof_queue(psod_ctx *ctx, const psod_sod_params *p,
   // largest halos first (centre-search tasks and growth), so that the
   // persistent workgroups do not finish on a giant halo picked up last
   auto size_order = [&](int32_t n, const int32_t *dn, int growth) -> int {
-    uint64_t *keys = (uint64_t *)psod_scratch(ctx, S_KEYS, (size_t)n * 8);
-    uint32_t *vals = (uint32_t *)psod_scratch(ctx, S_VALS, (size_t)n * 4);
-    if (!keys || !vals) return PSOD_E_NOMEM;
-    k_large_keys<<<grid_for(n, 256), 256, 0, st>>>(
-        c, plan, large, n, dn, cat->cell_start, growth, keys, vals);
+    int32_t *hist = (int32_t *)psod_scratch(ctx, S_KEYS, (size_t)n + 2048);
+    int32_t *ord = (int32_t *)psod_scratch(ctx, S_VALS, (size_t)n * 4);
+    if (!hist || !ord) return PSOD_E_NOMEM;
+    uint8_t *cls = (uint8_t *)(hist + 512);
+    PSOD_TRY(psod_fill_i32(ctx, hist, 512, 0));
+    k_large_keys<<<grid_for(n, growth ? KL_WG : 256), 256, 0, st>>>(
+        c, plan, large, n, dn, cat->cell_start, growth, cls, hist);
     PSOD_LAUNCH_CHECK();
-    PSOD_TRY(psod_radix_sort_u64(ctx, n, keys, vals, 48, dn));
-    PSOD_HIP(hipMemcpyAsync(large, vals, (size_t)n * 4,
+    k_class_scatter<<<grid_for(n, 256 * ORD_V), 256, 0, st>>>(cls, large, n,
+                                                              dn, hist, ord);
+    PSOD_LAUNCH_CHECK();
+    PSOD_HIP(hipMemcpyAsync(large, ord, (size_t)n * 4,
                             hipMemcpyDeviceToDevice, st));
     return PSOD_OK;
   };
@@ -4571,7 +4661,7 @@ static int grow_giants(psod_ctx *ctx, const SodCfg &c,
       uint32_t *vals =
           (uint32_t *)psod_scratch(ctx, S_GIANT_V, (size_t)n * 4);
       if (!vals) return PSOD_E_NOMEM;
-      PSOD_TRY(psod_radix_sort_u64(ctx, n, pool + sl[1 + 2 * k], vals, 64));
+      PSOD_TRY(psod_radix_sort_u64(ctx, n, pool + sl[1 + 2 * k], vals));
     }
     k_giant_cross<<<ngiant, GL_T, 0, st>>>(c, gs, hist, pool, pool_cap,
                                            cat->pos, S.counters, S.retry,
