@@ -73,6 +73,7 @@ enum ScratchSlot {
   S_GIANT_P,   // SOD: their collection slices
   S_GIANT_SEG, // SOD: per-segment counts of their cubes, prefix sums
   S_GIANT_V,   // SOD: values of the device-wide sorts of their bands
+  S_WIN,       // SOD: windows of 8 records for the centre search
   S_NSLOT
 };
 

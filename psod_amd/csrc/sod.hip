@@ -783,11 +783,16 @@ __device__ inline uint32_t sterm_bound(float g2, float eps2) {
                     8.5f);
 }
 
-// Next block of work of a wave from a shared counter (the first active
-// lane takes it; every lane gets it): waves that finish early take more.
+// Next block of work of a wave from a shared counter (lane 0 takes it;
+// every lane gets it): waves that finish early take more.  The lane is
+// opaque to the compiler: where a loop ends in `if (lane == 0) ...;
+// continue;` it may otherwise jump straight from that branch to the one
+// here, and the lanes that skip both then read their own zero and take
+// block 0 for ever.
 __device__ inline int32_t wave_next(int32_t *ctr) {
-  int32_t v = 0;
-  if ((threadIdx.x & 63) == 0) v = atomicAdd(ctr, 1);
+  int32_t v = 0, lane = (int32_t)(threadIdx.x & 63);
+  asm volatile("" : "+v"(lane));
+  if (lane == 0) v = atomicAdd(ctr, 1);
   return __builtin_amdgcn_readfirstlane(v);
 }
 
@@ -814,6 +819,97 @@ __device__ inline uint64_t group_reduce8(const uint64_t (&u)[8], int l) {
   return v;
 }
 
+// Windows: the records [8 w, 8 w + 8) that lie inside one cell of at least
+// WIN_CELL records, which is in Morton order, so a window is compact.  For
+// the cells around the halos that the bound visits, gwin[w] = the centre of
+// the window's box (block-relative like the records) and the squared
+// distance from that centre within which a candidates' box can meet one of
+// its records.  A task's box reaches less than half of the records of its 27
+// cells; testing 64 windows at once finds them for a few instructions per 64
+// records, where testing the records themselves took 37.
+constexpr int WIN_CELL = 64, WIN_WAVES = 32;
+
+__global__ void __launch_bounds__(256)
+k_centre_windows(SodCfg c, const int32_t *__restrict__ cell_start,
+                 const float4 *__restrict__ rec,
+                 const HaloPlan *__restrict__ plan,
+                 const int32_t *__restrict__ large, int32_t nlarge,
+                 const int32_t *__restrict__ dn, float4 *__restrict__ gwin) {
+  // WIN_WAVES waves per halo share the windows of the 5^3 cells around its
+  // seed (two cells' ranges per lane), eight windows per step; two halos may
+  // write the same window, with the same values
+  const int l = threadIdx.x & 63;
+  const int32_t u = (int32_t)(blockIdx.x * 4 + (threadIdx.x >> 6));
+  const int32_t e = u / WIN_WAVES, part = u % WIN_WAVES;
+  if (e >= nlarge || (dn && e >= *dn)) return;  // uniform per wave
+  const HaloPlan pl = plan[large[e]];
+  if (pl.centre >= 0 || pl.n5 < c.bound_min) return;
+  int32_t qa[2] = {0, 0}, qb[2] = {0, 0};
+  for (int h = 0; h < 2; h++)
+    if (l + 64 * h < 125) {
+      int di, dj, dk;
+      int32_t lc[3];
+      walk_off(l + 64 * h, 2, &di, &dj, &dk);
+      const int32_t key = key_at(c.nx, pl.cs, di, dj, dk, lc);
+      qa[h] = cell_start[key];
+      qb[h] = cell_start[key + 1];
+    }
+  const float reach = sqrtf(c.rs2f * 1.0001f + 1e-6f);
+  // whole windows of each cell, and the prefix of its steps of eight windows
+  int32_t w0[2], w1[2], ex[2], tot = 0;
+  for (int h = 0; h < 2; h++) {
+    const bool on = qb[h] - qa[h] >= WIN_CELL;
+    w0[h] = (qa[h] + 7) >> 3;
+    w1[h] = on ? qb[h] >> 3 : w0[h];
+    int32_t t;
+    ex[h] = tot + wave_excl((w1[h] - w0[h] + 7) >> 3, &t);
+    tot += t;
+  }
+  // the windows of step k: the last cell whose prefix is at most k (empty
+  // cells before it share the prefix)
+  auto first_window = [&](int32_t k, int32_t *end) {
+    const uint64_t m1 = __ballot(ex[1] <= k), m0 = __ballot(ex[0] <= k);
+    const int h = m1 ? 1 : 0;
+    const int i = 63 - __clzll((unsigned long long)(m1 ? m1 : m0));
+    const int32_t a = __builtin_amdgcn_readlane(h ? w0[1] : w0[0], i);
+    *end = __builtin_amdgcn_readlane(h ? w1[1] : w1[0], i);
+    return a + 8 * (k - __builtin_amdgcn_readlane(h ? ex[1] : ex[0], i));
+  };
+  int32_t w = 0, end = 0;
+  float4 r = make_float4(0.f, 0.f, 0.f, 0.f);
+  if (part < tot) {
+    w = first_window(part, &end);
+    r = rec[min(8 * w + l, 8 * end - 1)];
+  }
+  for (int32_t k = part; k < tot; k += WIN_WAVES) {
+    int32_t wn = 0, en = 0;
+    float4 rn = r;
+    if (k + WIN_WAVES < tot) {  // the next step's records
+      wn = first_window(k + WIN_WAVES, &en);
+      rn = rec[min(8 * wn + l, 8 * en - 1)];
+    }
+    float lo[3] = {r.x, r.y, r.z}, hi[3] = {r.x, r.y, r.z};
+#pragma unroll
+    for (int o = 1; o < 8; o <<= 1)
+#pragma unroll
+      for (int d = 0; d < 3; d++) {
+        lo[d] = fminf(lo[d], __shfl_xor(lo[d], o, 64));
+        hi[d] = fmaxf(hi[d], __shfl_xor(hi[d], o, 64));
+      }
+    const float m[3] = {0.5f * (lo[0] + hi[0]), 0.5f * (lo[1] + hi[1]),
+                        0.5f * (lo[2] + hi[2])};
+    // half the box's diagonal covers its records
+    const float d[3] = {hi[0] - m[0], hi[1] - m[1], hi[2] - m[2]};
+    const float R = sqrtf(d[0] * d[0] + d[1] * d[1] + d[2] * d[2]);
+    const float t = reach + R * 1.0001f + 4e-6f;
+    if ((l & 7) == 0 && w + (l >> 3) < end)
+      gwin[w + (l >> 3)] = make_float4(m[0], m[1], m[2], t * t);
+    w = wn;
+    end = en;
+    r = rn;
+  }
+}
+
 // Phase 0 of the centre search, one wave per task: each candidate's S is at
 // most the sum, over the neighbours of the 27 cells, of the term at the
 // neighbour's distance to the box of the candidate's 16 (candidates
@@ -824,27 +920,38 @@ __device__ inline uint64_t group_reduce8(const uint64_t (&u)[8], int l) {
 // group) in cub[t*27*8 + q*8 + g], the per-group totals in
 // cub[(nt*27 + t)*8 + g], the task's bound in ubt[t] and each halo's
 // largest task bound in hpil.
-__global__ void __launch_bounds__(256)
+// 6 waves per SIMD (80 VGPRs): 73.7 -> 56.7 ms at 1024^3
+__global__ void __launch_bounds__(256, 6)
 k_centre_bound(SodCfg c, const int32_t *__restrict__ cell_start,
                const float4 *__restrict__ rec, const HaloPlan *__restrict__ plan,
                const int32_t *__restrict__ large, const int4 *__restrict__ tasks,
                const int32_t *__restrict__ ntask_total, int32_t tcap,
                unsigned long long *__restrict__ hpil,
                unsigned long long *__restrict__ ubt,
-               unsigned long long *__restrict__ cub, int32_t *__restrict__ wq) {
+               unsigned long long *__restrict__ cub,
+               const float4 *__restrict__ gwin, int32_t *__restrict__ wq) {
+  __shared__ int32_t wqueue[4][80];  // windows in reach, per wave
   // the wave index is uniform: task fields and everything derived from
   // them go to scalar registers
   const int l = threadIdx.x & 63,
             w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const uint64_t below = l == 0 ? 0ull : (~0ull >> (64 - l));  // lanes < l
   const int32_t nt = *ntask_total;
+  // Tasks taken singly: four per wave of the launch.  Two at a time left the
+  // launch waiting for the waves that got two tasks of a giant core (zoom
+  // catalogue at 512^3 5.2 -> 4.0 ms); one at a time throughout costs the
+  // shared counter (1024^3: 56.7 -> 58.0 ms).
+  const int32_t lone = (int32_t)(gridDim.x * 16);
   const float cut = c.rs2f * 1.0001f + 1e-6f;  // conservative chunk culling
   // held in a vector register: the term's fused multiply-add takes it
   // without a move per term (71.8 -> 67.9 ms at 1024^3 with the maxima below)
   const float eps2v = __shfl(c.eps2f, 0, 64);
   for (;;) {
-    const int32_t t0 = wave_next(wq) * 2;
+    // the first tasks (of the largest halos) one at a time, then two
+    const int32_t u = wave_next(wq);
+    const int32_t t0 = u < lone ? u : lone + (u - lone) * 2;
     if (t0 >= nt) break;
-    const int32_t t1 = min(nt, t0 + 2);
+    const int32_t t1 = min(nt, t0 + (u < lone ? 1 : 2));
     for (int32_t t = t0; t < t1; t++) {
       const int4 tk = tasks[t];
       const HaloPlan pl = plan[large[tk.x]];
@@ -933,113 +1040,164 @@ k_centre_bound(SodCfg c, const int32_t *__restrict__ cell_start,
       uint32_t ubg[4];
 #pragma unroll
       for (int g = 0; g < 4; g++) ubg[g] = 0;
-      int nch = 0;  // chunks summed into ubg
-      // the position after chunk (q, s): the next chunk of cell q, else the
-      // first of the next cell with records (27: none left)
+      int nch = 0;  // steps of 64 records summed into ubg
+      // Batches: 64 windows of a cell of at least WIN_CELL records, or the
+      // records of a smaller cell, both one float4 per lane.  The first
+      // element of the batch after (q, s), q = 27 when there is none:
+      auto first_of = [&](int q) {
+        if (q >= 27) return 0;
+        const int32_t a = __builtin_amdgcn_readlane(qa, q),
+                      n = __builtin_amdgcn_readlane(qb, q) - a;
+        return n >= WIN_CELL ? a >> 3 : a;
+      };
       auto next_pos = [&](int &q, int32_t &s) {
         if (q >= 27) return;
+        const int32_t a = __builtin_amdgcn_readlane(qa, q),
+                      b = __builtin_amdgcn_readlane(qb, q);
         s += 64;
-        if (s >= __builtin_amdgcn_readlane(qb, q)) {
+        if (b - a < WIN_CELL || s >= (b + 7) >> 3) {
           rest &= ~(1ull << q);
           q = rest ? __ffsll((unsigned long long)rest) - 1 : 27;
-          s = q < 27 ? __builtin_amdgcn_readlane(qa, q) : 0;
+          s = first_of(q);
         }
       };
-      // unconditional loads, clamped to the chunk's cell (rec[0] when there
-      // is no chunk): no branch around them, so each wait is for the oldest
+      // unconditional loads, clamped to the cell (element 0 when there is no
+      // batch): no branch around them, so each wait is for the oldest
       auto load = [&](int q, int32_t s) {
-        const int32_t i =
-            q < 27 ? min(s + l, __builtin_amdgcn_readlane(qb, q) - 1) : 0;
-        const float4 v = rec[i];
-        return make_float3(v.x, v.y, v.z);
+        int32_t i = 0;
+        const float4 *p = rec;
+        if (q < 27) {
+          const int32_t a = __builtin_amdgcn_readlane(qa, q),
+                        b = __builtin_amdgcn_readlane(qb, q);
+          const bool win = b - a >= WIN_CELL;
+          p = win ? gwin : rec;
+          i = min(s + l, (win ? (b + 7) >> 3 : b) - 1);
+        }
+        return p[i];
       };
-      // the terms of chunk (q, s) of records r; the cell's sums are reduced
-      // when it is the cell's last chunk
-      auto sum_chunk = [&](int q, int32_t s, const float3 &r, bool cell_end) {
-        int ei, ej, ek;
-        walk_off(q, 1, &ei, &ej, &ek);
-        const int di = ci + ei, dj = cj + ej, dk = ck + ek;
-        const bool valid = s + l < __builtin_amdgcn_readlane(qb, q);
-        // block-local coordinates of the walked cell (8 divides nx)
-        const int32_t lx = (pl.cs[0] + di) & 7, ly = (pl.cs[1] + dj) & 7,
-                      lz = (pl.cs[2] + dk) & 7;
-        float vx = 0.f, vy = 0.f, vz = 0.f;
-        bool near = false;
-        if (valid) {
-          vx = cell_rel(r.x, lx, di);
-          vy = cell_rel(r.y, ly, dj);
-          vz = cell_rel(r.z, lz, dk);
-          // within reach of the task's box (its groups lie inside it): the
-          // coordinate minus its clamp to the box
-          const float ex = vx - __builtin_amdgcn_fmed3f(vx, cb0[0], hb[0]);
-          const float ey = vy - __builtin_amdgcn_fmed3f(vy, cb0[1], hb[1]);
-          const float ez = vz - __builtin_amdgcn_fmed3f(vz, cb0[2], hb[2]);
-          near = fmaf(ex, ex, fmaf(ey, ey, ez * ez)) <= cut;
-        }
-        if (near) {
-#pragma unroll
-          for (int g = 0; g < 4; g++) {
-            if (g < nbx) {
-              // distance to the box per axis: the coordinate minus its clamp
-              const float gx = vx - __builtin_amdgcn_fmed3f(vx, B[g][0], B[g][3]);
-              const float gy = vy - __builtin_amdgcn_fmed3f(vy, B[g][1], B[g][4]);
-              const float gz = vz - __builtin_amdgcn_fmed3f(vz, B[g][2], B[g][5]);
-              const float g2 = fmaf(gx, gx, fmaf(gy, gy, gz * gz));
-              ubg[g] += g2 <= cut ? sterm_bound(g2, eps2v) : 0u;
-            }
-          }
-        }
-        if (cell_end || ++nch == 255) {
+      auto flush = [&](bool cell_end, int q) {
+        if (nch > 0) {
           uint64_t u[8];
 #pragma unroll
-          for (int g = 0; g < 8; g++) {
+          for (int g = 0; g < 8; g++)
             u[g] = g < ngr ? ubg[g >> 1] : 0;  // both groups of the box
-          }
 #pragma unroll
           for (int g = 0; g < 4; g++) ubg[g] = 0;
           cellv += group_reduce8(u, l);
           nch = 0;
-          if (cell_end) {  // the cell is done
-            tot += cellv;
-            if ((l & 7) == 0) cb[q * 8 + (l >> 3)] = cellv;
-            cellv = 0;
-          }
+        }
+        if (cell_end) {  // the cell is done
+          tot += cellv;
+          if ((l & 7) == 0) cb[q * 8 + (l >> 3)] = cellv;
+          cellv = 0;
         }
       };
-      // chunks of 64 records of the cells in turn, three in flight: slots A,
-      // B, C hold consecutive chunks; once a slot's chunk is summed, the slot
-      // requests the chunk after the last one requested (tq, ts).  With one
-      // chunk in flight the kernel took 66.7 ms at 1024^3, with three 65.3.
-      int qA = rest ? __ffsll((unsigned long long)rest) - 1 : 27;
-      int32_t sA = qA < 27 ? __builtin_amdgcn_readlane(qa, qA) : 0;
-      int qB = qA, qC;
-      int32_t sB = sA, sC;
-      next_pos(qB, sB);
-      qC = qB;
-      sC = sB;
-      next_pos(qC, sC);
-      int tq = qC;
-      int32_t ts = sC;
-      float3 rA = load(qA, sA), rB = load(qB, sB), rC = load(qC, sC);
-      for (;;) {
-        if (qA >= 27) break;
-        sum_chunk(qA, sA, rA, qB != qA);
-        next_pos(tq, ts);
-        qA = tq;
-        sA = ts;
-        rA = load(qA, sA);
-        if (qB >= 27) break;
-        sum_chunk(qB, sB, rB, qC != qB);
-        next_pos(tq, ts);
-        qB = tq;
-        sB = ts;
-        rB = load(qB, sB);
-        if (qC >= 27) break;
-        sum_chunk(qC, sC, rC, qA != qC);
-        next_pos(tq, ts);
-        qC = tq;
-        sC = ts;
-        rC = load(qC, sC);
+      // squared distance of a point from the task's box
+      auto box_d2 = [&](float x, float y, float z) {
+        const float ex = x - __builtin_amdgcn_fmed3f(x, cb0[0], hb[0]);
+        const float ey = y - __builtin_amdgcn_fmed3f(y, cb0[1], hb[1]);
+        const float ez = z - __builtin_amdgcn_fmed3f(z, cb0[2], hb[2]);
+        return fmaf(ex, ex, fmaf(ey, ey, ez * ez));
+      };
+      int q = rest ? __ffsll((unsigned long long)rest) - 1 : 27;
+      int32_t s = first_of(q);
+      int qN = q;
+      int32_t sN = s;
+      next_pos(qN, sN);
+      float4 cur = load(q, s);
+      int qn = 0;  // windows queued
+      while (q < 27) {
+        const float4 nxt = load(qN, sN);  // one batch ahead
+        int ei, ej, ek;
+        walk_off(q, 1, &ei, &ej, &ek);
+        const int di = ci + ei, dj = cj + ej, dk = ck + ek;
+        // block-local coordinates of the walked cell (8 divides nx): a
+        // record's coordinate relative to the candidates' frame is u + o
+        const float ox = (float)(di - ((pl.cs[0] + di) & 7)),
+                    oy = (float)(dj - ((pl.cs[1] + dj) & 7)),
+                    oz = (float)(dk - ((pl.cs[2] + dk) & 7));
+        const int32_t a = __builtin_amdgcn_readlane(qa, q),
+                      b = __builtin_amdgcn_readlane(qb, q);
+        const bool cell_end = qN != q;
+        const bool win = b - a >= WIN_CELL;
+        int nq = 8, lim = 1;  // a small cell: one step, every lane
+        if (win) {
+          // windows in reach of the task's box; the cell's first and last
+          // window may be shared with its neighbours: always taken
+          const int32_t wi = s + l;
+          const bool part = (wi << 3) < a || (wi << 3) + 8 > b;
+          const bool near =
+              (wi << 3) < b &&
+              (part || box_d2(cur.x + ox, cur.y + oy, cur.z + oz) <= cur.w);
+          const uint64_t m = __ballot(near);
+          if (near) wqueue[w][qn + __popcll(m & below)] = wi;
+          qn += __popcll(m);
+          __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+          __builtin_amdgcn_wave_barrier();
+          __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+          nq = qn;
+          lim = cell_end ? qn : qn - 7;  // whole steps of 8 windows only
+        }
+        // eight windows (64 records) per step, the next step's requested
+        // before this one's are used
+        auto rec_of = [&](int k) {
+          return (wqueue[w][min(k + (l >> 3), nq - 1)] << 3) + (l & 7);
+        };
+        int32_t i = s + l;
+        float4 r = cur;
+        if (win && lim > 0) {
+          i = rec_of(0);
+          r = rec[min(max(i, a), b - 1)];
+        }
+        int k = 0;
+        for (;;) {
+          const bool more = k < lim;
+          if (more) {
+            int32_t in = i;
+            float4 rn = r;
+            if (win) {
+              in = rec_of(k + 8);
+              rn = rec[min(max(in, a), b - 1)];
+            }
+            const float vx = r.x + ox, vy = r.y + oy, vz = r.z + oz;
+            if (k + (l >> 3) < nq && i >= a && i < b) {
+#pragma unroll
+              for (int g = 0; g < 4; g++) {
+                if (g < nbx) {
+                  // distance to the box per axis: the coordinate minus its
+                  // clamp
+                  const float gx =
+                      vx - __builtin_amdgcn_fmed3f(vx, B[g][0], B[g][3]);
+                  const float gy =
+                      vy - __builtin_amdgcn_fmed3f(vy, B[g][1], B[g][4]);
+                  const float gz =
+                      vz - __builtin_amdgcn_fmed3f(vz, B[g][2], B[g][5]);
+                  const float g2 = fmaf(gx, gx, fmaf(gy, gy, gz * gz));
+                  ubg[g] += g2 <= cut ? sterm_bound(g2, eps2v) : 0u;
+                }
+              }
+            }
+            k += 8;
+            nch++;
+            i = in;
+            r = rn;
+          }
+          if (nch == 255 || (!more && cell_end)) flush(!more && cell_end, q);
+          if (!more) break;
+        }
+        if (win) {  // the windows left go to the queue's head
+          const int left = max(qn - k, 0);
+          const int32_t mv = l < left ? wqueue[w][k + l] : 0;
+          __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+          __builtin_amdgcn_wave_barrier();
+          __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+          if (l < left) wqueue[w][l] = mv;
+          qn = left;
+        }
+        q = qN;
+        s = sN;
+        cur = nxt;
+        next_pos(qN, sN);
       }
       if ((l & 7) == 0) cub[((int64_t)tcap * 27 + t) * 8 + (l >> 3)] = tot;
       unsigned long long ubmax = (l >> 3) < ngr ? tot : 0ull;
@@ -4270,10 +4428,18 @@ static int centre_search(psod_ctx *ctx, const SodCfg &c,
       nb = 4;
     return (unsigned)ctx->num_cus * (unsigned)nb;
   };
+  // 2 bytes per particle: the windows of 8 records
+  float4 *gwin = (float4 *)psod_scratch(
+      ctx, S_WIN, (size_t)(cat->npart / 8 + 2) * sizeof(float4));
+  if (!gwin) return PSOD_E_NOMEM;
+  k_centre_windows<<<grid_for((int64_t)nlarge * WIN_WAVES, 4), 256, 0, st>>>(
+      c, cat->cell_start, (const float4 *)cat->rec, plan, large, nlarge, dn,
+      gwin);
+  PSOD_LAUNCH_CHECK();
   const unsigned nwg = resident((const void *)k_centre_bound);
   k_centre_bound<<<nwg, 256, 0, st>>>(c, cat->cell_start,
                                       (const float4 *)cat->rec, plan, large,
-                                      tasks, ntot, tcap, hpil, ubt, cub, wq);
+                                      tasks, ntot, tcap, hpil, ubt, cub, gwin, wq);
   PSOD_LAUNCH_CHECK();
   k_centre_pilot<<<resident((const void *)k_centre_pilot), 256, 0, st>>>(
       c, cat->cell_start, (const float4 *)cat->rec, plan, large, tasks, ntot,
