@@ -737,9 +737,13 @@ k_subsort(const int32_t *__restrict__ cs, const int32_t *__restrict__ list,
   float4 *tr = BIG ? trec + (int64_t)blockIdx.x * tcap : nullptr;
   int32_t *tp = BIG && tperm ? tperm + (int64_t)blockIdx.x * tcap : nullptr;
   int32_t *tl = BIG && tlab ? tlab + (int64_t)blockIdx.x * tcap : nullptr;
-  // cells are taken SUB_B at a time: one counter shared by every workgroup
-  // of the launch, hundreds of thousands of small cells
-  constexpr int SUB_B = BIG ? 1 : 16;
+  // Cells are taken several at a time where there are many: one counter is
+  // shared by every workgroup of the launch, hundreds of thousands of small
+  // cells at 1024^3.  Where there are few, 16 at a time left them to a few
+  // workgroups in turn (2^21 particles: 73 -> 48 us and, above SUB_W
+  // records, 51 -> 9 us).
+  const int32_t SUB_B =
+      BIG ? 1 : min(16, max(1, nl / (int32_t)(2 * gridDim.x)));
   int32_t it = 0, end = 0;
   for (;;) {
     if (it == end) {

@@ -665,6 +665,25 @@ __device__ void small_growth_and_output(const SodCfg &c, SmallLds &S,
 // ---------------------------------------------------------------------------
 // large halos: centre search tasks
 // ---------------------------------------------------------------------------
+// record range of candidate cell l (walk_off order, lanes 0..26; else empty)
+// around a halo's seed cell
+__device__ inline void cand_cell(const SodCfg &c, const int32_t *cell_start,
+                                 const HaloPlan &pl, int l, int32_t *a,
+                                 int32_t *b) {
+  *a = *b = 0;
+  if (l < 27) {
+    int di, dj, dk;
+    walk_off(l, 1, &di, &dj, &dk);
+    int32_t lc[3];
+    const int32_t key = key_at(c.nx, pl.cs, di, dj, dk, lc);
+    *a = cell_start[key];
+    *b = cell_start[key + 1];
+  }
+}
+
+// One wave per halo, a candidate cell per lane (one thread per halo wrote
+// the thousands of tasks of a giant one alone: emit 0.70 ms at 1024^3, 0.34
+// on the 512^3 zoom, 0.08 at 256^3).
 __global__ void __launch_bounds__(256)
 k_task_count(SodCfg c, const int32_t *__restrict__ cell_start,
              HaloPlan *__restrict__ plan, const int32_t *__restrict__ large,
@@ -672,25 +691,19 @@ k_task_count(SodCfg c, const int32_t *__restrict__ cell_start,
              int32_t *__restrict__ ntask) {
   // nlarge bounds the launch; with dn the halos are the first *dn (entries
   // up to nlarge beyond them count no tasks, for the scan)
-  const int32_t e = blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= nlarge) return;
-  if (dn && e >= *dn) {
-    ntask[e] = 0;
-    return;
-  }
-  const HaloPlan pl = plan[large[e]];
+  const int l = threadIdx.x & 63;
+  const int32_t e = (int32_t)(blockIdx.x * 4 + (threadIdx.x >> 6));
+  if (e >= nlarge) return;  // uniform per wave
   int32_t nt = 0;
-  if (pl.centre < 0) {
-    for (int q = 0; q < 27; q++) {
-      int di, dj, dk;
-      walk_off(q, 1, &di, &dj, &dk);
-      int32_t lc[3];
-      const int32_t key = key_at(c.nx, pl.cs, di, dj, dk, lc);
-      const int32_t n = cell_start[key + 1] - cell_start[key];
-      nt += (n + 63) / 64;
+  if (!dn || e < *dn) {
+    const HaloPlan pl = plan[large[e]];
+    if (pl.centre < 0) {
+      int32_t a, b;
+      cand_cell(c, cell_start, pl, l, &a, &b);
+      nt = wave_sum((b - a + 63) >> 6);
     }
   }
-  ntask[e] = nt;
+  if (l == 0) ntask[e] = nt;
 }
 
 __global__ void __launch_bounds__(256)
@@ -700,24 +713,33 @@ k_task_emit(SodCfg c, const int32_t *__restrict__ cell_start,
             const int32_t *__restrict__ ntask,
             const int32_t *__restrict__ task0,
             const int32_t *__restrict__ overflow, int4 *__restrict__ tasks) {
-  const int32_t e = blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= nlarge || (dn && e >= *dn)) return;
+  const int l = threadIdx.x & 63;
+  const int32_t e = (int32_t)(blockIdx.x * 4 + (threadIdx.x >> 6));
+  if (e >= nlarge || (dn && e >= *dn)) return;  // uniform per wave
   const int32_t h = large[e];
   // tasks beyond the capacity of a captured pass: none are written
   const bool none = overflow && *overflow;
-  plan[h].ntask = none ? 0 : ntask[e];
-  plan[h].task0 = none ? 0 : task0[e];
-  if (none || ntask[e] == 0) return;
+  const int32_t nt = none ? 0 : ntask[e], t0 = none ? 0 : task0[e];
   const HaloPlan pl = plan[h];
-  int32_t t = task0[e];
-  for (int q = 0; q < 27; q++) {
-    int di, dj, dk;
-    walk_off(q, 1, &di, &dj, &dk);
-    int32_t lc[3];
-    const int32_t key = key_at(c.nx, pl.cs, di, dj, dk, lc);
-    const int32_t a = cell_start[key], b = cell_start[key + 1];
-    for (int32_t s = a; s < b; s += 64)
-      tasks[t++] = make_int4(e, q, s, min(b, s + 64) - s);
+  if (l == 0) {
+    plan[h].ntask = nt;
+    plan[h].task0 = t0;
+  }
+  if (nt == 0) return;
+  int32_t a, b, tot;
+  cand_cell(c, cell_start, pl, l, &a, &b);
+  const int32_t ex = wave_excl((b - a + 63) >> 6, &tot);
+  for (int32_t t = l; t - l < tot; t += 64) {  // uniform trip count
+    // the last cell whose prefix is at most t (empty cells share it)
+    int lo = 0;
+#pragma unroll
+    for (int o = 16; o > 0; o >>= 1) {
+      const int m = min(lo + o, 26);
+      if (__shfl(ex, m, 64) <= t) lo = m;
+    }
+    const int32_t s = __shfl(a, lo, 64) + 64 * (t - __shfl(ex, lo, 64)),
+                  n = __shfl(b, lo, 64) - s;
+    if (t < tot) tasks[t0 + t] = make_int4(e, lo, s, min(n, 64));
   }
 }
 
@@ -1345,13 +1367,16 @@ __device__ __forceinline__ uint64_t pilot_walk(const SodCfg &c,
   return acc;
 }
 
-// Pilot tasks with more than pilot_big records in reach (2^14 unless
-// PSOD_PILOT_BIG says otherwise) are split into PILOT_PIECES pieces of their
-// chunks, each summed by its own wave into per-candidate totals (integers:
-// the grouping does not change S).  One wave summing a 5e7-particle halo's
-// densest task alone took 41 ms.
-constexpr int32_t PILOT_PIECES = 64;
-constexpr int32_t PILOT_BIGCAP = 1024;  // split tasks per pass; more go whole
+// Pilot tasks with more than pilot_big records in reach (2^11 unless
+// PSOD_PILOT_BIG says otherwise) are split into pieces of their chunks, at
+// least PILOT_CHUNKS of them and at most PILOT_PIECES pieces, each summed by
+// its own wave into per-candidate totals (integers: the grouping does not
+// change S).  A wave sums a chunk of 64 neighbours for its 64 candidates in
+// about 1.5 us, so a task of 2^14 records alone held a mid-size pass for
+// 0.4 ms (pilots and pieces, ms: 256^3 0.78 + 0.12 -> 0.21 + 0.15, zoom
+// catalogue at 512^3 0.82 + 0.36 -> 0.25 + 0.39, 1024^3 2.1 + 0.8 -> 1.2 +
+// 1.4).
+constexpr int32_t PILOT_PIECES = 64, PILOT_CHUNKS = 16;
 
 // Pilots, one wave per task: the 64 candidates of a task (one per lane)
 // against the 27 cells around their cell (every neighbour within 1 cell lies
@@ -1359,8 +1384,10 @@ constexpr int32_t PILOT_BIGCAP = 1024;  // split tasks per pass; more go whole
 // (every task of a halo that skipped the bound) and folds their S into
 // hbest.  Dense cells are in Morton order of their 1/8-cell sub-cells, so
 // candidate groups and neighbour chunks are compact.  A task with more than
-// pilot_big records in reach is appended to big[] (count in *nbig, its
-// per-candidate totals in pacc cleared) and left to k_centre_pilot_big.
+// pilot_big records in reach is appended to big[] (count in nbig[0], at most
+// bigcap; more go whole), its pieces (slot << 6 | piece) to units[] (count
+// in nbig[1]), its per-candidate totals in pacc are cleared, and it is left
+// to k_centre_pilot_big.
 __global__ void __launch_bounds__(256)
 k_centre_pilot(SodCfg c, const int32_t *__restrict__ cell_start,
                const float4 *__restrict__ rec, const HaloPlan *__restrict__ plan,
@@ -1371,8 +1398,8 @@ k_centre_pilot(SodCfg c, const int32_t *__restrict__ cell_start,
                const unsigned long long *__restrict__ hpil,
                const unsigned long long *__restrict__ ubt,
                unsigned long long *__restrict__ cstat,
-               int32_t pilot_big, int32_t *__restrict__ big,
-               int32_t *__restrict__ nbig,
+               int32_t pilot_big, int32_t bigcap, int32_t *__restrict__ big,
+               int32_t *__restrict__ units, int32_t *__restrict__ nbig,
                unsigned long long *__restrict__ pacc,
                int32_t *__restrict__ wq) {
   __shared__ float4 nbuf[4][64];  // one neighbour chunk per wave
@@ -1393,11 +1420,19 @@ k_centre_pilot(SodCfg c, const int32_t *__restrict__ cell_start,
       PilotSetup P;
       pilot_setup(c, cell_start, rec, pl, tk, l, cut, P);
       if (wave_sum(P.qb - P.qa) > pilot_big) {
+        const int32_t C = wave_sum((P.qb - P.qa + 63) >> 6);
+        const int32_t np = min(PILOT_PIECES, (C + PILOT_CHUNKS - 1) / PILOT_CHUNKS);
         int32_t k = 0;
-        if (l == 0) k = atomicAdd(nbig, 1);
+        if (l == 0) k = atomicAdd(&nbig[0], 1);
         k = __builtin_amdgcn_readfirstlane(k);
-        if (k < PILOT_BIGCAP) {
-          if (l == 0) big[k] = t;
+        if (k < bigcap) {
+          int32_t u = 0;
+          if (l == 0) {
+            big[k] = t;
+            u = atomicAdd(&nbig[1], np);
+          }
+          u = __builtin_amdgcn_readfirstlane(u);
+          if (l < np) units[u + l] = (k << 6) | l;
           pacc[(int64_t)k * 64 + l] = 0;
           continue;
         }
@@ -1430,8 +1465,8 @@ k_centre_pilot(SodCfg c, const int32_t *__restrict__ cell_start,
 
 // Pieces of the split pilot tasks, one wave per (task, piece): piece p of a
 // task's C chunks in reach (walk_off order of the cells) is chunks
-// [p * per, (p + 1) * per), per = ceil(C / PILOT_PIECES); its sums are
-// added to the task's per-candidate totals.
+// [p * per, (p + 1) * per), per = ceil(C / its pieces); its sums are added
+// to the task's per-candidate totals.
 __global__ void __launch_bounds__(256)
 k_centre_pilot_big(SodCfg c, const int32_t *__restrict__ cell_start,
                    const float4 *__restrict__ rec,
@@ -1439,6 +1474,7 @@ k_centre_pilot_big(SodCfg c, const int32_t *__restrict__ cell_start,
                    const int32_t *__restrict__ large,
                    const int4 *__restrict__ tasks,
                    const int32_t *__restrict__ big,
+                   const int32_t *__restrict__ units,
                    const int32_t *__restrict__ nbig,
                    unsigned long long *__restrict__ pacc,
                    unsigned long long *__restrict__ cstat,
@@ -1446,13 +1482,13 @@ k_centre_pilot_big(SodCfg c, const int32_t *__restrict__ cell_start,
   __shared__ float4 nbuf[4][64];  // one neighbour chunk per wave
   const int l = threadIdx.x & 63,
             w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-  const int32_t nu = min(*nbig, PILOT_BIGCAP) * PILOT_PIECES;
+  const int32_t nu = nbig[1];
   const float cut = c.rs2f * 1.0001f + 1e-6f;  // conservative chunk culling
   unsigned long long st_pairs = 0;
   for (;;) {
     const int32_t u = wave_next(wq);
     if (u >= nu) break;
-    const int32_t b = u / PILOT_PIECES, p = u % PILOT_PIECES;
+    const int32_t b = units[u] >> 6, p = units[u] & 63;
     const int32_t t = big[b];
     const int4 tk = tasks[t];
     const HaloPlan pl = plan[large[tk.x]];
@@ -1462,7 +1498,8 @@ k_centre_pilot_big(SodCfg c, const int32_t *__restrict__ cell_start,
     const int32_t nch = l < 27 ? (P.qb - P.qa + 63) >> 6 : 0;
     int32_t C;
     const int32_t ex = wave_excl(nch, &C);
-    const int32_t per = (C + PILOT_PIECES - 1) / PILOT_PIECES;
+    const int32_t np = min(PILOT_PIECES, (C + PILOT_CHUNKS - 1) / PILOT_CHUNKS);
+    const int32_t per = (C + np - 1) / np;
     const int32_t k0 = p * per;
     if (k0 >= C) continue;
     // the cell holding chunk k0, and that chunk's first record
@@ -1486,7 +1523,7 @@ k_centre_pilot_big(SodCfg c, const int32_t *__restrict__ cell_start,
 __global__ void __launch_bounds__(256)
 k_centre_pilot_fin(const float4 *__restrict__ rec,
                    const int4 *__restrict__ tasks,
-                   const int32_t *__restrict__ big,
+                   const int32_t *__restrict__ big, int32_t bigcap,
                    const int32_t *__restrict__ nbig,
                    const unsigned long long *__restrict__ pacc,
                    uint64_t *__restrict__ taskres,
@@ -1494,7 +1531,7 @@ k_centre_pilot_fin(const float4 *__restrict__ rec,
                    unsigned long long *__restrict__ cstat) {
   const int l = threadIdx.x & 63;
   const int32_t b = (int32_t)(blockIdx.x * 4 + (threadIdx.x >> 6));
-  if (b >= min(*nbig, PILOT_BIGCAP)) return;
+  if (b >= min(nbig[0], bigcap)) return;
   const int32_t t = big[b];
   const int4 tk = tasks[t];
   const bool have = l < tk.w;
@@ -4319,11 +4356,9 @@ __global__ void k_copy_i32(const int32_t *__restrict__ a,
 }
 
 // records in reach above which a pilot task is split; PSOD_PILOT_BIG
-// overrides the default for tests (at least 64).  Pilots plus split pieces
-// at c3 / c4 (ms): 2^13 4.1 / 2.2, 2^14 3.0 / 2.3, 2^15 3.8 / 2.6, 2^16
-// 5.0 / 2.8.
+// overrides the default for tests (at least 64).
 static int32_t pilot_big() {
-  int32_t v = 1 << 14;
+  int32_t v = 1 << 11;
   if (const char *e = getenv("PSOD_PILOT_BIG")) {
     const long long x = atoll(e);
     if (x >= 64 && x <= INT32_MAX) v = (int32_t)x;
@@ -4359,9 +4394,8 @@ static int centre_search(psod_ctx *ctx, const SodCfg &c,
                          int32_t *task0, int32_t *ntot,
                          unsigned long long *hbest, F &&after_setup) {
   hipStream_t st = ctx->stream;
-  k_task_count<<<grid_for(nlarge, 256), 256, 0, st>>>(c, cat->cell_start,
-                                                       plan, large, nlarge, dn,
-                                                       ntask);
+  k_task_count<<<grid_for(nlarge, 4), 256, 0, st>>>(c, cat->cell_start, plan,
+                                                     large, nlarge, dn, ntask);
   PSOD_LAUNCH_CHECK();
   PSOD_TRY(psod_scan_i32(ctx, ntask, task0, nlarge, ntot));
   // tcap: tasks the buffers hold, and the stride of their layout
@@ -4381,14 +4415,16 @@ static int centre_search(psod_ctx *ctx, const SodCfg &c,
   }
   PSOD_TRY(after_setup());
   if (tcap == 0) return PSOD_OK;
+  // split pilot tasks, at most (a pass has about one pilot per bounded halo)
+  const int32_t bigcap = std::min(tcap, 2 * nlarge + 64);
   // tasks, their results, bounds, bounds per (cell, group) plus the
   // per-group totals (28 x 8 per task), the results of the groups (8 per
   // task), the work list of groups and its length, then the split pilot
   // tasks and their per-candidate totals
   int4 *tasks = (int4 *)psod_scratch(
       ctx, S_TASKRES,
-      (size_t)tcap * (sizeof(int4) + 24 + 28 * 8 * 8 + 8 * 16 + 8 * 4) + 256 +
-          (size_t)PILOT_BIGCAP * (4 + 64 * 8));
+      (size_t)tcap * (sizeof(int4) + 24 + 28 * 8 * 8 + 8 * 16 + 8 * 4) + 512 +
+          (size_t)bigcap * (4 + PILOT_PIECES * 4 + 64 * 8));
   if (!tasks) return PSOD_E_NOMEM;
   uint64_t *tres = (uint64_t *)(tasks + tcap);
   unsigned long long *ubt = (unsigned long long *)(tres + 2 * (int64_t)tcap);
@@ -4400,10 +4436,11 @@ static int centre_search(psod_ctx *ctx, const SodCfg &c,
   // the count of split pilot tasks
   int32_t *wq = nitems + 4;
   int32_t *nbig = wq + 4;
-  // split pilot tasks and their per-candidate totals
-  int32_t *big = nitems + 64;
-  unsigned long long *pacc = (unsigned long long *)(big + PILOT_BIGCAP);
-  k_task_emit<<<grid_for(nlarge, 256), 256, 0, st>>>(
+  // split pilot tasks, their per-candidate totals and their pieces
+  unsigned long long *pacc = (unsigned long long *)(nitems + 64);
+  int32_t *big = (int32_t *)(pacc + (int64_t)bigcap * 64);
+  int32_t *units = big + bigcap;
+  k_task_emit<<<grid_for(nlarge, 4), 256, 0, st>>>(
       c, cat->cell_start, plan, large, nlarge, dn, ntask, task0,
       dn ? overflow : nullptr, tasks);
   PSOD_LAUNCH_CHECK();
@@ -4443,15 +4480,17 @@ static int centre_search(psod_ctx *ctx, const SodCfg &c,
   PSOD_LAUNCH_CHECK();
   k_centre_pilot<<<resident((const void *)k_centre_pilot), 256, 0, st>>>(
       c, cat->cell_start, (const float4 *)cat->rec, plan, large, tasks, ntot,
-      tres, hbest, hpil, ubt, cstat, pilot_big(), big, nbig, pacc, wq + 1);
+      tres, hbest, hpil, ubt, cstat, pilot_big(), bigcap, big, units, nbig, pacc,
+      wq + 1);
   PSOD_LAUNCH_CHECK();
   k_centre_pilot_big<<<resident((const void *)k_centre_pilot_big), 256, 0,
                        st>>>(c, cat->cell_start, (const float4 *)cat->rec,
-                             plan, large, tasks, big, nbig, pacc, cstat,
-                             wq + 3);
+                             plan, large, tasks, big, units, nbig, pacc,
+                             cstat, wq + 3);
   PSOD_LAUNCH_CHECK();
-  k_centre_pilot_fin<<<PILOT_BIGCAP / 4, 256, 0, st>>>(
-      (const float4 *)cat->rec, tasks, big, nbig, pacc, tres, hbest, cstat);
+  k_centre_pilot_fin<<<grid_for(bigcap, 4), 256, 0, st>>>(
+      (const float4 *)cat->rec, tasks, big, bigcap, nbig, pacc, tres, hbest,
+      cstat);
   PSOD_LAUNCH_CHECK();
   k_task_items<<<grid_for(tcap, 256), 256, 0, st>>>(
       tasks, ntot, tcap, ubt, hpil, cub, hbest, items, nitems, cstat);
