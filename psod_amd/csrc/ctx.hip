@@ -133,7 +133,7 @@ int psod_use_device(psod_ctx *c) {
 }
 
 int psod_finish(psod_ctx *c) {
-  if (c->capturing) return PSOD_OK;
+  if (c->capturing || c->queueing) return PSOD_OK;
   PSOD_HIP(hipStreamSynchronize(c->stream));
   return PSOD_OK;
 }

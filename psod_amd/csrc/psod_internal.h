@@ -109,6 +109,9 @@ struct psod_ctx {
   // work without waiting, device scratch may not grow, and the SOD reads
   // its work counts on the device (GraphCaps bounds them)
   int capturing;
+  // set while psod_pass queues its stages: their entry points return
+  // without waiting for the stream
+  int queueing;
   struct GraphCaps {
     int64_t tasks;  // centre-search tasks of one pass, at most
   } gcap;
