@@ -784,12 +784,6 @@ __device__ inline float box_gap2(const float *a0, const float *a1,
   return s;
 }
 
-// neighbour cells of a candidate cell, nearest first (walk_off indices:
-// the cell itself, 6 faces, 12 edges, 8 corners)
-__constant__ int8_t kCellOrder[27] = {13, 4,  10, 12, 14, 16, 22, 1,  3,
-                                      5,  7,  9,  11, 15, 17, 19, 21, 23,
-                                      25, 0,  2,  6,  8,  18, 20, 24, 26};
-
 // Halos with fewer than SodCfg::bound_min particles in the 5^3 cells around
 // the seed (a tunable, 1024 by default) skip the bound: bounding costs about
 // as much as their exact sums.  With the items abandoned cell by cell,
@@ -818,27 +812,39 @@ __device__ inline int32_t wave_next(int32_t *ctr) {
   return __builtin_amdgcn_readfirstlane(v);
 }
 
-// Sums over the wave of u[g] for 8 groups, transposed: lane l ends with the
-// sum of group l >> 3.  Each exchange step hands half of the values still
-// held to the partner lane (10 64-bit exchanges instead of 8 x 6).
-__device__ inline uint64_t group_reduce8(const uint64_t (&u)[8], int l) {
-  const bool h5 = (l & 32) != 0, h4 = (l & 16) != 0, h3 = (l & 8) != 0;
-  uint64_t a[4], b[2];
-#pragma unroll
-  for (int i = 0; i < 4; i++) {
-    const uint64_t keep = h5 ? u[i + 4] : u[i], send = h5 ? u[i] : u[i + 4];
-    a[i] = keep + __shfl_xor(send, 32, 64);
-  }
+// Sums over the wave of u[g] for 4 boxes, transposed: lane l ends with the
+// sum of box l >> 4.  Each of the first two exchanges hands half of the
+// values still held to the partner lane.
+__device__ inline uint64_t box_reduce4(const uint64_t (&u)[4], int l) {
+  const bool h5 = (l & 32) != 0, h4 = (l & 16) != 0;
+  uint64_t a[2];
 #pragma unroll
   for (int i = 0; i < 2; i++) {
-    const uint64_t keep = h4 ? a[i + 2] : a[i], send = h4 ? a[i] : a[i + 2];
-    b[i] = keep + __shfl_xor(send, 16, 64);
+    const uint64_t keep = h5 ? u[i + 2] : u[i], send = h5 ? u[i] : u[i + 2];
+    a[i] = keep + __shfl_xor(send, 32, 64);
   }
-  uint64_t v = (h3 ? b[1] : b[0]) + __shfl_xor(h3 ? b[0] : b[1], 8, 64);
-  v += __shfl_xor(v, 4, 64);
-  v += __shfl_xor(v, 2, 64);
-  v += __shfl_xor(v, 1, 64);
+  uint64_t v = (h4 ? a[1] : a[0]) + __shfl_xor(h4 ? a[0] : a[1], 16, 64);
+#pragma unroll
+  for (int o = 8; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
   return v;
+}
+
+// Sum over the 64 lanes of a float, returned wave-uniform; all lanes must be
+// active (row shifts and broadcasts as in wave_incl_scan).
+__device__ inline float wave_sumf(float x) {
+  auto mv = [](float v, auto ctrl, auto rows) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(
+        0, __float_as_int(v), decltype(ctrl)::value, decltype(rows)::value, 0xf,
+        false));
+  };
+  using std::integral_constant;
+  x += mv(x, integral_constant<int, 0x111>(), integral_constant<int, 0xf>());
+  x += mv(x, integral_constant<int, 0x112>(), integral_constant<int, 0xf>());
+  x += mv(x, integral_constant<int, 0x114>(), integral_constant<int, 0xf>());
+  x += mv(x, integral_constant<int, 0x118>(), integral_constant<int, 0xf>());
+  x += mv(x, integral_constant<int, 0x142>(), integral_constant<int, 0xa>());
+  x += mv(x, integral_constant<int, 0x143>(), integral_constant<int, 0xc>());
+  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), 63));
 }
 
 // Windows: the records [8 w, 8 w + 8) that lie inside one cell of at least
@@ -937,20 +943,18 @@ k_centre_windows(SodCfg c, const int32_t *__restrict__ cell_start,
 // neighbour's distance to the box of the candidate's 16 (candidates
 // 16b..16b+15, Morton-compact).  Boxes of 8 bound tighter but cost twice as
 // many terms; with the items taken most promising first, 16 is faster
-// (c3: 8 -> 236 ms, 16 -> 218, 32 -> 235, 64 -> 263 ms of SOD).  The bound
-// of box b serves both groups of 8 inside it: stores the bound per (cell,
-// group) in cub[t*27*8 + q*8 + g], the per-group totals in
-// cub[(nt*27 + t)*8 + g], the task's bound in ubt[t] and each halo's
+// (c3: 8 -> 236 ms, 16 -> 218, 32 -> 235, 64 -> 263 ms of SOD).  Stores the
+// bound of box b in ubx[t*4 + b], the task's bound in ubt[t] and each halo's
 // largest task bound in hpil.
 // 6 waves per SIMD (80 VGPRs): 73.7 -> 56.7 ms at 1024^3
 __global__ void __launch_bounds__(256, 6)
 k_centre_bound(SodCfg c, const int32_t *__restrict__ cell_start,
                const float4 *__restrict__ rec, const HaloPlan *__restrict__ plan,
                const int32_t *__restrict__ large, const int4 *__restrict__ tasks,
-               const int32_t *__restrict__ ntask_total, int32_t tcap,
+               const int32_t *__restrict__ ntask_total,
                unsigned long long *__restrict__ hpil,
                unsigned long long *__restrict__ ubt,
-               unsigned long long *__restrict__ cub,
+               unsigned long long *__restrict__ ubx,
                const float4 *__restrict__ gwin, int32_t *__restrict__ wq) {
   __shared__ int32_t wqueue[4][80];  // windows in reach, per wave
   // the wave index is uniform: task fields and everything derived from
@@ -1033,7 +1037,6 @@ k_centre_bound(SodCfg c, const int32_t *__restrict__ cell_start,
         B[g][4] = __shfl(g1y, 16 * g, 64);
         B[g][5] = __shfl(g1z, 16 * g, 64);
       }
-      const int ngr = (tk.w + 7) >> 3;  // groups holding candidates
       const int nbx = (tk.w + 15) >> 4;  // boxes holding candidates
       // record ranges of the 27 cells, one per lane, all loaded at once; a
       // cell beyond reach of the candidates' box gets an empty range
@@ -1051,13 +1054,9 @@ k_centre_bound(SodCfg c, const int32_t *__restrict__ cell_start,
           qb = cell_start[key + 1];
         }
       }
-      unsigned long long *cb = cub + (int64_t)t * 27 * 8;
       uint64_t rest = __ballot(l < 27 && qa < qb);  // cells with records
-      for (int i = l; i < 27 * 8; i += 64)
-        if (!((rest >> (i >> 3)) & 1)) cb[i] = 0;
-      uint64_t tot = 0;    // bound of group l >> 3 over the cells done
-      uint64_t cellv = 0;  // the same for the current cell, flushed part
-      // this lane's neighbours of the current cell, per box: at most 255
+      uint64_t tot = 0;  // bound of box l >> 4, flushed part
+      // this lane's neighbours since the last flush, per box: at most 255
       // terms of at most 2^24 + 8 each before a flush
       uint32_t ubg[4];
 #pragma unroll
@@ -1097,22 +1096,15 @@ k_centre_bound(SodCfg c, const int32_t *__restrict__ cell_start,
         }
         return p[i];
       };
-      auto flush = [&](bool cell_end, int q) {
-        if (nch > 0) {
-          uint64_t u[8];
+      auto flush = [&]() {
+        uint64_t u[4];
 #pragma unroll
-          for (int g = 0; g < 8; g++)
-            u[g] = g < ngr ? ubg[g >> 1] : 0;  // both groups of the box
-#pragma unroll
-          for (int g = 0; g < 4; g++) ubg[g] = 0;
-          cellv += group_reduce8(u, l);
-          nch = 0;
+        for (int g = 0; g < 4; g++) {
+          u[g] = ubg[g];
+          ubg[g] = 0;
         }
-        if (cell_end) {  // the cell is done
-          tot += cellv;
-          if ((l & 7) == 0) cb[q * 8 + (l >> 3)] = cellv;
-          cellv = 0;
-        }
+        tot += box_reduce4(u, l);
+        nch = 0;
       };
       // squared distance of a point from the task's box
       auto box_d2 = [&](float x, float y, float z) {
@@ -1172,9 +1164,8 @@ k_centre_bound(SodCfg c, const int32_t *__restrict__ cell_start,
           r = rec[min(max(i, a), b - 1)];
         }
         int k = 0;
-        for (;;) {
-          const bool more = k < lim;
-          if (more) {
+        while (k < lim) {
+          {
             int32_t in = i;
             float4 rn = r;
             if (win) {
@@ -1200,12 +1191,10 @@ k_centre_bound(SodCfg c, const int32_t *__restrict__ cell_start,
               }
             }
             k += 8;
-            nch++;
+            if (++nch == 255) flush();
             i = in;
             r = rn;
           }
-          if (nch == 255 || (!more && cell_end)) flush(!more && cell_end, q);
-          if (!more) break;
         }
         if (win) {  // the windows left go to the queue's head
           const int left = max(qn - k, 0);
@@ -1221,9 +1210,11 @@ k_centre_bound(SodCfg c, const int32_t *__restrict__ cell_start,
         cur = nxt;
         next_pos(qN, sN);
       }
-      if ((l & 7) == 0) cub[((int64_t)tcap * 27 + t) * 8 + (l >> 3)] = tot;
-      unsigned long long ubmax = (l >> 3) < ngr ? tot : 0ull;
-      for (int o = 32; o > 0; o >>= 1) {
+      if (nch > 0) flush();
+      if ((l & 15) == 0) ubx[(int64_t)t * 4 + (l >> 4)] = tot;
+      unsigned long long ubmax = tot;  // 0 for boxes without candidates
+#pragma unroll
+      for (int o = 32; o >= 16; o >>= 1) {
         const unsigned long long v = __shfl_xor(ubmax, o, 64);
         ubmax = v > ubmax ? v : ubmax;
       }
@@ -1548,17 +1539,16 @@ k_centre_pilot_fin(const float4 *__restrict__ rec,
   }
 }
 
-// Work list of the exact phase: item t*8 + g (g even) for every box of 16
-// candidates (groups g and g+1, which share the box's bound) of a task that
-// was not a pilot, whose bound reaches the halo's best after the pilots.  A
-// box whose bound is below the best can neither hold the maximum nor tie
-// with it.
+// Work list of the exact phase: item t*4 + b for every box b of 16
+// candidates of a task that was not a pilot, whose bound reaches the halo's
+// best after the pilots.  A box whose bound is below the best can neither
+// hold the maximum nor tie with it.
 __global__ void __launch_bounds__(256)
 k_task_items(const int4 *__restrict__ tasks,
-             const int32_t *__restrict__ ntask_total, int32_t tcap,
+             const int32_t *__restrict__ ntask_total,
              const unsigned long long *__restrict__ ubt,
              const unsigned long long *__restrict__ hpil,
-             const unsigned long long *__restrict__ cub,
+             const unsigned long long *__restrict__ ubx,
              const unsigned long long *__restrict__ hbest,
              int32_t *__restrict__ items, int32_t *__restrict__ nitems,
              unsigned long long *__restrict__ cstat) {
@@ -1571,10 +1561,10 @@ k_task_items(const int4 *__restrict__ tasks,
     const unsigned long long ub = ubt[t];
     if (ub != hpil[tk.x]) {
       const unsigned long long best = hbest[tk.x];
-      const int ngr = (tk.w + 7) >> 3;
+      const int nbx = (tk.w + 15) >> 4;
       if (ub >= best)
-        for (int g = 0; g < ngr; g += 2)
-          if (cub[((int64_t)tcap * 27 + t) * 8 + g] >= best) mask |= 1u << g;
+        for (int b = 0; b < nbx; b++)
+          if (ubx[(int64_t)t * 4 + b] >= best) mask |= 1u << b;
       skipped = mask == 0;
     }
   }
@@ -1584,9 +1574,9 @@ k_task_items(const int4 *__restrict__ tasks,
   if ((threadIdx.x & 63) == 0 && tot > 0) base = atomicAdd(nitems, tot);
   int32_t p = __shfl(base, 0, 64) + ex;
   while (mask) {
-    const int g = __ffs(mask) - 1;
+    const int b = __ffs(mask) - 1;
     mask &= mask - 1;
-    items[p++] = t * 8 + g;
+    items[p++] = t * 4 + b;
   }
   const unsigned long long ns = wave_sum((unsigned long long)(skipped ? 1 : 0));
   if ((threadIdx.x & 63) == 0 && ns) atomicAdd(&cstat[1], ns);
@@ -1661,7 +1651,7 @@ k_class_scatter(const uint8_t *__restrict__ cls,
 __global__ void __launch_bounds__(256)
 k_item_keys(const int32_t *__restrict__ items,
             const int32_t *__restrict__ nitems, const int4 *__restrict__ tasks,
-            int32_t tcap, const unsigned long long *__restrict__ cub,
+            const unsigned long long *__restrict__ ubx,
             const unsigned long long *__restrict__ hbest,
             uint8_t *__restrict__ cls, int32_t *__restrict__ hist) {
   const int32_t i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -1670,9 +1660,8 @@ k_item_keys(const int32_t *__restrict__ items,
   uint32_t k = 0;
   if (i < n) {
     const int32_t it = items[i];
-    const int32_t t = it >> 3, g = it & 7;
-    const double ub = (double)cub[((int64_t)tcap * 27 + t) * 8 + g];
-    const double b = (double)hbest[tasks[t].x];
+    const double ub = (double)ubx[it];
+    const double b = (double)hbest[tasks[it >> 2].x];
     const double r = b > 0.0 ? ub / b : 5.0;
     k = 255u - (uint32_t)fmax(0.0, fmin((r - 1.0) * 64.0, 255.0));
     cls[i] = (uint8_t)k;
@@ -1680,41 +1669,60 @@ k_item_keys(const int32_t *__restrict__ items,
   count_class(i < n, k, hist);
 }
 
-// Exact phase, one wave per item (task t, candidates 8g..8g+15).  Lane l
-// takes candidate l & 15.  The neighbours within reach of the item's box are
-// queued in LDS across chunks and cells and taken 64 at a time, neighbour
-// u + (l >> 4) by lane l in steps of 4, so that every step evaluates 64
-// pairs.  Each pair's term comes from the same operands and operations as in
-// the pilots (neighbour minus candidate, the same fused squares), so S is
-// the same integer.  After each cell (nearest first: the cell itself, the 6
-// faces, the 12 edges, the 8 corners) the queue is drained and the item is
-// abandoned when no candidate's exact sum so far plus the bound of the
-// cells left reaches the halo's best.  A drain pads at most 3 entries, so
-// checking after every cell rather than every shell of cells costs little
-// and abandons earlier (44.4 -> 39.7 ms at 1024^3, 8% fewer pair tests).
-// Items of 8 candidates (the bound's boxes were of 8 then) took 236 ms of
-// SOD at c3 against 193 ms with boxes and items of 16.
-// 5 waves per SIMD (94 VGPRs, a few spilled): 48.2 -> 46.5 ms at 1024^3
-__global__ void __launch_bounds__(256, 5)
+// neighbour cells of a candidate cell, nearest first (walk_off indices:
+// the cell itself, 6 faces, 12 edges, 8 corners)
+__constant__ int8_t kCellOrder[27] = {13, 4,  10, 12, 14, 16, 22, 1,  3,
+                                      5,  7,  9,  11, 15, 17, 19, 21, 23,
+                                      25, 0,  2,  6,  8,  18, 20, 24, 26};
+
+// Exact phase, one wave per item (box b of task t, candidates 16b..16b+15).
+// Lane l takes candidate l & 15.  The neighbours within reach of the item's
+// box are queued in LDS across chunks and cells (nearest cells first) and
+// taken 64 at a time, neighbour u + (l >> 4) by lane l in steps of 4, so
+// that every step evaluates 64 pairs.  Each pair's term comes from the same
+// operands and operations as in the pilots (neighbour minus candidate, the
+// same fused squares), so S is the same integer.
+//
+// The item's bound is a sum of one term per neighbour, so the bound of the
+// neighbours not yet summed is the item's bound minus the terms of those
+// that were: every GRP_CHECK batches of 64 the item is abandoned when no
+// candidate's exact sum so far plus that reaches the halo's best.  On
+// sampled halos (n5 5e3..8e4) an item needs 35% of its neighbours; checked
+// at the ends of the cells, against bounds kept per cell, 46%.  The pair
+// tests run at the issue rate of their 13 instructions, so fewer of them is
+// what helps.  Taking the neighbours in shells of distance (windows by
+// their centre, 3 or 5 shells) needs 23-30% of them, but its window tests
+// and its registers cost what that saves (1024^3 36.9 ms against 39.7, zoom
+// catalogue at 512^3 11.5 against 9.6, 256^3 1.00 against 0.86; bounds per
+// cell 41.4, 10.0 and 0.85, and 0.1-4 ms more in the bound).  4 waves per
+// SIMD (128 VGPRs); 5 with a few spilled: 38.7, 10.3 and 0.87.
+constexpr int GRP_CHECK = 4;
+
+__global__ void __launch_bounds__(256, 4)
 k_centre_group(SodCfg c, const int32_t *__restrict__ cell_start,
                const float4 *__restrict__ rec, const HaloPlan *__restrict__ plan,
                const int32_t *__restrict__ large, const int4 *__restrict__ tasks,
-               const int32_t *__restrict__ ntask_total, int32_t tcap,
                const int32_t *__restrict__ items,
                const int32_t *__restrict__ nitems,
                unsigned long long *__restrict__ hbest,
-               const unsigned long long *__restrict__ cub,
+               const unsigned long long *__restrict__ ubx,
                uint64_t *__restrict__ itemres,
                unsigned long long *__restrict__ cstat,
                int32_t *__restrict__ wq) {
   __shared__ float4 gq[4][128];  // queued neighbours, one queue per wave
   const int l = threadIdx.x & 63,
             w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-  const int32_t nt = *ntask_total, ni = *nitems;
+  const int32_t ni = *nitems;
   const float cut = c.rs2f * 1.0001f + 1e-6f;  // conservative culling
+  const float eps2v = __shfl(c.eps2f, 0, 64);
   const uint64_t below = l == 0 ? 0ull : (~0ull >> (64 - l));  // lanes < l
   // this wave's statistics, added once at the end
   unsigned long long st_done = 0, st_skip = 0, st_abort = 0, st_pairs = 0;
+  auto lds_fence = [] {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  };
   // blocks of 2 items in list order (most promising first)
   for (;;) {
     const int32_t i0 = wave_next(wq) * 2;
@@ -1722,16 +1730,17 @@ k_centre_group(SodCfg c, const int32_t *__restrict__ cell_start,
     const int32_t i1 = min(ni, i0 + 2);
     for (int32_t i = i0; i < i1; i++) {
       const int32_t it = items[i];
-      const int32_t t = it >> 3, g = it & 7;
-      const int4 tk = tasks[t];
+      const int4 tk = tasks[it >> 2];
+      const int32_t first = 16 * (it & 3);
       uint64_t *res = itemres + 2 * (int64_t)it;
       unsigned long long best = __hip_atomic_load(
           &hbest[tk.x], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      if (cub[((int64_t)tcap * 27 + t) * 8 + g] < best) {
+      const unsigned long long bound = ubx[it];
+      if (bound < best) {
+        st_skip++;
         if (l == 0) {
           res[0] = 0;
           res[1] = ~0ull;
-          st_skip++;
         }
         continue;
       }
@@ -1740,13 +1749,13 @@ k_centre_group(SodCfg c, const int32_t *__restrict__ cell_start,
       walk_off(tk.y, 1, &ci, &cj, &ck);
       int32_t lc[3];
       key_at(c.nx, pl.cs, ci, cj, ck, lc);
-      const int nc = min(16, tk.w - 8 * g);  // candidates of the item
-      const int kc = l & 15;                // this lane's candidate
+      const int nc = min(16, tk.w - first);  // candidates of the item
+      const int kc = l & 15;                 // this lane's candidate
       // lanes of missing candidates sit beyond every cutoff
       float px = 1e30f, py = 1e30f, pz = 1e30f;
       int32_t pidx = 0;
       if (kc < nc) {
-        const float4 r = rec[tk.z + 8 * g + kc];
+        const float4 r = rec[tk.z + first + kc];
         px = cell_rel(r.x, lc[0], ci);
         py = cell_rel(r.y, lc[1], cj);
         pz = cell_rel(r.z, lc[2], ck);
@@ -1762,11 +1771,17 @@ k_centre_group(SodCfg c, const int32_t *__restrict__ cell_start,
       // the maxima in vector registers: v_med3 takes one scalar operand
       const float hb[3] = {__shfl(gb1[0], 0, 64), __shfl(gb1[1], 0, 64),
                            __shfl(gb1[2], 0, 64)};
-      // record ranges of the 27 cells nearest first and the item's bound in
-      // each, one per lane; a cell beyond reach of the item's box is empty
-      // (its bound is 0: none of its records is within reach of the group)
+      // squared distance from the item's box, computed as in the bound
+      auto box_d2 = [&](float x, float y, float z) {
+        const float ex = x - __builtin_amdgcn_fmed3f(x, gb0[0], hb[0]);
+        const float ey = y - __builtin_amdgcn_fmed3f(y, gb0[1], hb[1]);
+        const float ez = z - __builtin_amdgcn_fmed3f(z, gb0[2], hb[2]);
+        return fmaf(ex, ex, fmaf(ey, ey, ez * ez));
+      };
+      // record ranges of the 27 cells nearest first, one per lane; a cell
+      // beyond reach of the item's box is empty (none of its records is in
+      // the bound)
       int32_t qa = 0, qb = 0, cq = 0;
-      unsigned long long qbnd = 0;
       if (l < 27) {
         const int q = kCellOrder[l];
         cq = q;
@@ -1781,13 +1796,6 @@ k_centre_group(SodCfg c, const int32_t *__restrict__ cell_start,
           qa = cell_start[key];
           qb = cell_start[key + 1];
         }
-        qbnd = cub[(int64_t)t * 27 * 8 + q * 8 + g];
-      }
-      // bound of cells qi.. (nearest-first order): suffix sums over lanes
-#pragma unroll
-      for (int o = 1; o < 32; o <<= 1) {
-        const unsigned long long v = __shfl_down(qbnd, o, 64);
-        if (l + o < 27) qbnd += v;
       }
       uint64_t rest = __ballot(l < 27 && qa < qb);  // cells with records
       int qi = rest ? __ffsll((unsigned long long)rest) - 1 : 27;
@@ -1795,14 +1803,13 @@ k_centre_group(SodCfg c, const int32_t *__restrict__ cell_start,
       float4 rn = make_float4(0.f, 0.f, 0.f, 0.f);
       if (qi < 27 && s + l < __builtin_amdgcn_readlane(qb, qi)) rn = rec[s + l];
       // this lane's share of its candidate's sum: u32 steps of at most 2^24,
-      // folded into acc64 before 255 steps
+      // folded into acc64 before 255 steps; the bound terms of the
+      // neighbours that it queued
       uint32_t part = 0;
-      int nst = 0, qlen = 0;
-      uint64_t acc64 = 0, npair = 0;
+      int nst = 0, qlen = 0, nbat = 0;
+      uint64_t acc64 = 0, bt = 0;
+      uint32_t nsum = 0;  // batches summed
       bool aborted = false;
-      // n queued neighbours from the queue's head, 8 per step
-      // the queue's first 8 * ns entries, 8 per step (entries past the
-      // queued ones are padding beyond every cutoff)
       auto pair_step = [&](int j) {
         const float4 qv = gq[w][j];
         const float dx = qv.x - px, dy = qv.y - py, dz = qv.z - pz;
@@ -1837,88 +1844,74 @@ k_centre_group(SodCfg c, const int32_t *__restrict__ cell_start,
         // block-local coordinates of the walked cell (8 divides nx)
         const int32_t lx = (pl.cs[0] + di) & 7, ly = (pl.cs[1] + dj) & 7,
                       lz = (pl.cs[2] + dk) & 7;
-        bool near = false;
-        float vx = 0.f, vy = 0.f, vz = 0.f;
-        if (l < m) {
-          vx = cell_rel(r.x, lx, di);
-          vy = cell_rel(r.y, ly, dj);
-          vz = cell_rel(r.z, lz, dk);
-          // the coordinate minus its clamp to the item's box
-          const float ex = vx - __builtin_amdgcn_fmed3f(vx, gb0[0], hb[0]);
-          const float ey = vy - __builtin_amdgcn_fmed3f(vy, gb0[1], hb[1]);
-          const float ez = vz - __builtin_amdgcn_fmed3f(vz, gb0[2], hb[2]);
-          near = fmaf(ex, ex, fmaf(ey, ey, ez * ez)) <= cut;
-        }
+        const float vx = cell_rel(r.x, lx, di), vy = cell_rel(r.y, ly, dj),
+                    vz = cell_rel(r.z, lz, dk);
+        const float g2 = box_d2(vx, vy, vz);
+        const bool near = l < m && g2 <= cut;
         const uint64_t nm = __ballot(near);
-        const int nn = __popcll(nm);
-        if (near) gq[w][qlen + __popcll(nm & below)] = make_float4(vx, vy, vz, 0.f);
-        qlen += nn;
-        npair += (uint64_t)nn;
-        const bool cell_end = qn != qi;
-        if (qlen >= 64 || (cell_end && qlen > 0)) {
-          __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-          __builtin_amdgcn_wave_barrier();
-          __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-          if (qlen >= 64) {
-            // 64 entries in 8 steps at fixed LDS offsets
-            fold(16);
-#pragma unroll
-            for (int u = 0; u < 16; u++) pair_step(4 * u + (l >> 4));
-            // move the entries past them to the queue's head
-            qlen -= 64;
-            float4 mv = make_float4(0.f, 0.f, 0.f, 0.f);
-            if (l < qlen) mv = gq[w][64 + l];
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-            if (l < qlen) gq[w][l] = mv;
-          }
-          if (cell_end && qlen > 0) {
-            // at most 63 left: pad to a multiple of 8 and take them too
-            const int ns = (qlen + 3) >> 2;
-            if (l >= qlen && l < 4 * ns)
-              gq[w][l] = make_float4(1e30f, 1e30f, 1e30f, 0.f);
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-            fold(ns);
-            for (int u = 0; u < ns; u++) pair_step(4 * u + (l >> 4));
-            qlen = 0;
-          }
-          __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-          __builtin_amdgcn_wave_barrier();
-          __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        if (near) {
+          gq[w][qlen + __popcll(nm & below)] = make_float4(vx, vy, vz, 0.f);
+          bt += sterm_bound(g2, eps2v);
         }
-        if (cell_end && qn < 27) {
-          // every cell before qn is summed, the cells from qn on are bounded
-          acc64 += part;
-          part = 0;
-          nst = 0;
-          uint64_t v = acc64;  // sum over the 4 lanes of each candidate
-          v += __shfl_xor(v, 16, 64);
-          v += __shfl_xor(v, 32, 64);
-          const uint32_t blo = __builtin_amdgcn_readlane((uint32_t)qbnd, qn);
-          const uint32_t bhi =
-              __builtin_amdgcn_readlane((uint32_t)(qbnd >> 32), qn);
-          const unsigned long long rem = ((unsigned long long)bhi << 32) | blo;
-          if (__ballot(l < nc && v + rem >= best) == 0) {
-            aborted = true;
-            break;
+        qlen += __popcll(nm);
+        if (qlen >= 64) {
+          lds_fence();
+          fold(16);
+#pragma unroll
+          for (int u = 0; u < 16; u++) pair_step(4 * u + (l >> 4));
+          nsum++;
+          // the entries past them go to the queue's head
+          qlen -= 64;
+          float4 mv = make_float4(0.f, 0.f, 0.f, 0.f);
+          if (l < qlen) mv = gq[w][64 + l];
+          lds_fence();
+          if (l < qlen) gq[w][l] = mv;
+          lds_fence();
+          if (++nbat == GRP_CHECK) {
+            nbat = 0;
+            // The bound of the neighbours not summed (unseen, or queued) in
+            // floats: each of its three parts is good to 1e-6 of the whole.
+            float seen = (float)bt;
+            if (l < qlen)
+              seen -= (float)sterm_bound(box_d2(mv.x, mv.y, mv.z), eps2v);
+            const float all = (float)bound;
+            const float left = fmaxf(all - wave_sumf(seen), 0.f) + 4e-6f * all;
+            acc64 += part;
+            part = 0;
+            nst = 0;
+            uint64_t v = acc64;  // sum over the 4 lanes of each candidate
+            v += __shfl_xor(v, 16, 64);
+            v += __shfl_xor(v, 32, 64);
+            best = __hip_atomic_load(&hbest[tk.x], __ATOMIC_RELAXED,
+                                     __HIP_MEMORY_SCOPE_AGENT);
+            if (__ballot(l < nc && v + (uint64_t)left + 1 >= best) == 0) {
+              aborted = true;
+              break;
+            }
           }
-          best = __hip_atomic_load(&hbest[tk.x], __ATOMIC_RELAXED,
-                                   __HIP_MEMORY_SCOPE_AGENT);
         }
         qi = qn;
         s = sn;
       }
       if (aborted) {
+        st_abort++;
+        st_pairs += 64ull * nsum * (uint64_t)nc;
         if (l == 0) {
           res[0] = 0;
           res[1] = ~0ull;
-          st_abort++;
-          st_pairs += npair * (uint64_t)nc;
         }
         continue;
+      }
+      st_pairs += (64ull * nsum + qlen) * (uint64_t)nc;
+      // the queue's rest, at most 63, padded with entries beyond every cutoff
+      if (qlen > 0) {
+        const int ns = (qlen + 3) >> 2;
+        if (l >= qlen && l < 4 * ns)
+          gq[w][l] = make_float4(1e30f, 1e30f, 1e30f, 0.f);
+        lds_fence();
+        fold(ns);
+        for (int u = 0; u < ns; u++) pair_step(4 * u + (l >> 4));
+        lds_fence();
       }
       acc64 += part;
       uint64_t tot = acc64;  // sum over the 4 lanes of each candidate
@@ -1929,12 +1922,11 @@ k_centre_group(SodCfg c, const int32_t *__restrict__ cell_start,
       uint64_t key = l < nc ? (((uint64_t)(uint32_t)tk.y << 32) | (uint32_t)pidx)
                             : ~0ull;
       wave_argmax(acc, key);
+      st_done++;
       if (l == 0) {
         res[0] = acc;
         res[1] = key;
         atomicMax(&hbest[tk.x], (unsigned long long)acc);
-        st_done++;
-        st_pairs += npair * (uint64_t)nc;
       }
     }
   }
@@ -1972,8 +1964,8 @@ k_centre_reduce(HaloPlan *__restrict__ plan, const int32_t *__restrict__ large,
   for (int32_t t = pl.task0 + l; t < pl.task0 + pl.ntask; t += 64) {
     const uint64_t a = taskres[2 * (int64_t)t], k = taskres[2 * (int64_t)t + 1];
     if (better(a, k, ba, bk)) { ba = a; bk = k; }
-    for (int g = 0; g < 8; g++) {
-      const int64_t it = (int64_t)t * 8 + g;
+    for (int b = 0; b < 4; b++) {
+      const int64_t it = (int64_t)t * 4 + b;
       const uint64_t a2 = itemres[2 * it], k2 = itemres[2 * it + 1];
       if (better(a2, k2, ba, bk)) { ba = a2; bk = k2; }
     }
@@ -4417,21 +4409,20 @@ static int centre_search(psod_ctx *ctx, const SodCfg &c,
   if (tcap == 0) return PSOD_OK;
   // split pilot tasks, at most (a pass has about one pilot per bounded halo)
   const int32_t bigcap = std::min(tcap, 2 * nlarge + 64);
-  // tasks, their results, bounds, bounds per (cell, group) plus the
-  // per-group totals (28 x 8 per task), the results of the groups (8 per
-  // task), the work list of groups and its length, then the split pilot
+  // tasks, their results, bounds, the bounds and results of their boxes (4
+  // per task), the work list of boxes and its length, then the split pilot
   // tasks and their per-candidate totals
   int4 *tasks = (int4 *)psod_scratch(
       ctx, S_TASKRES,
-      (size_t)tcap * (sizeof(int4) + 24 + 28 * 8 * 8 + 8 * 16 + 8 * 4) + 512 +
+      (size_t)tcap * (sizeof(int4) + 24 + 4 * 8 + 4 * 16 + 4 * 4) + 512 +
           (size_t)bigcap * (4 + PILOT_PIECES * 4 + 64 * 8));
   if (!tasks) return PSOD_E_NOMEM;
   uint64_t *tres = (uint64_t *)(tasks + tcap);
   unsigned long long *ubt = (unsigned long long *)(tres + 2 * (int64_t)tcap);
-  unsigned long long *cub = ubt + tcap;
-  uint64_t *ires = (uint64_t *)(cub + (int64_t)tcap * 28 * 8);
-  int32_t *items = (int32_t *)(ires + 16 * (int64_t)tcap);
-  int32_t *nitems = items + 8 * (int64_t)tcap;
+  unsigned long long *ubx = ubt + tcap;
+  uint64_t *ires = (uint64_t *)(ubx + 4 * (int64_t)tcap);
+  int32_t *items = (int32_t *)(ires + 8 * (int64_t)tcap);
+  int32_t *nitems = items + 4 * (int64_t)tcap;
   // work counters of the bound, pilot, group and split-pilot launches, and
   // the count of split pilot tasks
   int32_t *wq = nitems + 4;
@@ -4446,8 +4437,8 @@ static int centre_search(psod_ctx *ctx, const SodCfg &c,
   PSOD_LAUNCH_CHECK();
   k_res_init<<<grid_for(tcap, 256), 256, 0, st>>>(tres, tcap);
   PSOD_LAUNCH_CHECK();
-  k_res_init<<<grid_for(8 * (int64_t)tcap, 256), 256, 0, st>>>(
-      ires, 8 * (int64_t)tcap);
+  k_res_init<<<grid_for(4 * (int64_t)tcap, 256), 256, 0, st>>>(
+      ires, 4 * (int64_t)tcap);
   PSOD_LAUNCH_CHECK();
   // hbest[nlarge..nlarge+3]: units evaluated, units skipped, pair tests,
   // units abandoned; then each halo's largest task bound
@@ -4476,7 +4467,7 @@ static int centre_search(psod_ctx *ctx, const SodCfg &c,
   const unsigned nwg = resident((const void *)k_centre_bound);
   k_centre_bound<<<nwg, 256, 0, st>>>(c, cat->cell_start,
                                       (const float4 *)cat->rec, plan, large,
-                                      tasks, ntot, tcap, hpil, ubt, cub, gwin, wq);
+                                      tasks, ntot, hpil, ubt, ubx, gwin, wq);
   PSOD_LAUNCH_CHECK();
   k_centre_pilot<<<resident((const void *)k_centre_pilot), 256, 0, st>>>(
       c, cat->cell_start, (const float4 *)cat->rec, plan, large, tasks, ntot,
@@ -4493,10 +4484,10 @@ static int centre_search(psod_ctx *ctx, const SodCfg &c,
       cstat);
   PSOD_LAUNCH_CHECK();
   k_task_items<<<grid_for(tcap, 256), 256, 0, st>>>(
-      tasks, ntot, tcap, ubt, hpil, cub, hbest, items, nitems, cstat);
+      tasks, ntot, ubt, hpil, ubx, hbest, items, nitems, cstat);
   PSOD_LAUNCH_CHECK();
   // items sorted by their bound over the halo's best, largest first
-  int32_t ni = 8 * tcap;  // capacity (device count) or the exact count
+  int32_t ni = 4 * tcap;  // capacity (device count) or the exact count
   if (!dn) {
     PSOD_HIP(hipMemcpyAsync(&ni, nitems, 4, hipMemcpyDeviceToHost, st));
     PSOD_HIP(hipStreamSynchronize(st));
@@ -4508,8 +4499,8 @@ static int centre_search(psod_ctx *ctx, const SodCfg &c,
     if (!hist || !ord) return PSOD_E_NOMEM;
     uint8_t *cls = (uint8_t *)(hist + 512);
     PSOD_TRY(psod_fill_i32(ctx, hist, 512, 0));
-    k_item_keys<<<grid_for(ni, 256), 256, 0, st>>>(items, nitems, tasks, tcap,
-                                                   cub, hbest, cls, hist);
+    k_item_keys<<<grid_for(ni, 256), 256, 0, st>>>(items, nitems, tasks, ubx,
+                                                   hbest, cls, hist);
     PSOD_LAUNCH_CHECK();
     k_class_scatter<<<grid_for(ni, 256 * ORD_V), 256, 0, st>>>(
         cls, items, ni, nitems, hist, ord);
@@ -4517,8 +4508,8 @@ static int centre_search(psod_ctx *ctx, const SodCfg &c,
     list = ord;
   }
   k_centre_group<<<resident((const void *)k_centre_group), 256, 0, st>>>(
-      c, cat->cell_start, (const float4 *)cat->rec, plan, large, tasks, ntot,
-      tcap, list, nitems, hbest, cub, ires, cstat, wq + 2);
+      c, cat->cell_start, (const float4 *)cat->rec, plan, large, tasks, list,
+      nitems, hbest, ubx, ires, cstat, wq + 2);
   PSOD_LAUNCH_CHECK();
   k_centre_reduce<<<grid_for(nlarge, 4), 256, 0, st>>>(plan, large, nlarge, dn,
                                                        tres, ires);
