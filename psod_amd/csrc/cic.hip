@@ -14,9 +14,9 @@
 // its 8^3 block, and R*u - floor(R*u) is exact for R in {1, 2}.  Each lane
 // takes K consecutive particles of the sorted list and keeps the 8 node sums
 // in registers while they share the same lower node (dense cells), adding
-// them to LDS only when it changes (the upper x plane stays in registers
-// when the next particle lies in the next cell along x).  Tiles are dispatched densest first, so
-// that the long tiles of halo cores overlap the rest.
+// them to LDS only when it changes.  Tiles are dispatched densest first, so
+// that the long tiles of halo cores overlap the rest; the largest are cut
+// into pieces whose node sums meet in memory.
 #include "psod_internal.h"
 
 #include <algorithm>
@@ -87,17 +87,35 @@ __device__ inline void tile_seg(int s, int *bi, int *bj, int *bk, int *loc,
 constexpr int DEP_T = 512;  // threads of a deposit workgroup (one tile)
 constexpr int DEP_K = 4;  // consecutive particles per lane
 constexpr int32_t DEP_CAPD = 8192;  // dense tiles dispatched first, at most
+// Tiles of at least DEP_BIG own particles are deposited in pieces of about
+// DEP_PIECE of them, one workgroup each: a 6e6-particle halo's central tile
+// alone held the launch for 2.6 ms (1.1 for the rest of 512^3).
+constexpr int32_t DEP_BIG = 1 << 17, DEP_PIECE = 1 << 15, DEP_BIGCAP = 512;
+
+// Tiles cut into pieces: count[0] tiles (slots), count[1] pieces; slot s is
+// tile[s], in np[s] pieces, done[s] of them finished, its node sums in
+// acc[s * 4096 ..]; unit[u] = (slot, piece).  cap = 0: none.
+struct BigTiles {
+  int32_t cap, ucap;
+  int32_t *count, *tile, *np, *done;
+  int2 *unit;
+  unsigned long long *acc;
+};
 
 // Dense tiles (at least dense_tile own particles, a tunable) are listed so
 // that they are dispatched first: their long runs then overlap the rest
-// instead of trailing it.  listed[tile] = 1 for a tile in dlist.
+// instead of trailing it.  listed[tile] = 1 for a tile in dlist or in B.
+// Clears the node sums of B's slots as well (any grid of at least ntile
+// threads).
 __global__ void k_tile_dense(const int32_t *__restrict__ cell_start,
                              int32_t nb, int32_t TB, int32_t ntile, int32_t capd,
                              int32_t dense_tile,
                              int32_t *__restrict__ listed,
                              int32_t *__restrict__ dcount,
-                             int32_t *__restrict__ dlist) {
+                             int32_t *__restrict__ dlist, BigTiles B) {
   const int32_t tile = blockIdx.x * blockDim.x + threadIdx.x;
+  for (int32_t i = tile; i < B.cap * 4096; i += gridDim.x * blockDim.x)
+    B.acc[i] = 0ull;
   if (tile >= ntile) return;
   const int32_t nt = nb / TB;
   const int tx = tile % nt, ty = (tile / nt) % nt, tz = tile / (nt * nt);
@@ -108,7 +126,19 @@ __global__ void k_tile_dense(const int32_t *__restrict__ cell_start,
       n += cell_start[(b0 + TB) * BS3] - cell_start[b0 * BS3];
     }
   int32_t f = 0;
-  if (n >= dense_tile) {
+  if (B.cap > 0 && n >= DEP_BIG) {
+    const int32_t s = atomicAdd(&B.count[0], 1);
+    if (s < B.cap) {
+      const int32_t np = (n + DEP_PIECE - 1) / DEP_PIECE,
+                    u = atomicAdd(&B.count[1], np);
+      B.tile[s] = tile;
+      B.np[s] = np;
+      B.done[s] = 0;
+      for (int32_t i = 0; i < np; i++) B.unit[u + i] = make_int2(s, i);
+      f = 1;
+    }
+  }
+  if (!f && n >= dense_tile) {
     const int32_t k = atomicAdd(dcount, 1);
     if (k < capd) {
       dlist[k] = tile;
@@ -132,9 +162,26 @@ __device__ inline int32_t tile_of_block(int32_t b, int32_t ntile, int32_t capd,
   return (capd > 0 && listed[tile]) ? -1 : tile;
 }
 
+// x within [0,1]; 0 for NaN
+__device__ inline float clamp01(float x) {
+  return __builtin_amdgcn_fmed3f(x, 0.0f, 1.0f);
+}
+
 // Deposit of the (8*TB*R)^3 nodes owned by one tile.  Own particles come
-// from TB^2 contiguous runs of TB blocks; halo particles from the ranges of
-// tile_seg(), found by binary search on their prefix counts.
+// from the TB^3 blocks, in runs of TB; halo particles from the ranges of
+// tile_seg(), found by binary search on their prefix counts.  The first
+// B.ucap workgroups take the pieces of the tiles in B.
+//
+// A weight becomes 2^36 fixed point by one rounding to an integer float
+// (v_rndne) and an FP64 add onto 2^52: the low bits of the sum are the
+// integer sum, exact up to 2^16 unit weights, and leave the register by one
+// 64-bit subtraction.  Bound by VALU issue (85 %) and the LDS atomics
+// together, at 1.9 TB/s of records and nodes: 1024^3 8.66 -> 8.0 ms, zoom
+// catalogue at 512^3 (with the pieces) 2.66 -> 1.10 ms, 256^3 on 512^3 nodes
+// 0.42 -> 0.40 ms.  Slower at 1024^3: a margin of nodes in LDS instead of the
+// bounds checks (9.2: fewer waves fit), 2, 3 or 8 particles per lane (9.0,
+// 8.7, 10.9), the upper x plane kept in registers when the next particle lies
+// in the next cell (8.2), workgroups of 1024 (11.0).
 template <int R, int TB>
 __global__ void __launch_bounds__(DEP_T)
 k_cic_deposit(const int32_t *__restrict__ cell_start,
@@ -142,33 +189,42 @@ k_cic_deposit(const int32_t *__restrict__ cell_start,
               int32_t shift, double norm, int32_t capd,
               const int32_t *__restrict__ dcount,
               const int32_t *__restrict__ dlist,
-              const int32_t *__restrict__ listed, float *__restrict__ grid) {
+              const int32_t *__restrict__ listed, BigTiles B,
+              float *__restrict__ grid) {
   constexpr int NN = 8 * TB * R;  // owned nodes per axis
   constexpr int NS = TileSegs<TB>::N;
+  constexpr int NB = TB * TB * TB;  // own blocks
   __shared__ unsigned long long acc[NN * NN * NN];
   __shared__ int32_t hstart[NS];
   __shared__ int32_t hpre[NS + 1];
-  __shared__ int8_t hoff[NS][3];
-  __shared__ int32_t ostart[TB * TB], opre[TB * TB + 1];
-  __shared__ int32_t obnd[TB * TB][TB];  // own-list position of each block
-  __shared__ int32_t wtot[DEP_T / 64];
+  __shared__ uint16_t hoff[NS];  // block offset, each axis + 2 in 4 bits
+  __shared__ int32_t ostart[NB], opre[NB + 1];  // own blocks, x fastest
+  __shared__ int32_t wtot[DEP_T / 64], lastpiece;
   const int32_t nb = nx >> 3;
   const int32_t nt = nb / TB;  // tiles per axis
-  const int32_t tile = tile_of_block(blockIdx.x, nt * nt * nt, capd, dcount,
-                                     dlist, listed);
+  int32_t tile, slot = -1, piece = 0, np = 1;
+  if ((int32_t)blockIdx.x < B.ucap) {
+    if ((int32_t)blockIdx.x >= B.count[1]) return;
+    const int2 u = B.unit[blockIdx.x];
+    slot = u.x;
+    piece = u.y;
+    np = B.np[slot];
+    tile = B.tile[slot];
+  } else {
+    tile = tile_of_block((int32_t)blockIdx.x - B.ucap, nt * nt * nt, capd,
+                         dcount, dlist, listed);
+  }
   if (tile < 0) return;  // uniform per workgroup: before any barrier
   const int tx = tile % nt, ty = (tile / nt) % nt, tz = tile / (nt * nt);
   const int bx0 = tx * TB, by0 = ty * TB, bz0 = tz * TB;
   const int l = threadIdx.x & 63;
   for (int i = threadIdx.x; i < NN * NN * NN; i += DEP_T) acc[i] = 0ull;
-  // own runs: blocks (bx0..bx0+TB-1, by0+j, bz0+k) are consecutive keys
-  if (threadIdx.x < TB * TB) {
-    const int j = threadIdx.x % TB, k = threadIdx.x / TB;
-    const int32_t b0 = ((bz0 + k) * nb + (by0 + j)) * nb + bx0;
+  if (threadIdx.x < NB) {
+    const int q = threadIdx.x % TB, j = (threadIdx.x / TB) % TB,
+              k = threadIdx.x / (TB * TB);
+    const int32_t b0 = ((bz0 + k) * nb + (by0 + j)) * nb + bx0 + q;
     ostart[threadIdx.x] = cell_start[b0 * BS3];
-    for (int q = 0; q < TB; q++)
-      obnd[threadIdx.x][q] = cell_start[(b0 + q) * BS3];
-    opre[threadIdx.x + 1] = cell_start[(b0 + TB) * BS3];
+    opre[threadIdx.x + 1] = cell_start[(b0 + 1) * BS3];
   }
   // halo ranges and their prefix counts (blocks of DEP_T ranges)
   int32_t carry = 0;
@@ -185,9 +241,7 @@ k_cic_deposit(const int32_t *__restrict__ cell_start,
       cnt = cell_start[k0 + len] - a;
       hstart[s] = a;
       // offset of the neighbour block relative to the tile origin, blocks
-      hoff[s][0] = (int8_t)bi;
-      hoff[s][1] = (int8_t)bj;
-      hoff[s][2] = (int8_t)bk;
+      hoff[s] = (uint16_t)(((bk + 2) << 8) | ((bj + 2) << 4) | (bi + 2));
     }
     const int w = threadIdx.x >> 6;
     const int32_t inc = wave_incl_scan(cnt);
@@ -202,123 +256,176 @@ k_cic_deposit(const int32_t *__restrict__ cell_start,
   if (threadIdx.x == 0) {
     hpre[NS] = carry;
     opre[0] = 0;
-    // prefix of the own runs (their ends were stored in opre[1..]) and the
-    // own-list position of every block
+    // prefix of the own blocks (their ends were stored in opre[1..])
     int32_t p = 0;
-    for (int r = 0; r < TB * TB; r++) {
-      const int32_t n = opre[r + 1] - ostart[r];
-      for (int q = 0; q < TB; q++) obnd[r][q] = p + (obnd[r][q] - ostart[r]);
-      opre[r + 1] = p + n;
-      p += n;
+    for (int r = 0; r < NB; r++) {
+      p += opre[r + 1] - ostart[r];
+      opre[r + 1] = p;
     }
   }
   __syncthreads();
-  const int32_t nown = opre[TB * TB];
+  const int32_t nown = opre[NB];
   const int32_t ntot = nown + hpre[NS];
-  // register sums of the current lower node and their flush to LDS
-  unsigned long long ra[8] = {0ull, 0ull, 0ull, 0ull, 0ull, 0ull, 0ull, 0ull};
-  int32_t rid = -1, rix = 0, riy = 0, riz = 0;
-  // the 4 nodes of x offset h of the current lower node
-  auto flush = [&](int h) {
+  // register sums of the current lower node (2^52 + integer) and their flush
+  // to LDS
+  constexpr double MAGIC = 4503599627370496.0;  // 2^52
+  double ra[8];
+#pragma unroll
+  for (int c = 0; c < 8; c++) ra[c] = MAGIC;
+  int32_t rid = -1, rix = 0, riy = 0, riz = 0, run = 0;
+  auto flush = [&]() {
     if (rid < 0) return;
 #pragma unroll
-    for (int c = h; c < 8; c += 2) {
+    for (int c = 0; c < 8; c++) {
       const int ax = rix + (c & 1), ay = riy + ((c >> 1) & 1), az = riz + (c >> 2);
       if ((unsigned)ax < (unsigned)NN && (unsigned)ay < (unsigned)NN &&
           (unsigned)az < (unsigned)NN)
-        atomicAdd(&acc[(az * NN + ay) * NN + ax], ra[c]);
+        atomicAdd(&acc[(az * NN + ay) * NN + ax],
+                  (unsigned long long)(__double_as_longlong(ra[c]) -
+                                       __double_as_longlong(MAGIC)));
     }
   };
+  // this workgroup's share of the list: all of it, or a piece
+  const int32_t per = ((ntot + np - 1) / np + DEP_T * DEP_K - 1) /
+                      (DEP_T * DEP_K) * (DEP_T * DEP_K);
+  const int32_t lo0 = min(piece * (int64_t)per, (int64_t)ntot),
+                hi0 = min((int64_t)lo0 + per, (int64_t)ntot);
   // lane l of wave w takes list positions base + w*64*K + l*K + j, j < K.
   // All K records of a lane are requested before the first is used, so that
   // a wave keeps K loads per lane in flight.
   const int wv = threadIdx.x >> 6;
-  for (int32_t base = 0; base < ntot; base += DEP_T * DEP_K) {
+  for (int32_t base = lo0; base < hi0; base += DEP_T * DEP_K) {
     float4 rv[DEP_K];
     int32_t ob[DEP_K];  // block offset of the record, packed; 0 = none
+    int32_t send = -1, sdel = 0, soff = 0;  // end of the segment at hand
 #pragma unroll
     for (int j = 0; j < DEP_K; j++) {
       const int32_t t = base + wv * 64 * DEP_K + l * DEP_K + j;
       ob[j] = 0;
-      if (t < ntot) {
-        int32_t k = 0, bxo = 0, byo = 0, bzo = 0;
-        if (t < nown) {
-          int r = 0;
-          while (r + 1 < TB * TB && opre[r + 1] <= t) r++;
-          k = ostart[r] + (t - opre[r]);
-          byo = r % TB;
-          bzo = r / TB;
-          for (int q = 1; q < TB; q++)
-            if (t >= obnd[r][q]) bxo = q;
-        } else {
-          const int32_t th = t - nown;
-          int lo = 0, hi = NS;  // last s with hpre[s] <= th
-          while (hi - lo > 1) {
-            const int mid = (lo + hi) >> 1;
-            if (hpre[mid] <= th) lo = mid; else hi = mid;
+      if (t < hi0) {
+        if (t >= send) {  // the next segment: record = t + sdel
+          if (t < nown) {
+            int lo = 0;  // last own block with opre <= t
+#pragma unroll
+            for (int o = NB / 2; o > 0; o >>= 1)
+              if (opre[lo + o] <= t) lo += o;
+            send = opre[lo + 1];
+            sdel = ostart[lo] - opre[lo];
+            soff = ((lo / (TB * TB) + 2) << 8) | ((lo / TB % TB + 2) << 4) |
+                   (lo % TB + 2);
+          } else {
+            const int32_t th = t - nown;
+            int lo = 0, hi = NS;  // last s with hpre[s] <= th
+            while (hi - lo > 1) {
+              const int mid = (lo + hi) >> 1;
+              if (hpre[mid] <= th) lo = mid; else hi = mid;
+            }
+            send = nown + hpre[lo + 1];
+            sdel = hstart[lo] - hpre[lo] - nown;
+            soff = hoff[lo];
           }
-          k = hstart[lo] + (th - hpre[lo]);
-          bxo = hoff[lo][0];
-          byo = hoff[lo][1];
-          bzo = hoff[lo][2];
         }
-        ob[j] = ((bzo + 2) << 8) | ((byo + 2) << 4) | (bxo + 2);
-        rv[j] = rec[k];
+        ob[j] = soff;
+        rv[j] = rec[t + sdel];
       }
+    }
+    // sums of one node stay below 2^52
+    run += DEP_K;
+    if (run > 32768) {
+      flush();
+      rid = -1;
+#pragma unroll
+      for (int c = 0; c < 8; c++) ra[c] = MAGIC;
+      run = DEP_K;
     }
 #pragma unroll
     for (int j = 0; j < DEP_K; j++) {
       if (ob[j] == 0) break;
-      const int32_t bxo = (ob[j] & 15) - 2, byo = ((ob[j] >> 4) & 15) - 2,
-                    bzo = (ob[j] >> 8) - 2;
       // lower node (tile-relative) and exact offsets
       const float4 r = rv[j];
       const float qx = (float)R * r.x, qy = (float)R * r.y, qz = (float)R * r.z;
       const float fx0 = floorf(qx), fy0 = floorf(qy), fz0 = floorf(qz);
-      const int32_t ix = 8 * R * bxo + (int32_t)fx0;
-      const int32_t iy = 8 * R * byo + (int32_t)fy0;
-      const int32_t iz = 8 * R * bzo + (int32_t)fz0;
+      const int32_t ix = 8 * R * ((ob[j] & 15) - 2) + (int32_t)fx0;
+      const int32_t iy = 8 * R * (((ob[j] >> 4) & 15) - 2) + (int32_t)fy0;
+      const int32_t iz = 8 * R * ((ob[j] >> 8) - 2) + (int32_t)fz0;
       const float fx = qx - fx0, fy = qy - fy0, fz = qz - fz0;
-      const float wx[2] = {1.0f - fx, fx}, wy[2] = {1.0f - fy, fy},
-                  wz[2] = {1.0f - fz, fz};
       const int32_t id = ((iz + 16) * 64 + (iy + 16)) * 64 + (ix + 16);
       if (id != rid) {
-        // the next cell along x: its lower x plane is the current node's
-        // upper one, whose sums stay in registers
-        const bool carry = rid >= 0 && id == rid + 1;
-        flush(0);
-        if (!carry) flush(1);
+        flush();
 #pragma unroll
-        for (int c = 0; c < 8; c += 2) {
-          ra[c] = carry ? ra[c + 1] : 0ull;
-          ra[c + 1] = 0ull;
-        }
+        for (int c = 0; c < 8; c++) ra[c] = MAGIC;
+        run = DEP_K;
         rid = id;
         rix = ix;
         riy = iy;
         riz = iz;
       }
+      // (wx wy) wz with the scale, a power of two, in wz
+      // (a position that is not finite has offsets NaN: weight 0, by the clamp)
+      const float wx[2] = {clamp01(1.0f - fx), clamp01(fx)},
+                  wy[2] = {clamp01(1.0f - fy), clamp01(fy)},
+                  wz[2] = {clamp01(1.0f - fz) * FIX_SCALE,
+                           clamp01(fz) * FIX_SCALE};
 #pragma unroll
       for (int c = 0; c < 8; c++)
-        ra[c] += __float2ull_rn(wx[c & 1] * wy[(c >> 1) & 1] * wz[c >> 2] *
-                                FIX_SCALE);
+        ra[c] += (double)rintf(wx[c & 1] * wy[(c >> 1) & 1] * wz[c >> 2]);
     }
   }
-  flush(0);
-  flush(1);
+  flush();
   __syncthreads();
   const int32_t gx0 = bx0 * 8 * R, gy0 = by0 * 8 * R, gz0 = bz0 * 8 * R;
+  unsigned long long *bacc = B.acc + (int64_t)max(slot, 0) * 4096;
+  if (slot >= 0) {
+    // the pieces' sums meet in memory (integers: any order); the last piece
+    // to finish writes the tile
+    for (int i = threadIdx.x; i < NN * NN * NN; i += DEP_T)
+      if (acc[i]) atomicAdd(&bacc[i], acc[i]);
+    __threadfence();
+    __syncthreads();
+    if (threadIdx.x == 0)
+      lastpiece = atomicAdd(&B.done[slot], 1) == np - 1;
+    __syncthreads();
+    if (!lastpiece) return;
+    __threadfence();
+  }
   for (int i = threadIdx.x; i < NN * NN * NN; i += DEP_T) {
     const int ax = i % NN, ay = (i / NN) % NN, az = i / (NN * NN);
     const int32_t gx = (gx0 + ax + shift) & (ng - 1);
     const int32_t gy = (gy0 + ay + shift) & (ng - 1);
     const int32_t gz = (gz0 + az + shift) & (ng - 1);
+    const unsigned long long v =
+        slot >= 0 ? __hip_atomic_load(&bacc[i], __ATOMIC_RELAXED,
+                                      __HIP_MEMORY_SCOPE_AGENT)
+                  : acc[i];
     grid[((int64_t)gz * ng + gy) * ng + gx] =
-        (float)((double)acc[i] * FIX_INV * norm);
+        (float)((double)v * FIX_INV * norm);
   }
 }
 
-// CIC^-1 of the block's own particles from its (8R+1)^3 nodes.
+// A block of more than INT_CH records is shared by several workgroups: the
+// first INT_CH of them by its own, the rest by one extra each, listed here as
+// (block, piece).  A halo core's block alone held the launch: zoom catalogue
+// at 512^3 2.30 -> 0.87 ms, 1024^3 8.5 -> 6.9, 128^3 70 -> 21 us, with the
+// keys below (pieces of 2^14: 35 us at 128^3).
+constexpr int32_t INT_CH = 1 << 12;
+// below this the list costs more than an uneven launch (one more kernel)
+constexpr int64_t INT_SPLIT_MIN = 1 << 21;
+__global__ void __launch_bounds__(256)
+k_interp_split(const int32_t *__restrict__ cell_start, int32_t nblk,
+               int32_t ucap, int32_t *__restrict__ count,
+               int2 *__restrict__ unit) {
+  const int32_t b = blockIdx.x * 256 + threadIdx.x;
+  if (b >= nblk) return;
+  const int32_t n = cell_start[b * BS3 + BS3] - cell_start[b * BS3];
+  if (n <= INT_CH) return;
+  const int32_t ne = (n - 1) / INT_CH;
+  const int32_t u = atomicAdd(count, ne);
+  for (int32_t i = 0; i < ne && u + i < ucap; i++)
+    unit[u + i] = make_int2(b, i + 1);
+}
+
+// CIC^-1 of the block's own particles from its (8R+1)^3 nodes.  Workgroups
+// before ucap take the extra pieces; ucap = 0: no block is shared.
 template <int R>
 __global__ void __launch_bounds__(256)
 k_cic_interp(const int32_t *__restrict__ cell_start,
@@ -326,11 +433,19 @@ k_cic_interp(const int32_t *__restrict__ cell_start,
              int32_t shift, const float *__restrict__ grid,
              float *__restrict__ rho_sorted, float *__restrict__ rho,
              const int32_t *__restrict__ lab_sorted, int64_t nhalo,
-             unsigned long long *__restrict__ seed_key) {
+             unsigned long long *__restrict__ seed_key, int32_t ucap,
+             const int32_t *__restrict__ ucount,
+             const int2 *__restrict__ unit) {
   constexpr int NN = 8 * R + 1;
   __shared__ float g[NN * NN * NN];
   const int32_t nb = nx >> 3;
-  const int32_t blk = blockIdx.x;
+  int32_t blk = (int32_t)blockIdx.x - ucap, piece = 0;
+  if (blk < 0) {
+    if ((int32_t)blockIdx.x >= ucount[0]) return;
+    const int2 u = unit[blockIdx.x];
+    blk = u.x;
+    piece = u.y;
+  }
   const int bx = blk % nb, by = (blk / nb) % nb, bz = blk / (nb * nb);
   const int32_t gx0 = bx * 8 * R, gy0 = by * 8 * R, gz0 = bz * 8 * R;
   const bool seeds = seed_key && lab_sorted;
@@ -338,7 +453,9 @@ k_cic_interp(const int32_t *__restrict__ cell_start,
   // are requested before the nodes are staged, and each round requests the
   // next round's before its own are used, so that the loads of a block are
   // in flight together rather than one after the other.
-  const int32_t s0 = cell_start[blk * BS3], s1 = cell_start[blk * BS3 + BS3];
+  const int32_t s0 = cell_start[blk * BS3] + piece * INT_CH,
+                sb = cell_start[blk * BS3 + BS3],
+                s1 = ucap > 0 ? min(sb, s0 + INT_CH) : sb;
   float4 r = make_float4(0.f, 0.f, 0.f, 0.f);
   int32_t h = -1;
   if (s0 + (int32_t)threadIdx.x < s1) {
@@ -353,8 +470,20 @@ k_cic_interp(const int32_t *__restrict__ cell_start,
     g[i] = grid[((int64_t)gz * ng + gy) * ng + gx];
   }
   __syncthreads();
+  // the label at hand (uniform over the wave; -1: none), each lane's best key
+  // of it, and the wave's maximum of them, given to the label
+  int32_t held = -1;
+  unsigned long long hkey = 0ull;
+  auto give = [&]() {
+    if (held < 0) return;
+    const uint32_t kh = (uint32_t)(hkey >> 32);
+    const uint32_t mh = wave_max_u32(kh);
+    const uint32_t ml = wave_max_u32(kh == mh ? (uint32_t)hkey : 0u);
+    if ((threadIdx.x & 63) == 0)
+      atomicMax(&seed_key[held], ((unsigned long long)mh << 32) | ml);
+  };
   // uniform trip count so that every lane of a wave takes part in the
-  // per-label reduction of the seed keys
+  // reduction of the seed keys
   for (int32_t base = s0; base < s1; base += 256) {
     const int32_t k = base + threadIdx.x;
     const bool ok = k < s1;
@@ -393,25 +522,24 @@ k_cic_interp(const int32_t *__restrict__ cell_start,
           mem ? (((unsigned long long)__float_as_uint(rf) << 32) |
                  (unsigned long long)(0xFFFFFFFFu - (uint32_t)idx))
               : 0ull;
-      // one atomic per distinct label of the wave (members of a halo are
-      // contiguous in cell order)
-      uint64_t todo = __ballot(mem);
+      // Members of a halo are neighbours in cell order: each lane keeps its
+      // best key of the label at hand, and the wave reduces them only when
+      // other labels appear (a 64-bit shuffle maximum per round and label:
+      // zoom catalogue at 512^3 1.6 ms against 0.9).
+      if (mem && h == held) hkey = key > hkey ? key : hkey;
+      uint64_t todo = __ballot(mem && h != held);
       while (todo) {
-        const int leader = __ffsll((unsigned long long)todo) - 1;
-        const int32_t hl = __shfl(h, leader, 64);
-        const bool mine = mem && h == hl;
-        unsigned long long v = mine ? key : 0ull;
-        for (int o = 32; o > 0; o >>= 1) {
-          const unsigned long long w = __shfl_xor(v, o, 64);
-          v = w > v ? w : v;
-        }
-        if ((int)(threadIdx.x & 63) == leader) atomicMax(&seed_key[hl], v);
+        give();
+        held = __builtin_amdgcn_readlane(h, __ffsll((unsigned long long)todo) - 1);
+        const bool mine = mem && h == held;
+        hkey = mine ? key : 0ull;
         todo &= ~__ballot(mine);
       }
     }
     r = rn;
     h = hn;
   }
+  give();
 }
 
 static int check_grid_args(int32_t nx, int32_t ng, int32_t shift) {
@@ -442,33 +570,34 @@ static int32_t deposit_tiles(int32_t nx, int32_t ng, int32_t *TB,
 static int deposit_queue(psod_ctx *ctx, int64_t npart, int32_t nx,
                          const int32_t *d_cell_start, const float *d_rec,
                          int32_t ng, int32_t shift, float *d_grid,
-                         int32_t *listed) {
+                         int32_t *listed, const BigTiles &B) {
   int32_t TB, ntile, capd;
   (void)deposit_tiles(nx, ng, &TB, &ntile, &capd);
   const int32_t nb = nx / 8;
   const double norm = (double)ng * (double)ng * (double)ng / (double)npart;
   int32_t *dcount = listed + ntile, *dlist = dcount + 32;
   hipStream_t st = ctx->stream;
-  const unsigned nblk = (unsigned)(ntile + capd);
+  const unsigned nblk = (unsigned)(B.ucap + ntile + capd);
   if (capd > 0) {
-    PSOD_TRY(psod_fill_i32(ctx, dcount, 1, 0));
-    k_tile_dense<<<grid_for(ntile, 256), 256, 0, st>>>(
+    PSOD_TRY(psod_fill_i32(ctx, dcount, 3, 0));
+    k_tile_dense<<<std::max(grid_for(ntile, 256), 4u * (unsigned)B.cap), 256, 0,
+                   st>>>(
         d_cell_start, nb, TB, ntile, capd,
-        psod_tunables_for(ctx, nx).dense_tile, listed, dcount, dlist);
+        psod_tunables_for(ctx, nx).dense_tile, listed, dcount, dlist, B);
     PSOD_LAUNCH_CHECK();
   }
   if (ng == nx && TB == 2)
     k_cic_deposit<1, 2><<<nblk, DEP_T, 0, st>>>(
         d_cell_start, (const float4 *)d_rec, nx, ng, shift, norm, capd, dcount,
-        dlist, listed, d_grid);
+        dlist, listed, B, d_grid);
   else if (ng == nx)
     k_cic_deposit<1, 1><<<nblk, DEP_T, 0, st>>>(
         d_cell_start, (const float4 *)d_rec, nx, ng, shift, norm, capd, dcount,
-        dlist, listed, d_grid);
+        dlist, listed, B, d_grid);
   else
     k_cic_deposit<2, 1><<<nblk, DEP_T, 0, st>>>(
         d_cell_start, (const float4 *)d_rec, nx, ng, shift, norm, capd, dcount,
-        dlist, listed, d_grid);
+        dlist, listed, B, d_grid);
   PSOD_LAUNCH_CHECK();
   return PSOD_OK;
 }
@@ -482,11 +611,26 @@ extern "C" int psod_cic_deposit(psod_ctx *ctx, int64_t npart, int32_t nx,
   if (npart <= 0 || !d_cell_start || !d_rec || !d_grid)
     return psod_set_error(PSOD_E_ARG, "psod_cic_deposit: bad arguments");
   int32_t TB, ntile, capd;
-  const int32_t nlist = deposit_tiles(nx, ng, &TB, &ntile, &capd);
-  int32_t *listed = (int32_t *)psod_scratch(ctx, S_TILE, (size_t)nlist * 4);
-  if (!listed) return PSOD_E_NOMEM;
+  const size_t nlist = (size_t)deposit_tiles(nx, ng, &TB, &ntile, &capd);
+  // the tile list, then the tiles in pieces: 3 ints per slot, their units
+  // and their node sums
+  BigTiles B = {};
+  B.cap = (int32_t)std::min<int64_t>(std::min<int64_t>(ntile, DEP_BIGCAP),
+                                     npart / DEP_BIG);
+  B.ucap = B.cap > 0 ? (int32_t)(npart / DEP_PIECE) + B.cap : 0;
+  const size_t o1 = (nlist * 4 + 255) & ~(size_t)255,
+               o2 = o1 + (((size_t)B.cap * 12 + 255) & ~(size_t)255),
+               o3 = o2 + (((size_t)B.ucap * 8 + 255) & ~(size_t)255);
+  char *buf = (char *)psod_scratch(ctx, S_TILE, o3 + (size_t)B.cap * 4096 * 8);
+  if (!buf) return PSOD_E_NOMEM;
+  B.count = (int32_t *)buf + ntile + 1;  // beside the dense-tile count
+  B.tile = (int32_t *)(buf + o1);
+  B.np = B.tile + B.cap;
+  B.done = B.np + B.cap;
+  B.unit = (int2 *)(buf + o2);
+  B.acc = (unsigned long long *)(buf + o3);
   PSOD_TRY(deposit_queue(ctx, npart, nx, d_cell_start, d_rec, ng, shift,
-                         d_grid, listed));
+                         d_grid, (int32_t *)buf, B));
   return psod_finish(ctx);
 }
 
@@ -546,8 +690,9 @@ extern "C" int psod_cic_deposit_noalloc(psod_ctx *ctx, int64_t npart,
     return psod_set_error(PSOD_E_DEVICE, "psod_cic_deposit_noalloc: the "
                           "fixed tile list of device %d is not set up",
                           ctx->device);
+  // no tiles in pieces: their sums would need memory
   return deposit_queue(ctx, npart, nx, d_cell_start, d_rec, ng, shift, d_grid,
-                       listed);
+                       listed, BigTiles{});
 }
 
 extern "C" int psod_cic_interp(psod_ctx *ctx, int64_t npart, int32_t nx,
@@ -566,16 +711,29 @@ extern "C" int psod_cic_interp(psod_ctx *ctx, int64_t npart, int32_t nx,
   // that no fill queued elsewhere can race the atomics below
   if (d_seed_key && d_lab_sorted && nhalo > 0)
     PSOD_TRY(psod_fill_u64(ctx, d_seed_key, nhalo, 0));
+  int32_t ucap = 0, *ucount = nullptr;
+  int2 *unit = nullptr;
+  if (npart >= INT_SPLIT_MIN) {
+    const int32_t cap = (int32_t)(npart / INT_CH);
+    ucount = (int32_t *)psod_scratch(ctx, S_TILE, 256 + (size_t)cap * 8);
+    if (!ucount) return PSOD_E_NOMEM;
+    ucap = cap;
+    unit = (int2 *)(ucount + 64);
+    PSOD_TRY(psod_fill_i32(ctx, ucount, 1, 0));
+    k_interp_split<<<grid_for(nblk, 256), 256, 0, ctx->stream>>>(
+        d_cell_start, (int32_t)nblk, ucap, ucount, unit);
+    PSOD_LAUNCH_CHECK();
+  }
   if (ng == nx)
-    k_cic_interp<1><<<nblk, 256, 0, ctx->stream>>>(
+    k_cic_interp<1><<<nblk + (unsigned)ucap, 256, 0, ctx->stream>>>(
         d_cell_start, (const float4 *)d_rec, nx, ng, shift, d_grid,
         d_rho_sorted, d_rho, d_lab_sorted, nhalo,
-        (unsigned long long *)d_seed_key);
+        (unsigned long long *)d_seed_key, ucap, ucount, unit);
   else
-    k_cic_interp<2><<<nblk, 256, 0, ctx->stream>>>(
+    k_cic_interp<2><<<nblk + (unsigned)ucap, 256, 0, ctx->stream>>>(
         d_cell_start, (const float4 *)d_rec, nx, ng, shift, d_grid,
         d_rho_sorted, d_rho, d_lab_sorted, nhalo,
-        (unsigned long long *)d_seed_key);
+        (unsigned long long *)d_seed_key, ucap, ucount, unit);
   PSOD_LAUNCH_CHECK();
   return psod_finish(ctx);
 }

@@ -227,4 +227,16 @@ __device__ inline int32_t wave_incl_scan(int32_t v) {
   return v;
 }
 
+// Largest value over the lanes (every lane active), in every lane.
+__device__ inline uint32_t wave_max_u32(uint32_t v) {
+  auto step = [&](int32_t w) { v = max(v, (uint32_t)w); };
+  step(__builtin_amdgcn_update_dpp(0, (int32_t)v, 0x111, 0xf, 0xf, false));
+  step(__builtin_amdgcn_update_dpp(0, (int32_t)v, 0x112, 0xf, 0xf, false));
+  step(__builtin_amdgcn_update_dpp(0, (int32_t)v, 0x114, 0xf, 0xf, false));
+  step(__builtin_amdgcn_update_dpp(0, (int32_t)v, 0x118, 0xf, 0xf, false));
+  step(__builtin_amdgcn_update_dpp(0, (int32_t)v, 0x142, 0xa, 0xf, false));
+  step(__builtin_amdgcn_update_dpp(0, (int32_t)v, 0x143, 0xc, 0xf, false));
+  return (uint32_t)__builtin_amdgcn_readlane((int32_t)v, 63);
+}
+
 __device__ inline uint64_t ballot64(bool p) { return __ballot(p); }
