@@ -944,8 +944,16 @@ k_centre_windows(SodCfg c, const int32_t *__restrict__ cell_start,
 // 16b..16b+15, Morton-compact).  Boxes of 8 bound tighter but cost twice as
 // many terms; with the items taken most promising first, 16 is faster
 // (c3: 8 -> 236 ms, 16 -> 218, 32 -> 235, 64 -> 263 ms of SOD).  Stores the
-// bound of box b in ubx[t*4 + b], the task's bound in ubt[t] and each halo's
-// largest task bound in hpil.
+// bound of box b in ubx[t*4 + b], the task's bound in ubt[t], its estimate in
+// est[t] and each halo's largest estimate in hpil.
+//
+// The estimate is S at the middle of the task's box with the candidates
+// within half the box's diagonal, the records of its cell at 0.3 cells and
+// those of the other cells at the cells' centres.  The task with a halo's
+// largest estimate is its pilot: on sampled halos (n5 5e3..4e5) its best S is
+// 0.97 of the largest, where the task with the largest bound (loose boxes
+// far from the core among them) reached 0.72 and let twice as many boxes
+// through to the items.  An estimate decides only what is summed first.
 // 6 waves per SIMD (80 VGPRs): 73.7 -> 56.7 ms at 1024^3
 __global__ void __launch_bounds__(256, 6)
 k_centre_bound(SodCfg c, const int32_t *__restrict__ cell_start,
@@ -953,6 +961,7 @@ k_centre_bound(SodCfg c, const int32_t *__restrict__ cell_start,
                const int32_t *__restrict__ large, const int4 *__restrict__ tasks,
                const int32_t *__restrict__ ntask_total,
                unsigned long long *__restrict__ hpil,
+               uint32_t *__restrict__ est,
                unsigned long long *__restrict__ ubt,
                unsigned long long *__restrict__ ubx,
                const float4 *__restrict__ gwin, int32_t *__restrict__ wq) {
@@ -983,10 +992,10 @@ k_centre_bound(SodCfg c, const int32_t *__restrict__ cell_start,
       const HaloPlan pl = plan[large[tk.x]];
       if (pl.n5 < c.bound_min) {
         // few particles around the seed: every task of the halo is evaluated
-        // exactly by the pilots (an all-ones bound makes each one a pilot)
+        // exactly by the pilots (an all-ones estimate makes each one a pilot)
         if (l == 0) {
-          ubt[t] = ~0ull;
-          atomicMax(&hpil[tk.x], ~0ull);
+          est[t] = ~0u;
+          atomicMax(&hpil[tk.x], (unsigned long long)~0u);
         }
         continue;
       }
@@ -1041,6 +1050,7 @@ k_centre_bound(SodCfg c, const int32_t *__restrict__ cell_start,
       // record ranges of the 27 cells, one per lane, all loaded at once; a
       // cell beyond reach of the candidates' box gets an empty range
       int32_t qa = 0, qb = 0;
+      float e = 0.f;  // the estimate's share of this lane
       if (l < 27) {
         int ei, ej, ek;
         walk_off(l, 1, &ei, &ej, &ek);
@@ -1053,6 +1063,27 @@ k_centre_bound(SodCfg c, const int32_t *__restrict__ cell_start,
           qa = cell_start[key];
           qb = cell_start[key + 1];
         }
+        float d2 = 0.1f;  // own cell
+        if (l != 13) {
+          const float dx = nb0[0] + 0.5f - 0.5f * (cb0[0] + cb1[0]),
+                      dy = nb0[1] + 0.5f - 0.5f * (cb0[1] + cb1[1]),
+                      dz = nb0[2] + 0.5f - 0.5f * (cb0[2] + cb1[2]);
+          d2 = dx * dx + dy * dy + dz * dz + 0.15f;
+        }
+        e = (float)(qb - qa) * __builtin_amdgcn_rsqf(d2 + c.eps2f);
+      } else if (l == 27) {
+        const float dx = cb1[0] - cb0[0], dy = cb1[1] - cb0[1],
+                    dz = cb1[2] - cb0[2];
+        e = (float)tk.w *
+            __builtin_amdgcn_rsqf(0.25f * (dx * dx + dy * dy + dz * dz) +
+                                  c.eps2f);
+      }
+      const float esum = wave_sumf(e);
+      if (l == 0) {
+        // a positive float orders like its bits, below the all-ones above
+        const uint32_t u = __float_as_uint(fmaxf(esum, 0.f));
+        est[t] = u;
+        atomicMax(&hpil[tk.x], (unsigned long long)u);
       }
       uint64_t rest = __ballot(l < 27 && qa < qb);  // cells with records
       uint64_t tot = 0;  // bound of box l >> 4, flushed part
@@ -1218,10 +1249,7 @@ k_centre_bound(SodCfg c, const int32_t *__restrict__ cell_start,
         const unsigned long long v = __shfl_xor(ubmax, o, 64);
         ubmax = v > ubmax ? v : ubmax;
       }
-      if (l == 0) {
-        ubt[t] = ubmax;
-        atomicMax(&hpil[tk.x], ubmax);
-      }
+      if (l == 0) ubt[t] = ubmax;
     }
   }
 }
@@ -1371,9 +1399,8 @@ constexpr int32_t PILOT_PIECES = 64, PILOT_CHUNKS = 16;
 
 // Pilots, one wave per task: the 64 candidates of a task (one per lane)
 // against the 27 cells around their cell (every neighbour within 1 cell lies
-// there).  Evaluates exactly the tasks holding their halo's largest bound
-// (every task of a halo that skipped the bound) and folds their S into
-// hbest.  Dense cells are in Morton order of their 1/8-cell sub-cells, so
+// there).  Evaluates exactly the tasks holding their halo's largest estimate
+// (every task of a halo that skips the bound) and folds their S into hbest.  Dense cells are in Morton order of their 1/8-cell sub-cells, so
 // candidate groups and neighbour chunks are compact.  A task with more than
 // pilot_big records in reach is appended to big[] (count in nbig[0], at most
 // bigcap; more go whole), its pieces (slot << 6 | piece) to units[] (count
@@ -1387,7 +1414,7 @@ k_centre_pilot(SodCfg c, const int32_t *__restrict__ cell_start,
                uint64_t *__restrict__ taskres,
                unsigned long long *__restrict__ hbest,
                const unsigned long long *__restrict__ hpil,
-               const unsigned long long *__restrict__ ubt,
+               const uint32_t *__restrict__ est,
                unsigned long long *__restrict__ cstat,
                int32_t pilot_big, int32_t bigcap, int32_t *__restrict__ big,
                int32_t *__restrict__ units, int32_t *__restrict__ nbig,
@@ -1406,7 +1433,7 @@ k_centre_pilot(SodCfg c, const int32_t *__restrict__ cell_start,
     const int32_t t1 = min(nt, t0 + 16);
     for (int32_t t = t0; t < t1; t++) {
       const int4 tk = tasks[t];
-      if (ubt[t] != hpil[tk.x]) continue;
+      if (est[t] != hpil[tk.x]) continue;
       const HaloPlan pl = plan[large[tk.x]];
       PilotSetup P;
       pilot_setup(c, cell_start, rec, pl, tk, l, cut, P);
@@ -1546,8 +1573,9 @@ k_centre_pilot_fin(const float4 *__restrict__ rec,
 __global__ void __launch_bounds__(256)
 k_task_items(const int4 *__restrict__ tasks,
              const int32_t *__restrict__ ntask_total,
-             const unsigned long long *__restrict__ ubt,
+             const uint32_t *__restrict__ est,
              const unsigned long long *__restrict__ hpil,
+             const unsigned long long *__restrict__ ubt,
              const unsigned long long *__restrict__ ubx,
              const unsigned long long *__restrict__ hbest,
              int32_t *__restrict__ items, int32_t *__restrict__ nitems,
@@ -1558,9 +1586,8 @@ k_task_items(const int4 *__restrict__ tasks,
   bool skipped = false;
   if (t < nt) {
     const int4 tk = tasks[t];
-    const unsigned long long ub = ubt[t];
-    if (ub != hpil[tk.x]) {
-      const unsigned long long best = hbest[tk.x];
+    if (est[t] != hpil[tk.x]) {
+      const unsigned long long ub = ubt[t], best = hbest[tk.x];
       const int nbx = (tk.w + 15) >> 4;
       if (ub >= best)
         for (int b = 0; b < nbx; b++)
@@ -1644,26 +1671,24 @@ k_class_scatter(const uint8_t *__restrict__ cls,
     if (t0 + j * 256 + (int32_t)threadIdx.x < n) out[base[k[j]] + r[j]] = v[j];
 }
 
-// Classes of the items: the ratio of the item's bound to its halo's best
-// after the pilots, largest first (the groups most likely to raise the best
-// run first; those after them meet a higher best).  64 classes per unit of
-// the ratio, up to 5.
+// Classes of the items by their bounds, which grow with the neighbours in
+// reach: the longest items first, and those of one halo together.  By the
+// bound over the halo's best (most promising first) the longest items were
+// spread over the list and ended last (zoom catalogue at 512^3 9.3 ms against
+// 4.2, 512^3 3.0 against 2.7, 256^3 0.75 against 0.54, with the items taken
+// singly at first; 1024^3 36.4 against 36.5): after a good pilot the order
+// hardly changes what is abandoned.
 __global__ void __launch_bounds__(256)
 k_item_keys(const int32_t *__restrict__ items,
-            const int32_t *__restrict__ nitems, const int4 *__restrict__ tasks,
+            const int32_t *__restrict__ nitems,
             const unsigned long long *__restrict__ ubx,
-            const unsigned long long *__restrict__ hbest,
             uint8_t *__restrict__ cls, int32_t *__restrict__ hist) {
   const int32_t i = blockIdx.x * blockDim.x + threadIdx.x;
   const int32_t n = *nitems;
   if ((int32_t)(blockIdx.x * blockDim.x) >= n) return;  // uniform
   uint32_t k = 0;
   if (i < n) {
-    const int32_t it = items[i];
-    const double ub = (double)ubx[it];
-    const double b = (double)hbest[tasks[it >> 2].x];
-    const double r = b > 0.0 ? ub / b : 5.0;
-    k = 255u - (uint32_t)fmax(0.0, fmin((r - 1.0) * 64.0, 255.0));
+    k = cost_class((double)ubx[items[i]] * (1.0 / SFIX));
     cls[i] = (uint8_t)k;
   }
   count_class(i < n, k, hist);
@@ -1723,11 +1748,17 @@ k_centre_group(SodCfg c, const int32_t *__restrict__ cell_start,
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
   };
-  // blocks of 2 items in list order (most promising first)
+  // Items in list order (longest first), one at a time for the first 16 per
+  // wave of the launch: pairs of long items hold its end (zoom catalogue at
+  // 512^3, in pairs only 8.1 ms, the first 4 per wave singly 5.3, 16 4.2).
+  // Then in pairs, which spare the shared counter (1024^3, all singly: 37.6
+  // ms against 36.5).
+  const int32_t lone = (int32_t)gridDim.x * 64;
   for (;;) {
-    const int32_t i0 = wave_next(wq) * 2;
+    const int32_t u = wave_next(wq);
+    const int32_t i0 = u < lone ? u : lone + (u - lone) * 2;
     if (i0 >= ni) break;
-    const int32_t i1 = min(ni, i0 + 2);
+    const int32_t i1 = min(ni, i0 + (u < lone ? 1 : 2));
     for (int32_t i = i0; i < i1; i++) {
       const int32_t it = items[i];
       const int4 tk = tasks[it >> 2];
@@ -4414,7 +4445,7 @@ static int centre_search(psod_ctx *ctx, const SodCfg &c,
   // tasks and their per-candidate totals
   int4 *tasks = (int4 *)psod_scratch(
       ctx, S_TASKRES,
-      (size_t)tcap * (sizeof(int4) + 24 + 4 * 8 + 4 * 16 + 4 * 4) + 512 +
+      (size_t)tcap * (sizeof(int4) + 24 + 4 * 8 + 4 * 16 + 4 * 4 + 4) + 512 +
           (size_t)bigcap * (4 + PILOT_PIECES * 4 + 64 * 8));
   if (!tasks) return PSOD_E_NOMEM;
   uint64_t *tres = (uint64_t *)(tasks + tcap);
@@ -4422,7 +4453,8 @@ static int centre_search(psod_ctx *ctx, const SodCfg &c,
   unsigned long long *ubx = ubt + tcap;
   uint64_t *ires = (uint64_t *)(ubx + 4 * (int64_t)tcap);
   int32_t *items = (int32_t *)(ires + 8 * (int64_t)tcap);
-  int32_t *nitems = items + 4 * (int64_t)tcap;
+  uint32_t *est = (uint32_t *)(items + 4 * (int64_t)tcap);
+  int32_t *nitems = (int32_t *)(est + (((int64_t)tcap + 1) & ~1));
   // work counters of the bound, pilot, group and split-pilot launches, and
   // the count of split pilot tasks
   int32_t *wq = nitems + 4;
@@ -4441,7 +4473,7 @@ static int centre_search(psod_ctx *ctx, const SodCfg &c,
       ires, 4 * (int64_t)tcap);
   PSOD_LAUNCH_CHECK();
   // hbest[nlarge..nlarge+3]: units evaluated, units skipped, pair tests,
-  // units abandoned; then each halo's largest task bound
+  // units abandoned; then each halo's largest estimate
   unsigned long long *cstat = hbest + nlarge;
   unsigned long long *hpil = cstat + 4;
   PSOD_TRY(psod_fill_u64(ctx, (uint64_t *)hbest, 2 * (int64_t)nlarge + 4, 0));
@@ -4467,11 +4499,12 @@ static int centre_search(psod_ctx *ctx, const SodCfg &c,
   const unsigned nwg = resident((const void *)k_centre_bound);
   k_centre_bound<<<nwg, 256, 0, st>>>(c, cat->cell_start,
                                       (const float4 *)cat->rec, plan, large,
-                                      tasks, ntot, hpil, ubt, ubx, gwin, wq);
+                                      tasks, ntot, hpil, est, ubt, ubx, gwin,
+                                      wq);
   PSOD_LAUNCH_CHECK();
   k_centre_pilot<<<resident((const void *)k_centre_pilot), 256, 0, st>>>(
       c, cat->cell_start, (const float4 *)cat->rec, plan, large, tasks, ntot,
-      tres, hbest, hpil, ubt, cstat, pilot_big(), bigcap, big, units, nbig, pacc,
+      tres, hbest, hpil, est, cstat, pilot_big(), bigcap, big, units, nbig, pacc,
       wq + 1);
   PSOD_LAUNCH_CHECK();
   k_centre_pilot_big<<<resident((const void *)k_centre_pilot_big), 256, 0,
@@ -4484,9 +4517,9 @@ static int centre_search(psod_ctx *ctx, const SodCfg &c,
       cstat);
   PSOD_LAUNCH_CHECK();
   k_task_items<<<grid_for(tcap, 256), 256, 0, st>>>(
-      tasks, ntot, ubt, hpil, ubx, hbest, items, nitems, cstat);
+      tasks, ntot, est, hpil, ubt, ubx, hbest, items, nitems, cstat);
   PSOD_LAUNCH_CHECK();
-  // items sorted by their bound over the halo's best, largest first
+  // items ordered by their bounds, largest first
   int32_t ni = 4 * tcap;  // capacity (device count) or the exact count
   if (!dn) {
     PSOD_HIP(hipMemcpyAsync(&ni, nitems, 4, hipMemcpyDeviceToHost, st));
@@ -4499,8 +4532,8 @@ static int centre_search(psod_ctx *ctx, const SodCfg &c,
     if (!hist || !ord) return PSOD_E_NOMEM;
     uint8_t *cls = (uint8_t *)(hist + 512);
     PSOD_TRY(psod_fill_i32(ctx, hist, 512, 0));
-    k_item_keys<<<grid_for(ni, 256), 256, 0, st>>>(items, nitems, tasks, ubx,
-                                                   hbest, cls, hist);
+    k_item_keys<<<grid_for(ni, 256), 256, 0, st>>>(items, nitems, ubx, cls,
+                                                   hist);
     PSOD_LAUNCH_CHECK();
     k_class_scatter<<<grid_for(ni, 256 * ORD_V), 256, 0, st>>>(
         cls, items, ni, nitems, hist, ord);
