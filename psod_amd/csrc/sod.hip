@@ -2010,6 +2010,7 @@ k_centre_reduce(HaloPlan *__restrict__ plan, const int32_t *__restrict__ large,
 // ---------------------------------------------------------------------------
 constexpr int GL_T = 512;
 constexpr int SORT_CAP = 4096;
+constexpr int SORT_LDS = 8192;  // keys that the workgroup sorts in LDS
 // segments of possible crossing bins per threshold; ranges of collected
 // bins (the last slot holds the second threshold's band)
 constexpr int SEGCAP = 4;
@@ -2027,7 +2028,7 @@ constexpr int64_t HIST_SLICE = HIST_MAX + 64;
 struct GrowShared {
   uint64_t skey[SORT_CAP];
   int32_t pre[GL_T + 1];
-  int32_t st[GL_T];
+  int32_t st[GL_T];  // first record less its number in the round
   int32_t sdi[GL_T];  // per segment: di of the cell at x = 0 of its block
   int32_t spk[GL_T];  // per segment: dj, dk (12 bits each, +2048), y & 7, z & 7
   int32_t red_i[GL_T / 64];
@@ -2264,26 +2265,42 @@ __device__ inline void cube_walk(const SodCfg &c, GrowShared &G,
       all += G.red_i[i];
     }
     G.pre[threadIdx.x] = off + ex;
-    G.st[threadIdx.x] = st;
+    G.st[threadIdx.x] = st - (off + ex);
     G.sdi[threadIdx.x] = sdi;
     G.spk[threadIdx.x] = spk;
-    if (threadIdx.x == 0) G.pre[GL_T] = all;
     __syncthreads();
-    const int nq = (int)min((int64_t)GL_T, qe - base);
-    // CW_U particles per thread per step: their searches and loads are
-    // independent, so their latencies overlap
+    // CW_U particles per thread per step, the next step's requested before
+    // this step's are used.  Their segments are searched side by side in
+    // fixed steps (segments past the last start at `all`): one search after
+    // the other took longer than the rest of the step (k_grow_large 1024^3
+    // 13.6 -> 11.6 ms, 256^3 1.09 -> 0.78; of that the request ahead 0.4).
+    int qn[CW_U];
+    float4 rn[CW_U];
+    auto fetch = [&](int32_t j0) {
+      int32_t j[CW_U];
+#pragma unroll
+      for (int u = 0; u < CW_U; u++) {
+        j[u] = min(j0 + u * GL_T, all - 1);
+        qn[u] = 0;
+      }
+#pragma unroll
+      for (int o = GL_T / 2; o > 0; o >>= 1)
+#pragma unroll
+        for (int u = 0; u < CW_U; u++)
+          if (G.pre[qn[u] + o] <= j[u]) qn[u] += o;
+#pragma unroll
+      for (int u = 0; u < CW_U; u++) rn[u] = rec[G.st[qn[u]] + j[u]];
+    };
+    if (all > 0) fetch(threadIdx.x);
     for (int32_t j0 = threadIdx.x; j0 < all; j0 += CW_U * GL_T) {
       int qq[CW_U];
       float4 rv[CW_U];
 #pragma unroll
       for (int u = 0; u < CW_U; u++) {
-        const int32_t j = j0 + u * GL_T;
-        qq[u] = 0;
-        if (j < all) {
-          qq[u] = bsearch_last_le(G.pre, nq, j);
-          rv[u] = rec[G.st[qq[u]] + (j - G.pre[qq[u]])];
-        }
+        qq[u] = qn[u];
+        rv[u] = rn[u];
       }
+      fetch(j0 + CW_U * GL_T);
 #pragma unroll
       for (int u = 0; u < CW_U; u++) {
         if (j0 + u * GL_T >= all) continue;
@@ -2331,29 +2348,247 @@ __device__ inline double rad3_for(int64_t k, double mpart, double delta) {
 }
 
 
+// Sort of n <= SORT_LDS distinct keys src (LDS or global memory) to dst by
+// the workgroup, in LDS: kb (n keys; may be src and dst) and bins
+// (SORT_LDS entries).  The keys' distance bits, which order like the
+// distances, are counted in up to SORT_LDS bins over their range (at most
+// the top 20 octaves of d2: the rest share the first bin), the keys placed by
+// their bins, and each ranked by the smaller keys of its bin.  About 20 LDS
+// accesses per key; the bitonic network takes 4 per key and step, 91 steps
+// for 8192 keys (bands of 4437 keys 195 -> 27 us; all halos whose cubes are
+// sorted whole at 1024^3 half the workgroup time, k_grow_large 11.6 -> 9.3
+// ms, 256^3 0.78 -> 0.61).
+// Returns false with the keys in kb in any order when a bin holds more than
+// SORT_BIN keys (coincident particles, lattices).
+constexpr int32_t SORT_BIN = 128;
+constexpr int SORT_PER = SORT_LDS / GL_T;
+
+__device__ inline bool block_bin_sort(const uint64_t *src, uint64_t *dst,
+                                      int32_t n, uint64_t *kb, int32_t *bins,
+                                      GrowShared &G) {
+  const int l = threadIdx.x & 63, w = threadIdx.x >> 6;
+  uint64_t k[SORT_PER];
+  uint32_t lo = 0xFFFFFFFFu, hi = 0u;
+#pragma unroll
+  for (int i = 0; i < SORT_PER; i++) {
+    const int32_t j = threadIdx.x + i * GL_T;
+    if (j < n) {
+      k[i] = src[j];
+      lo = min(lo, (uint32_t)(k[i] >> 32));
+      hi = max(hi, (uint32_t)(k[i] >> 32));
+    }
+  }
+  lo = ~wave_max_u32(~lo);
+  hi = wave_max_u32(hi);
+  const int32_t nbin = max(1024, min(SORT_LDS, next_pow2(n)));
+  for (int32_t b = threadIdx.x; b < nbin; b += GL_T) bins[b] = 0;
+  if (l == 0) {
+    G.pre[w] = (int32_t)lo;
+    G.pre[w + GL_T / 64] = (int32_t)hi;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < GL_T / 64; i++) {
+    lo = min(lo, (uint32_t)G.pre[i]);
+    hi = max(hi, (uint32_t)G.pre[i + GL_T / 64]);
+  }
+  if (hi - lo > (20u << 23)) lo = hi - (20u << 23);
+  int sh = 0;
+  while (((hi - lo) >> sh) >= (uint32_t)nbin) sh++;
+  auto bin = [&](uint64_t x) {
+    const uint32_t u = (uint32_t)(x >> 32);
+    return u > lo ? (int32_t)((u - lo) >> sh) : 0;
+  };
+  int32_t r[SORT_PER];
+#pragma unroll
+  for (int i = 0; i < SORT_PER; i++)
+    if ((int32_t)threadIdx.x + i * GL_T < n) r[i] = atomicAdd(&bins[bin(k[i])], 1);
+  __syncthreads();
+  // exclusive prefix per wave (its nbin / 8 bins), the waves' sums in red_i
+  const int32_t per = nbin / (GL_T / 64);
+  int32_t run = 0, big = 0;
+  for (int32_t b = w * per + l; b < (w + 1) * per; b += 64) {
+    const int32_t v = bins[b], inc = wave_incl_scan(v);
+    bins[b] = run + inc - v;
+    big = max(big, v);
+    run += __builtin_amdgcn_readlane(inc, 63);
+  }
+  big = (int32_t)wave_max_u32((uint32_t)big);
+  if (l == 0) {
+    G.red_i[w] = run;
+    G.pre[w] = big;
+  }
+  __syncthreads();
+  int32_t before[GL_T / 64], sum = 0;
+#pragma unroll
+  for (int i = 0; i < GL_T / 64; i++) {
+    before[i] = sum;
+    sum += G.red_i[i];
+    big = max(big, G.pre[i]);
+  }
+  for (int32_t b = w * per + l; b < (w + 1) * per; b += 64) {
+    int32_t add = 0;
+#pragma unroll
+    for (int i = 0; i < GL_T / 64; i++) add = i == w ? before[i] : add;
+    bins[b] += add;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < SORT_PER; i++)
+    if ((int32_t)threadIdx.x + i * GL_T < n) kb[bins[bin(k[i])] + r[i]] = k[i];
+  __syncthreads();
+  if (big > SORT_BIN) return false;  // uniform
+#pragma unroll
+  for (int i = 0; i < SORT_PER; i++)
+    if ((int32_t)threadIdx.x + i * GL_T < n) {
+      const int32_t b = bin(k[i]), s0 = bins[b],
+                    s1 = b + 1 < nbin ? bins[b + 1] : n;
+      int32_t p = s0;
+      for (int32_t j = s0; j < s1; j++) p += kb[j] < k[i];
+      r[i] = p;
+    }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < SORT_PER; i++)
+    if ((int32_t)threadIdx.x + i * GL_T < n) dst[r[i]] = k[i];
+  __threadfence_block();
+  __syncthreads();
+  return true;
+}
+
 // Pool slots reserved for n collected keys: n itself when the keys are
 // sorted in LDS, the next power of two otherwise (padding for the bitonic
 // network on global memory).
 __device__ inline int64_t pool_slots(int64_t n) {
-  if (n <= SORT_CAP) return n;
+  if (n <= SORT_LDS) return n;
   int64_t p = 1;
   while (p < n) p <<= 1;
   return p;
 }
 
-// sorts the n keys at pool[0..n) ascending; pool holds pool_slots(n) slots
-__device__ void block_sort_pool(uint64_t *pool, int32_t n, GrowShared &G) {
+// the n <= SORT_LDS keys at p[0..n) sorted in place; K, bins: LDS
+__device__ inline void block_sort_lds(uint64_t *p, int32_t n, uint64_t *K,
+                                      int32_t *bins, GrowShared &G,
+                                      const uint64_t *src) {
+  if (block_bin_sort(src, p, n, K, bins, G)) return;
+  const int np = next_pow2(n < 2 ? 2 : n);
+  for (int i = n + threadIdx.x; i < np; i += GL_T) K[i] = ~0ull;
+  __syncthreads();
+  lds_bitonic<GL_T>(K, np);
+  for (int i = threadIdx.x; i < n; i += GL_T) p[i] = K[i];
+  __threadfence_block();
+  __syncthreads();
+}
+
+// The smallest keys of p[0..n), n > SORT_LDS, up to a bin edge of their
+// distance bits and at most SORT_LDS of them, moved to p[0..m) and sorted;
+// the others fill p[m..n) in any order.  Returns m; 0 when the first bin
+// alone holds too many (p unchanged).
+// Not inline: its registers would spill the kernel's (1024^3 growth 9.3 ms
+// against 9.0).
+__device__ __attribute__((noinline)) int32_t
+block_sort_head(uint64_t *p, int32_t n, uint64_t *K, int32_t *bins,
+                GrowShared &G) {
+  const int l = threadIdx.x & 63, w = threadIdx.x >> 6;
+  uint32_t lo = 0xFFFFFFFFu, hi = 0u;
+  for (int32_t i = threadIdx.x; i < n; i += GL_T) {
+    lo = min(lo, (uint32_t)(p[i] >> 32));
+    hi = max(hi, (uint32_t)(p[i] >> 32));
+  }
+  lo = ~wave_max_u32(~lo);
+  hi = wave_max_u32(hi);
+  for (int32_t b = threadIdx.x; b < SORT_LDS; b += GL_T) bins[b] = 0;
+  if (l == 0) {
+    G.pre[w] = (int32_t)lo;
+    G.pre[w + GL_T / 64] = (int32_t)hi;
+  }
+  if (threadIdx.x == 0) G.pre[32] = G.pre[33] = G.pre[34] = 0;
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < GL_T / 64; i++) {
+    lo = min(lo, (uint32_t)G.pre[i]);
+    hi = max(hi, (uint32_t)G.pre[i + GL_T / 64]);
+  }
+  if (hi - lo > (20u << 23)) lo = hi - (20u << 23);
+  int sh = 0;
+  while (((hi - lo) >> sh) >= (uint32_t)SORT_LDS) sh++;
+  auto bin = [&](uint64_t x) {
+    const uint32_t u = (uint32_t)(x >> 32);
+    return u > lo ? (int32_t)((u - lo) >> sh) : 0;
+  };
+  for (int32_t i = threadIdx.x; i < n; i += GL_T) atomicAdd(&bins[bin(p[i])], 1);
+  __syncthreads();
+  // the bin where the prefix passes SORT_LDS
+  constexpr int32_t per = SORT_LDS / (GL_T / 64);
+  int32_t run = 0;
+  for (int32_t b = w * per + l; b < (w + 1) * per; b += 64)
+    run += __builtin_amdgcn_readlane(wave_incl_scan(bins[b]), 63);
+  if (l == 0) G.red_i[w] = run;
+  __syncthreads();
+  run = 0;
+  for (int i = 0; i < w; i++) run += G.red_i[i];
+  for (int32_t b = w * per + l; b < (w + 1) * per; b += 64) {
+    const int32_t v = bins[b], inc = wave_incl_scan(v);
+    if (run + inc > SORT_LDS && run + inc - v <= SORT_LDS) {
+      G.pre[36] = b;
+      G.pre[37] = run + inc - v;
+    }
+    run += __builtin_amdgcn_readlane(inc, 63);
+  }
+  __syncthreads();
+  const int32_t cut = G.pre[36], m = G.pre[37];
+  if (m == 0) return 0;  // uniform
+  int32_t *vac = bins;  // places at m and after that the moved keys leave
+  const uint64_t below = l == 0 ? 0ull : (~0ull >> (64 - l));
+  for (int32_t b0 = 0; b0 < n; b0 += GL_T) {
+    const int32_t i = b0 + (int32_t)threadIdx.x;
+    const uint64_t x = i < n ? p[i] : ~0ull;
+    const bool sel = i < n && bin(x) < cut;
+    const uint64_t ms = __ballot(sel), mv = __ballot(sel && i >= m);
+    int32_t s0 = 0, v0 = 0;
+    if (l == 0 && ms) s0 = atomicAdd(&G.pre[32], (int32_t)__popcll(ms));
+    if (l == 0 && mv) v0 = atomicAdd(&G.pre[33], (int32_t)__popcll(mv));
+    s0 = __builtin_amdgcn_readfirstlane(s0);
+    v0 = __builtin_amdgcn_readfirstlane(v0);
+    if (sel) K[s0 + __popcll(ms & below)] = x;
+    if (sel && i >= m) vac[v0 + __popcll(mv & below)] = i;
+  }
+  __syncthreads();
+  for (int32_t i = threadIdx.x; i < m; i += GL_T) {
+    const uint64_t x = p[i];
+    if (bin(x) >= cut) p[vac[atomicAdd(&G.pre[34], 1)]] = x;
+  }
+  __threadfence_block();
+  __syncthreads();
+  block_sort_lds(p, m, K, bins, G, K);
+  return m;
+}
+
+// sorts the n keys at pool[0..n) ascending; pool holds pool_slots(n) slots;
+// lh: LDS of SORT_LDS keys, overwritten.  Up to SORT_HEADS pieces of
+// SORT_LDS keys are taken off the smallest keys one after the other (two
+// reads of the rest each): bands of 2.3e4 keys in three ranges 1.04 -> 0.14
+// ms (k_grow_large 512^3, 4 thresholds, 2.8 -> 2.1 ms), k_giant_cross at
+// 1024^3 5.0 -> 1.1 ms.
+constexpr int32_t SORT_HEADS = 8;
+__device__ void block_sort_pool(uint64_t *pool, int32_t n, GrowShared &G,
+                                int32_t *lh) {
   if (n <= 1) return;
-  if (n <= SORT_CAP) {
-    const int np = next_pow2(n);
-    for (int i = threadIdx.x; i < np; i += GL_T)
-      G.skey[i] = i < n ? pool[i] : ~0ull;
-    __syncthreads();
-    lds_bitonic<GL_T>(G.skey, np);
-    for (int i = threadIdx.x; i < n; i += GL_T) pool[i] = G.skey[i];
-    __threadfence_block();
-    __syncthreads();
-    return;
+  static_assert(sizeof(G.skey) >= SORT_LDS * 4, "the bins live in skey");
+  if (n <= SORT_LDS * SORT_HEADS) {
+    uint64_t *K = (uint64_t *)lh;
+    int32_t *bins = (int32_t *)G.skey;
+    int32_t done = 0;
+    bool cut = true;
+    while (cut && n - done > SORT_LDS) {
+      const int32_t m = block_sort_head(pool + done, n - done, K, bins, G);
+      cut = m > 0;
+      done += m;
+    }
+    if (cut) {
+      block_sort_lds(pool + done, n - done, K, bins, G, pool + done);
+      return;
+    }
   }
   // The bitonic network over np = next_pow2(n) keys (padding ~0 sorts
   // last).  Its steps (k, j) with j < SORT_CAP pair keys of one block of
@@ -2833,7 +3068,8 @@ __device__ inline int32_t grow_cross(const SodCfg &c, GrowShared &G,
                                      const int32_t *hist, uint64_t *pool,
                                      const float *pos, GrowVars &V,
                                      HaloResult &res, const double *xcs,
-                                     int64_t pool_cap, uint32_t presorted) {
+                                     int64_t pool_cap, uint32_t presorted,
+                                     int32_t *lh) {
   const int32_t *C = hist;
   const int32_t nb = V.nb;
   const float scale = V.scale;
@@ -2842,7 +3078,7 @@ __device__ inline int32_t grow_cross(const SodCfg &c, GrowShared &G,
   const int nr = G.nr;
   for (int r = 0; r < nr; r++)
     if (!((presorted >> r) & 1))
-      block_sort_pool(pool + G.off[r], (int32_t)(G.k1[r] - G.k0[r]), G);
+      block_sort_pool(pool + G.off[r], (int32_t)(G.k1[r] - G.k0[r]), G, lh);
   // key of rank k (1-based) among the collected ranges
   auto key_rank = [&](int64_t k) {
     int r = 0;
@@ -2997,7 +3233,7 @@ __device__ inline void grow_finish(const SodCfg &c, GrowShared &G,
                                    uint64_t *pool, const float *pos,
                                    const GrowVars &V, HaloResult &res,
                                    const double *xcs, const ProfileSums &S,
-                                   psod_halo_out out) {
+                                   psod_halo_out out, int32_t *lh) {
   const CellRef &cr = V.cr;
   const int32_t nin = res.count[0];
   const double xc[3] = {(double)cr.c[0] + (double)cr.f[0],
@@ -3029,7 +3265,7 @@ __device__ inline void grow_finish(const SodCfg &c, GrowShared &G,
       for (int j = 0; j < V.ns2 && best == 0; j++) {
         const int32_t n2 = (int32_t)(G.k1[R2 + j] - G.k0[R2 + j]);
         uint64_t *p2 = pool + G.off[R2 + j];
-        block_sort_pool(p2, n2, G);
+        block_sort_pool(p2, n2, G, lh);
         const int64_t kb = G.k0[R2 + j];
         int32_t bestk = -1;
         for (int32_t t = threadIdx.x; t < n2; t += GL_T) {
@@ -3088,7 +3324,7 @@ __device__ inline void grow_close(const SodCfg &c, int32_t *counters,
 // bin surely holds a crossing.  Returns 0 with res and the profile written,
 // else the reach to try next.  A halo whose cube held a few thousand
 // particles took 150-190 us through the bins and the three walks.
-static_assert(LIGHT_CAP <= HIST_LDS / 2, "light keys live in the bins' LDS");
+static_assert(LIGHT_CAP <= HIST_LDS / 2 && LIGHT_CAP <= SORT_LDS, "light keys live in the bins' LDS");
 
 __device__ __forceinline__ int32_t
 grow_light(const SodCfg &c, GrowShared &G, uint64_t *K,
@@ -3099,10 +3335,13 @@ grow_light(const SodCfg &c, GrowShared &G, uint64_t *K,
   cube_walk(c, G, cell_start, rec, cr, W, -1.0f, INFINITY,
             [&](float d2, int32_t idx, const float4 &, int, int, int,
                 const int32_t *, int64_t j) { K[j] = d2key(d2, idx); });
-  const int32_t np = next_pow2(n < 2 ? 2 : n);
-  for (int32_t j = n + threadIdx.x; j < np; j += GL_T) K[j] = ~0ull;
   __syncthreads();
-  lds_bitonic<GL_T>(K, np);
+  if (!block_bin_sort(K, K, n, K, (int32_t *)G.skey, G)) {
+    const int32_t np = next_pow2(n < 2 ? 2 : n);
+    for (int32_t j = n + threadIdx.x; j < np; j += GL_T) K[j] = ~0ull;
+    __syncthreads();
+    lds_bitonic<GL_T>(K, np);
+  }
   // The ranks, the reach test and the growth of the reach are those of the
   // binned steps: only particles with d2 < W^2 are ranked (they sort before
   // the others), a threshold not crossed among them doubles the reach, and
@@ -3501,7 +3740,7 @@ k_grow_large(SodCfg c, const int32_t *__restrict__ cell_start,
       __threadfence_block();
       __syncthreads();
       for (int r = 0; r < nr; r++)
-        block_sort_pool(pool + G.off[r], (int32_t)(G.k1[r] - G.k0[r]), G);
+        block_sort_pool(pool + G.off[r], (int32_t)(G.k1[r] - G.k0[r]), G, lh);
       // key of rank k (1-based) among the collected ranges
       auto key_rank = [&](int64_t k) {
         int r = 0;
@@ -3704,7 +3943,7 @@ k_grow_large(SodCfg c, const int32_t *__restrict__ cell_start,
           for (int j = 0; j < ns2 && best == 0; j++) {
             const int32_t n2 = (int32_t)(G.k1[R2 + j] - G.k0[R2 + j]);
             uint64_t *p2 = pool + G.off[R2 + j];
-            block_sort_pool(p2, n2, G);
+            block_sort_pool(p2, n2, G, lh);
             const int64_t kb = G.k0[R2 + j];
             int32_t bestk = -1;
             for (int32_t t = threadIdx.x; t < n2; t += GL_T) {
@@ -4215,6 +4454,7 @@ k_giant_cross(SodCfg c, GiantState *__restrict__ S,
               unsigned long long *__restrict__ needmax, psod_halo_out out,
               int32_t *__restrict__ wq) {
   __shared__ GrowShared G;
+  __shared__ __align__(16) int32_t lh[HIST_LDS];  // keys of a sort
   if (blockIdx.x == 0 && threadIdx.x == 0) wq[3] = 0;
   GiantState &T = S[blockIdx.x];
   const int32_t step0 = T.step;
@@ -4227,7 +4467,8 @@ k_giant_cross(SodCfg c, GiantState *__restrict__ S,
   HaloResult res = T.res;
   double xcs[3] = {T.xcs[0], T.xcs[1], T.xcs[2]};
   const int32_t step =
-      grow_cross(c, G, hist, pool, pos, V, res, xcs, pool_cap, T.presorted);
+      grow_cross(c, G, hist, pool, pos, V, res, xcs, pool_cap, T.presorted,
+                 lh);
   __syncthreads();
   if (step == GS_FAILED)
     grow_close(c, counters, retry, needmax, G.need, V, res, true, out);
@@ -4251,6 +4492,7 @@ k_giant_finish(SodCfg c, GiantState *__restrict__ S,
                int32_t *__restrict__ retry,
                unsigned long long *__restrict__ needmax, psod_halo_out out) {
   __shared__ GrowShared G;
+  __shared__ __align__(16) int32_t lh[HIST_LDS];  // keys of a sort
   GiantState &T = S[blockIdx.x];
   const int32_t step0 = T.step;
   __syncthreads();
@@ -4268,7 +4510,7 @@ k_giant_finish(SodCfg c, GiantState *__restrict__ S,
   uint64_t *pool = pool_all + (int64_t)blockIdx.x * pool_cap;
   HaloResult res = T.res;
   double xcs[3] = {T.xcs[0], T.xcs[1], T.xcs[2]};
-  grow_finish(c, G, pool, pos, V, res, xcs, P, out);
+  grow_finish(c, G, pool, pos, V, res, xcs, P, out, lh);
   grow_close(c, counters, retry, needmax, 0, V, res, false, out);
   if (threadIdx.x == 0) T.step = GS_DONE;
 }
