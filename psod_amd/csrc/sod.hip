@@ -786,9 +786,7 @@ __device__ inline float box_gap2(const float *a0, const float *a1,
 
 // Halos with fewer than SodCfg::bound_min particles in the 5^3 cells around
 // the seed (a tunable, 1024 by default) skip the bound: bounding costs about
-// as much as their exact sums.  With the items abandoned cell by cell,
-// 1024 gave 140.6 ms of SOD at c3 against 144.2 (2048), 141.6 (512) and
-// 149.8 ms (4096).
+// as much as their exact sums.
 
 // Upper bound of the term of any pair at squared distance >= g2 within the
 // cutoff.  The float d2 of a pair is at least g2 up to a few ulps, hence the
@@ -1396,6 +1394,36 @@ __device__ __forceinline__ uint64_t pilot_walk(const SodCfg &c,
 // catalogue at 512^3 0.82 + 0.36 -> 0.25 + 0.39, 1024^3 2.1 + 0.8 -> 1.2 +
 // 1.4).
 constexpr int32_t PILOT_PIECES = 64, PILOT_CHUNKS = 16;
+// A launch of few pilots (at most PILOT_FEW per CU) leaves most waves idle
+// while one wave walks 2^11 records in 0.2 ms: there the pieces start at
+// 2^8 records and hold 4 chunks (pilots and pieces, us: 256^3 199 + 148 ->
+// 104 + 145, 128^3 232 + 172 -> 118 + 132; pieces of 2 chunks 104 + 184).
+constexpr int32_t PILOT_FEW = 8;
+__device__ inline int32_t pilot_chunks(int32_t nlist, int32_t few) {
+  return nlist <= few ? PILOT_CHUNKS / 4 : PILOT_CHUNKS;
+}
+
+// The tasks that are pilots (their estimate is the halo's largest), listed:
+// waves of k_centre_pilot that looked for them among 16 tasks each held up to
+// 16 pilots (1024^3 1.40 -> 0.70 + 0.15 ms, 512^3 with many halos below
+// bound_min 1.65 -> 0.89).
+__global__ void __launch_bounds__(256)
+k_pilot_list(const int4 *__restrict__ tasks,
+             const int32_t *__restrict__ ntask_total,
+             const unsigned long long *__restrict__ hpil,
+             const uint32_t *__restrict__ est, int32_t *__restrict__ list,
+             int32_t *__restrict__ nlist) {
+  const int32_t t = blockIdx.x * blockDim.x + threadIdx.x;
+  const bool on = t < *ntask_total && est[t] == hpil[tasks[t].x];
+  const uint64_t m = __ballot(on);
+  if (m == 0) return;
+  const int l = threadIdx.x & 63;
+  int32_t base = 0;
+  if (l == 0) base = atomicAdd(nlist, (int32_t)__popcll(m));
+  base = __builtin_amdgcn_readfirstlane(base);
+  if (on)
+    list[base + __popcll(m & (l == 0 ? 0ull : (~0ull >> (64 - l))))] = t;
+}
 
 // Pilots, one wave per task: the 64 candidates of a task (one per lane)
 // against the 27 cells around their cell (every neighbour within 1 cell lies
@@ -1410,69 +1438,67 @@ __global__ void __launch_bounds__(256)
 k_centre_pilot(SodCfg c, const int32_t *__restrict__ cell_start,
                const float4 *__restrict__ rec, const HaloPlan *__restrict__ plan,
                const int32_t *__restrict__ large, const int4 *__restrict__ tasks,
-               const int32_t *__restrict__ ntask_total,
+               const int32_t *__restrict__ list,
+               const int32_t *__restrict__ nlist,
                uint64_t *__restrict__ taskres,
                unsigned long long *__restrict__ hbest,
-               const unsigned long long *__restrict__ hpil,
-               const uint32_t *__restrict__ est,
                unsigned long long *__restrict__ cstat,
-               int32_t pilot_big, int32_t bigcap, int32_t *__restrict__ big,
+               int32_t pilot_big, int32_t few, int32_t bigcap, int32_t *__restrict__ big,
                int32_t *__restrict__ units, int32_t *__restrict__ nbig,
                unsigned long long *__restrict__ pacc,
                int32_t *__restrict__ wq) {
   __shared__ float4 nbuf[4][64];  // one neighbour chunk per wave
   const int l = threadIdx.x & 63,
             w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-  const int32_t nt = *ntask_total;
+  const int32_t nt = *nlist;
+  const int32_t per = pilot_chunks(nt, few);
+  if (nt <= few) pilot_big = min(pilot_big, 1 << 8);
   const float cut = c.rs2f * 1.0001f + 1e-6f;  // conservative chunk culling
   // this wave's statistics, added once at the end
   unsigned long long st_done = 0, st_pairs = 0;
   for (;;) {
-    const int32_t t0 = wave_next(wq) * 16;
-    if (t0 >= nt) break;
-    const int32_t t1 = min(nt, t0 + 16);
-    for (int32_t t = t0; t < t1; t++) {
-      const int4 tk = tasks[t];
-      if (est[t] != hpil[tk.x]) continue;
-      const HaloPlan pl = plan[large[tk.x]];
-      PilotSetup P;
-      pilot_setup(c, cell_start, rec, pl, tk, l, cut, P);
-      if (wave_sum(P.qb - P.qa) > pilot_big) {
-        const int32_t C = wave_sum((P.qb - P.qa + 63) >> 6);
-        const int32_t np = min(PILOT_PIECES, (C + PILOT_CHUNKS - 1) / PILOT_CHUNKS);
-        int32_t k = 0;
-        if (l == 0) k = atomicAdd(&nbig[0], 1);
-        k = __builtin_amdgcn_readfirstlane(k);
-        if (k < bigcap) {
-          int32_t u = 0;
-          if (l == 0) {
-            big[k] = t;
-            u = atomicAdd(&nbig[1], np);
-          }
-          u = __builtin_amdgcn_readfirstlane(u);
-          if (l < np) units[u + l] = (k << 6) | l;
-          pacc[(int64_t)k * 64 + l] = 0;
-          continue;
+    const int32_t i = wave_next(wq);
+    if (i >= nt) break;
+    const int32_t t = list[i];
+    const int4 tk = tasks[t];
+    const HaloPlan pl = plan[large[tk.x]];
+    PilotSetup P;
+    pilot_setup(c, cell_start, rec, pl, tk, l, cut, P);
+    if (wave_sum(P.qb - P.qa) > pilot_big) {
+      const int32_t C = wave_sum((P.qb - P.qa + 63) >> 6);
+      const int32_t np = min(PILOT_PIECES, (C + per - 1) / per);
+      int32_t k = 0;
+      if (l == 0) k = atomicAdd(&nbig[0], 1);
+      k = __builtin_amdgcn_readfirstlane(k);
+      if (k < bigcap) {
+        int32_t u = 0;
+        if (l == 0) {
+          big[k] = t;
+          u = atomicAdd(&nbig[1], np);
         }
+        u = __builtin_amdgcn_readfirstlane(u);
+        if (l < np) units[u + l] = (k << 6) | l;
+        pacc[(int64_t)k * 64 + l] = 0;
+        continue;
       }
-      uint64_t rest = __ballot(l < 27 && P.qa < P.qb);  // cells with records
-      const int q = rest ? __ffsll((unsigned long long)rest) - 1 : 27;
-      const int32_t s = q < 27 ? __builtin_amdgcn_readlane(P.qa, q) : 0;
-      uint64_t npair = 0;  // neighbours tested per candidate
-      uint64_t acc = pilot_walk(c, rec, pl, P, nbuf[w], l, cut, rest, q, s,
-                                INT32_MAX, npair);
-      uint64_t key = P.have
-                         ? (((uint64_t)(uint32_t)tk.y << 32) | (uint32_t)P.pidx)
-                         : ~0ull;
-      if (!P.have) acc = 0;
-      wave_argmax(acc, key);
-      if (l == 0) {
-        taskres[2 * (int64_t)t] = acc;
-        taskres[2 * (int64_t)t + 1] = key;
-        atomicMax(&hbest[tk.x], (unsigned long long)acc);
-        st_done++;
-        st_pairs += npair * (uint64_t)tk.w;
-      }
+    }
+    uint64_t rest = __ballot(l < 27 && P.qa < P.qb);  // cells with records
+    const int q = rest ? __ffsll((unsigned long long)rest) - 1 : 27;
+    const int32_t s = q < 27 ? __builtin_amdgcn_readlane(P.qa, q) : 0;
+    uint64_t npair = 0;  // neighbours tested per candidate
+    uint64_t acc = pilot_walk(c, rec, pl, P, nbuf[w], l, cut, rest, q, s,
+                              INT32_MAX, npair);
+    uint64_t key = P.have
+                       ? (((uint64_t)(uint32_t)tk.y << 32) | (uint32_t)P.pidx)
+                       : ~0ull;
+    if (!P.have) acc = 0;
+    wave_argmax(acc, key);
+    if (l == 0) {
+      taskres[2 * (int64_t)t] = acc;
+      taskres[2 * (int64_t)t + 1] = key;
+      atomicMax(&hbest[tk.x], (unsigned long long)acc);
+      st_done++;
+      st_pairs += npair * (uint64_t)tk.w;
     }
   }
   if (l == 0 && st_done) {
@@ -1494,13 +1520,14 @@ k_centre_pilot_big(SodCfg c, const int32_t *__restrict__ cell_start,
                    const int32_t *__restrict__ big,
                    const int32_t *__restrict__ units,
                    const int32_t *__restrict__ nbig,
+                   const int32_t *__restrict__ nlist, int32_t few,
                    unsigned long long *__restrict__ pacc,
                    unsigned long long *__restrict__ cstat,
                    int32_t *__restrict__ wq) {
   __shared__ float4 nbuf[4][64];  // one neighbour chunk per wave
   const int l = threadIdx.x & 63,
             w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-  const int32_t nu = nbig[1];
+  const int32_t nu = nbig[1], pch = pilot_chunks(*nlist, few);
   const float cut = c.rs2f * 1.0001f + 1e-6f;  // conservative chunk culling
   unsigned long long st_pairs = 0;
   for (;;) {
@@ -1516,7 +1543,7 @@ k_centre_pilot_big(SodCfg c, const int32_t *__restrict__ cell_start,
     const int32_t nch = l < 27 ? (P.qb - P.qa + 63) >> 6 : 0;
     int32_t C;
     const int32_t ex = wave_excl(nch, &C);
-    const int32_t np = min(PILOT_PIECES, (C + PILOT_CHUNKS - 1) / PILOT_CHUNKS);
+    const int32_t np = min(PILOT_PIECES, (C + pch - 1) / pch);
     const int32_t per = (C + np - 1) / np;
     const int32_t k0 = p * per;
     if (k0 >= C) continue;
@@ -4697,8 +4724,8 @@ static int centre_search(psod_ctx *ctx, const SodCfg &c,
   int32_t *items = (int32_t *)(ires + 8 * (int64_t)tcap);
   uint32_t *est = (uint32_t *)(items + 4 * (int64_t)tcap);
   int32_t *nitems = (int32_t *)(est + (((int64_t)tcap + 1) & ~1));
-  // work counters of the bound, pilot, group and split-pilot launches, and
-  // the count of split pilot tasks
+  // work counters of the bound, pilot, group and split-pilot launches, the
+  // counts of split pilot tasks and their pieces, and (wq[7]) of the pilots
   int32_t *wq = nitems + 4;
   int32_t *nbig = wq + 4;
   // split pilot tasks, their per-candidate totals and their pieces
@@ -4744,15 +4771,20 @@ static int centre_search(psod_ctx *ctx, const SodCfg &c,
                                       tasks, ntot, hpil, est, ubt, ubx, gwin,
                                       wq);
   PSOD_LAUNCH_CHECK();
+  const int32_t few = PILOT_FEW * ctx->num_cus;
+  // the list of pilots takes the work list's place until that is made
+  k_pilot_list<<<grid_for(tcap, 256), 256, 0, st>>>(tasks, ntot, hpil, est,
+                                                    items, wq + 7);
+  PSOD_LAUNCH_CHECK();
   k_centre_pilot<<<resident((const void *)k_centre_pilot), 256, 0, st>>>(
-      c, cat->cell_start, (const float4 *)cat->rec, plan, large, tasks, ntot,
-      tres, hbest, hpil, est, cstat, pilot_big(), bigcap, big, units, nbig, pacc,
-      wq + 1);
+      c, cat->cell_start, (const float4 *)cat->rec, plan, large, tasks, items,
+      wq + 7, tres, hbest, cstat, pilot_big(), few, bigcap, big, units, nbig,
+      pacc, wq + 1);
   PSOD_LAUNCH_CHECK();
   k_centre_pilot_big<<<resident((const void *)k_centre_pilot_big), 256, 0,
                        st>>>(c, cat->cell_start, (const float4 *)cat->rec,
-                             plan, large, tasks, big, units, nbig, pacc,
-                             cstat, wq + 3);
+                             plan, large, tasks, big, units, nbig, wq + 7, few,
+                             pacc, cstat, wq + 3);
   PSOD_LAUNCH_CHECK();
   k_centre_pilot_fin<<<grid_for(bigcap, 4), 256, 0, st>>>(
       (const float4 *)cat->rec, tasks, big, bigcap, nbig, pacc, tres, hbest,
