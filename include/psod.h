@@ -61,7 +61,7 @@ int64_t psod_scratch_bytes(psod_ctx *ctx);
  * tasks of 64 candidates and items of 16), out[5] units skipped by their
  * upper bound, out[6] candidate-neighbour pair tests, out[7] centre-search
  * tasks in all, out[8] centre-search time in ns, out[9] items abandoned
- * part way (exact sums plus the bound of the remaining neighbour cells
+ * part way (exact sums plus the bound of the remaining neighbours
  * below the best S), out[10] giant halos grown by the staged launches,
  * out[11] their cycles (a cycle per reach tried), out[12] halos of the
  * workgroup path whose growth cube was sorted whole in LDS.

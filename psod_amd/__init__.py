@@ -322,7 +322,7 @@ class Context:
         one wave, by one workgroup, re-run with larger collection slices,
         the keys per slice of that re-run, and the centre search of the
         large halos: its tasks (64 candidates of one cell) in all, units
-        evaluated exactly (pilot tasks and groups of 8 candidates), units
+        evaluated exactly (pilot tasks and boxes of 16 candidates), units
         skipped by their bound, groups abandoned part-way, pair tests and
         the search's time; giant halos grown by the staged launches and
         their cycles; workgroup halos whose growth cube was sorted whole in
