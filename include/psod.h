@@ -362,7 +362,9 @@ int psod_density_order_f64(psod_ctx *ctx, int64_t npart, const double *d_rho,
  *                       overdens2, accepted(0/1)
  *   rad_bins [maxrec*nbins], mass_bins [maxrec*nbins]
  *   alive [npart] final exclusion flags; structure [npart] accepted iamas.
- * Returns PSOD_E_CAPACITY / PSOD_E_UNCLOSED like the reference's zone abort. */
+ * Returns PSOD_E_CAPACITY / PSOD_E_UNCLOSED like the reference's zone abort,
+ * at the first failing seed in seed order; the outputs are then those of the
+ * seeds before it. */
 typedef struct {
   int32_t nx, ncut;
   double seuil, seuil2, mmin;

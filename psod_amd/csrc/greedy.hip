@@ -57,8 +57,18 @@ struct GState {
   int32_t first[2];              // first unprocessed seed order
   int32_t nready[2], nunits[2];
   int32_t total, nrec;           // ready seeds so far, records so far
+  int32_t last;                  // largest order of a seed with a record
 };
 enum { GF_NSEL = 1, GF_GCAP = 2, GF_UNCLOSED = 3 };
+
+// End of the orders still to run, within the window from lo: a failed seed
+// ends the zone, but the seeds before it that wait on their neighbours run
+// on (one of them may be the first to fail); those after it do not count.
+__device__ inline int32_t window_end(const GState *S, int32_t npart_new,
+                                     int32_t lo) {
+  const int64_t end = (int64_t)min((unsigned long long)npart_new, S->fail >> 8);
+  return (int32_t)min(end, lo + GWIN);
+}
 
 // One ready seed of a round: its pool entries [off, off + n1), of which the
 // first nnear / ncand entries of the near / candidate lists are set; its
@@ -127,7 +137,7 @@ k_mark(GreedyCfg c, const int32_t *__restrict__ isort,
        int32_t npart_new, int par, GState *__restrict__ S,
        int32_t *__restrict__ bmin) {
   const int32_t lo = S->first[1 - par];
-  const int32_t hi = (int32_t)min((int64_t)npart_new, lo + GWIN);
+  const int32_t hi = window_end(S, npart_new, lo);
   const int64_t o = lo + (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (blockIdx.x == 0 && threadIdx.x == 0) {
     S->total += S->nready[1 - par];
@@ -136,7 +146,7 @@ k_mark(GreedyCfg c, const int32_t *__restrict__ isort,
     S->nunits[par] = 0;
     S->cursor[par] = 0;
   }
-  if (o >= hi || done[o] || S->fail != ~0ull) return;
+  if (o >= hi || done[o]) return;
   const int32_t s = isort[o] - 1;
   if (!alive[slot_of[s]]) return;
   int32_t b[3];
@@ -157,9 +167,8 @@ k_ready(GreedyCfg c, const int32_t *__restrict__ isort,
         int32_t npart_new, int par, GState *__restrict__ S,
         const int32_t *__restrict__ bmin, int32_t *__restrict__ ready) {
   const int32_t lo = S->first[1 - par];
-  const int32_t hi = (int32_t)min((int64_t)npart_new, lo + GWIN);
+  const int32_t hi = window_end(S, npart_new, lo);
   const int64_t o = lo + (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (S->fail != ~0ull) return;
   int32_t open = INT32_MAX;
   bool go = false;
   if (o < hi && !done[o]) {
@@ -850,7 +859,10 @@ k_greedy_grow(GreedyCfg c, const int32_t *__restrict__ isort,
     const double rayon = rad(masse - 1);
     const double volume = 2.0 / 3.0 * TWOPI_REF * (rayon * rayon * rayon);
     const double amass = (double)masse;
-    if (threadIdx.x == 0) S.n = atomicAdd(&St->nrec, 1);
+    if (threadIdx.x == 0) {
+      S.n = atomicAdd(&St->nrec, 1);
+      atomicMax(&St->last, o);
+    }
     __syncthreads();
     const int64_t row = S.n;
     // profile (main file:2103-2115): counts of r < r_j.  Every particle
@@ -1023,59 +1035,75 @@ extern "C" int psod_host_spherover(psod_ctx *ctx, int64_t npart,
     PSOD_HIP(hipMemcpyAsync(dids, ids, (size_t)npart * 8, hipMemcpyHostToDevice, st));
   k_inverse_perm<<<grid_for(npart, 256), 256, 0, st>>>(perm, npart, slot_of);
   PSOD_LAUNCH_CHECK();
-  k_set_u8<<<grid_for(npart, 256, 4096), 256, 0, st>>>(alive_s, npart, 1);
-  PSOD_LAUNCH_CHECK();
-  PSOD_HIP(hipMemsetAsync(dstruct, 0, (size_t)npart * 8, st));
-  PSOD_HIP(hipMemsetAsync(done, 0, (size_t)nn, st));
   // isort: 1-based particle indices
   if (npart_new > 0)
     PSOD_HIP(hipMemcpyAsync(dseeds, isort, (size_t)npart_new * 4,
                             hipMemcpyHostToDevice, st));
-  PSOD_TRY(psod_fill_i32(ctx, bmin, nbk, INT32_MAX));
+  // The seeds of orders below nnew, from the start: rounds over a sliding
+  // window of seeds, GROUNDS of them queued at a time; the window, the counts
+  // and the work lists stay on the device.
   GState hs;
-  memset(&hs, 0, sizeof(hs));
-  hs.fail = ~0ull;
-  PSOD_HIP(hipMemcpyAsync(S, &hs, sizeof(hs), hipMemcpyHostToDevice, st));
-  PSOD_HIP(hipStreamSynchronize(st));
-  // Rounds over a sliding window of seeds, GROUNDS of them queued at a time:
-  // the window, the counts and the work lists stay on the device.
-  const int32_t nnew = (int32_t)npart_new;
-  int32_t lo = 0;
-  int64_t ran = 0;  // ready seeds so far
-  while (lo < nnew && hs.fail == ~0ull) {
-    const int32_t lo0 = lo;
-    for (int r = 0; r < GROUNDS; r++) {
-      const int par = r & 1;
-      // the window starts at lo0 or later
-      const unsigned gw = grid_for(std::min<int64_t>(GWIN, nnew - lo0), 256);
-      k_mark<<<gw, 256, 0, st>>>(c, dseeds, slot_of, dpos, alive_s, done, nnew,
-                                 par, S, bmin);
-      PSOD_LAUNCH_CHECK();
-      k_ready<<<gw, 256, 0, st>>>(c, dseeds, slot_of, dpos, alive_s, done,
-                                  nnew, par, S, bmin, ready);
-      PSOD_LAUNCH_CHECK();
-      k_greedy_gather<<<(unsigned)ctx->num_cus, GA_T, 0, st>>>(
-          c, dseeds, cs, (const float4 *)drec, dpos, alive_s, done, par, S,
-          ready, info, units, G, pcap);
-      PSOD_LAUNCH_CHECK();
-      k_greedy_bound<<<(unsigned)ctx->num_cus * 4, GC_T, 0, st>>>(
-          par, S, info, units, G);
-      PSOD_LAUNCH_CHECK();
-      k_greedy_centre<<<(unsigned)ctx->num_cus * 4, 256, 0, st>>>(
-          c, dseeds, dpos, par, S, ready, info, units, G, ures, bmin, nbk);
-      PSOD_LAUNCH_CHECK();
-      k_greedy_grow<<<(unsigned)ctx->num_cus, GG_T, 0, st>>>(
-          c, dseeds, dpos, ids ? dids : nullptr, alive_s, done, par, S, ready,
-          info, ures, G, dstruct, recs, radb, massb);
-      PSOD_LAUNCH_CHECK();
-    }
-    PSOD_HIP(hipMemcpyAsync(&hs, S, sizeof(hs), hipMemcpyDeviceToHost, st));
+  auto run = [&](int32_t nnew) -> int {
+    k_set_u8<<<grid_for(npart, 256, 4096), 256, 0, st>>>(alive_s, npart, 1);
+    PSOD_LAUNCH_CHECK();
+    PSOD_HIP(hipMemsetAsync(dstruct, 0, (size_t)npart * 8, st));
+    PSOD_HIP(hipMemsetAsync(done, 0, (size_t)nn, st));
+    PSOD_TRY(psod_fill_i32(ctx, bmin, nbk, INT32_MAX));
+    memset(&hs, 0, sizeof(hs));
+    hs.fail = ~0ull;
+    hs.last = -1;
+    PSOD_HIP(hipMemcpyAsync(S, &hs, sizeof(hs), hipMemcpyHostToDevice, st));
     PSOD_HIP(hipStreamSynchronize(st));
-    lo = hs.first[(GROUNDS - 1) & 1];
-    const int64_t r1 = (int64_t)hs.total + hs.nready[(GROUNDS - 1) & 1];
-    if (hs.fail == ~0ull && lo == lo0 && r1 == ran)
-      return psod_set_error(PSOD_E_DEVICE, "spherover: no progress");
-    ran = r1;
+    int32_t lo = 0, end = nnew;
+    int64_t ran = 0;  // ready seeds so far
+    while (lo < end) {
+      const int32_t lo0 = lo, end0 = end;
+      for (int r = 0; r < GROUNDS; r++) {
+        const int par = r & 1;
+        // the window starts at lo0 or later
+        const unsigned gw = grid_for(std::min<int64_t>(GWIN, nnew - lo0), 256);
+        k_mark<<<gw, 256, 0, st>>>(c, dseeds, slot_of, dpos, alive_s, done,
+                                   nnew, par, S, bmin);
+        PSOD_LAUNCH_CHECK();
+        k_ready<<<gw, 256, 0, st>>>(c, dseeds, slot_of, dpos, alive_s, done,
+                                    nnew, par, S, bmin, ready);
+        PSOD_LAUNCH_CHECK();
+        k_greedy_gather<<<(unsigned)ctx->num_cus, GA_T, 0, st>>>(
+            c, dseeds, cs, (const float4 *)drec, dpos, alive_s, done, par, S,
+            ready, info, units, G, pcap);
+        PSOD_LAUNCH_CHECK();
+        k_greedy_bound<<<(unsigned)ctx->num_cus * 4, GC_T, 0, st>>>(
+            par, S, info, units, G);
+        PSOD_LAUNCH_CHECK();
+        k_greedy_centre<<<(unsigned)ctx->num_cus * 4, 256, 0, st>>>(
+            c, dseeds, dpos, par, S, ready, info, units, G, ures, bmin, nbk);
+        PSOD_LAUNCH_CHECK();
+        k_greedy_grow<<<(unsigned)ctx->num_cus, GG_T, 0, st>>>(
+            c, dseeds, dpos, ids ? dids : nullptr, alive_s, done, par, S,
+            ready, info, ures, G, dstruct, recs, radb, massb);
+        PSOD_LAUNCH_CHECK();
+      }
+      PSOD_HIP(hipMemcpyAsync(&hs, S, sizeof(hs), hipMemcpyDeviceToHost, st));
+      PSOD_HIP(hipStreamSynchronize(st));
+      lo = hs.first[(GROUNDS - 1) & 1];
+      end = (int32_t)std::min<uint64_t>((uint64_t)nnew, hs.fail >> 8);
+      const int64_t r1 = (int64_t)hs.total + hs.nready[(GROUNDS - 1) & 1];
+      if (lo < end && lo == lo0 && r1 == ran && end == end0)
+        return psod_set_error(PSOD_E_DEVICE, "spherover: no progress");
+      ran = r1;
+    }
+    return PSOD_OK;
+  };
+  PSOD_TRY(run((int32_t)npart_new));
+  // Every seed before the failing one has run now.  Where seeds after it did
+  // too, in rounds before it, the seeds before it run again by themselves: the
+  // zone ends with the particles that these captured, no others.
+  const uint64_t fail = hs.fail;
+  if (fail != ~0ull && hs.last > (int64_t)(fail >> 8)) {
+    PSOD_TRY(run((int32_t)(fail >> 8)));
+    if (hs.fail != ~0ull)
+      return psod_set_error(PSOD_E_DEVICE, "spherover: seed %lld failed in a "
+                            "second run only", (long long)(hs.fail >> 8) + 1);
   }
   // records, in seed order up to the first failing seed
   const int64_t nr = hs.nrec;
@@ -1101,7 +1129,7 @@ extern "C" int psod_host_spherover(psod_ctx *ctx, int64_t npart,
     PSOD_HIP(hipMemcpyAsync(structure, dstruct, (size_t)npart * 8,
                             hipMemcpyDeviceToHost, st));
   PSOD_HIP(hipStreamSynchronize(st));
-  const int64_t upto = hs.fail == ~0ull ? npart_new : (int64_t)(hs.fail >> 8);
+  const int64_t upto = fail == ~0ull ? npart_new : (int64_t)(fail >> 8);
   std::vector<int32_t> order((size_t)nr);
   std::iota(order.begin(), order.end(), 0);
   std::sort(order.begin(), order.end(), [&](int32_t a, int32_t b) {
@@ -1135,9 +1163,9 @@ extern "C" int psod_host_spherover(psod_ctx *ctx, int64_t npart,
     k++;
   }
   *nrec = k;
-  if (hs.fail != ~0ull) {
-    const long long seed1 = (long long)(hs.fail >> 8) + 1;
-    const int code = (int)(hs.fail & 255);
+  if (fail != ~0ull) {
+    const long long seed1 = (long long)(fail >> 8) + 1;
+    const int code = (int)(fail & 255);
     if (code == GF_GCAP)
       return psod_set_error(PSOD_E_CAPACITY,
                             "spherover: seed %lld gathers more than %lld "
