@@ -1166,12 +1166,13 @@ k_centre_bound(SodCfg c, const int32_t *__restrict__ cell_start,
         int nq = 8, lim = 1;  // a small cell: one step, every lane
         if (win) {
           // windows in reach of the task's box; the cell's first and last
-          // window may be shared with its neighbours: always taken
+          // window may be shared with its neighbours: always taken, as is
+          // one with a record that is not finite (its box or reach is NaN)
           const int32_t wi = s + l;
           const bool part = (wi << 3) < a || (wi << 3) + 8 > b;
           const bool near =
               (wi << 3) < b &&
-              (part || box_d2(cur.x + ox, cur.y + oy, cur.z + oz) <= cur.w);
+              (part || !(box_d2(cur.x + ox, cur.y + oy, cur.z + oz) > cur.w));
           const uint64_t m = __ballot(near);
           if (near) wqueue[w][qn + __popcll(m & below)] = wi;
           qn += __popcll(m);
