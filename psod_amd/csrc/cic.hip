@@ -94,7 +94,9 @@ constexpr int32_t DEP_BIG = 1 << 17, DEP_PIECE = 1 << 15, DEP_BIGCAP = 512;
 
 // Tiles cut into pieces: count[0] tiles (slots), count[1] pieces; slot s is
 // tile[s], in np[s] pieces, done[s] of them finished, its node sums in
-// acc[s * 4096 ..]; unit[u] = (slot, piece).  cap = 0: none.
+// acc[s * 4096 ..]; unit[u] = (slot, piece), or (-1, ..): nothing.  cap = 0:
+// none.  The lists are sized by the npart of the call; a tile whose pieces
+// would not fit (cell_start counts more records) is not cut.
 struct BigTiles {
   int32_t cap, ucap;
   int32_t *count, *tile, *np, *done;
@@ -131,11 +133,13 @@ __global__ void k_tile_dense(const int32_t *__restrict__ cell_start,
     if (s < B.cap) {
       const int32_t np = (n + DEP_PIECE - 1) / DEP_PIECE,
                     u = atomicAdd(&B.count[1], np);
+      const bool fits = u <= B.ucap - np;
       B.tile[s] = tile;
       B.np[s] = np;
       B.done[s] = 0;
-      for (int32_t i = 0; i < np; i++) B.unit[u + i] = make_int2(s, i);
-      f = 1;
+      for (int32_t i = 0; i < np && u + i < B.ucap; i++)
+        B.unit[u + i] = make_int2(fits ? s : -1, i);
+      f = fits;
     }
   }
   if (!f && n >= dense_tile) {
@@ -206,6 +210,7 @@ k_cic_deposit(const int32_t *__restrict__ cell_start,
   if ((int32_t)blockIdx.x < B.ucap) {
     if ((int32_t)blockIdx.x >= B.count[1]) return;
     const int2 u = B.unit[blockIdx.x];
+    if (u.x < 0) return;
     slot = u.x;
     piece = u.y;
     np = B.np[slot];
@@ -425,7 +430,9 @@ k_interp_split(const int32_t *__restrict__ cell_start, int32_t nblk,
 }
 
 // CIC^-1 of the block's own particles from its (8R+1)^3 nodes.  Workgroups
-// before ucap take the extra pieces; ucap = 0: no block is shared.
+// before ucap take the extra pieces; no block is shared where ucap = 0 or
+// where the pieces are more than ucap (cell_start counts more records than
+// the npart of the call, which sized the list).
 template <int R>
 __global__ void __launch_bounds__(256)
 k_cic_interp(const int32_t *__restrict__ cell_start,
@@ -440,8 +447,10 @@ k_cic_interp(const int32_t *__restrict__ cell_start,
   __shared__ float g[NN * NN * NN];
   const int32_t nb = nx >> 3;
   int32_t blk = (int32_t)blockIdx.x - ucap, piece = 0;
+  const int32_t nu = ucap > 0 ? ucount[0] : 0;
+  const bool shared = ucap > 0 && nu <= ucap;
   if (blk < 0) {
-    if ((int32_t)blockIdx.x >= ucount[0]) return;
+    if (!shared || (int32_t)blockIdx.x >= nu) return;
     const int2 u = unit[blockIdx.x];
     blk = u.x;
     piece = u.y;
@@ -462,7 +471,7 @@ k_cic_interp(const int32_t *__restrict__ cell_start,
   // in flight together rather than one after the other.
   const int32_t s0 = cell_start[blk * BS3] + piece * INT_CH,
                 sb = cell_start[blk * BS3 + BS3],
-                s1 = ucap > 0 ? min(sb, s0 + INT_CH) : sb;
+                s1 = shared ? min(sb, s0 + INT_CH) : sb;
   float4 r = make_float4(0.f, 0.f, 0.f, 0.f);
   int32_t h = -1;
   if (s0 + (int32_t)threadIdx.x < s1) {
