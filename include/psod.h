@@ -17,8 +17,9 @@
  *
  * Conventions: positions are float32 xyz triplets (Fortran posf(3,N)) in box
  * units [0,1).  Grids are x fastest: (iz*ng + iy)*ng + ix.  nx (SOD cells per
- * side) and ng (CIC nodes per side) are powers of two; nx >= 8.  npart <
- * 2^31.  Indices returned are 0-based except where a comment says 1-based.
+ * side) and ng (CIC nodes per side) are powers of two; nx >= 8.  npart <=
+ * PSOD_NPART_MAX wherever particles are sorted into cells, else < 2^31.
+ * Indices returned are 0-based except where a comment says 1-based.
  * A context is used by one host thread at a time.
  */
 #ifndef PSOD_H
@@ -42,6 +43,10 @@ extern "C" {
 
 #define PSOD_MAXDELTA 4
 #define PSOD_BLOCK 8        /* cells are stored in 8^3-cell blocks            */
+/* particles of a cell-sorted catalogue, at most: 2^31 - 2^16.  Records are
+ * indexed with 32 bits, and the kernels step past the end of a list by up to
+ * a few thousand records before they compare. */
+#define PSOD_NPART_MAX 2147418112LL
 
 typedef struct psod_ctx psod_ctx;
 

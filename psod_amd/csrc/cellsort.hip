@@ -871,8 +871,9 @@ extern "C" int psod_cell_sort(psod_ctx *ctx, int64_t npart, const float *d_pos,
                               const int32_t *d_labels, int32_t nx,
                               int32_t *d_cell_start, int32_t *d_perm,
                               float *d_rec, int32_t *d_lab_sorted) {
+  PSOD_TRY(psod_check_npart("psod_cell_sort", npart));
   PSOD_TRY(psod_use_device(ctx));
-  if (npart < 0 || npart >= (1ll << 31) || !d_pos || !d_cell_start || !d_rec)
+  if (npart < 0 || !d_pos || !d_cell_start || !d_rec)
     return psod_set_error(PSOD_E_ARG, "psod_cell_sort: bad arguments");
   if (nx < 8 || nx > 1024 || (nx & (nx - 1)))
     return psod_set_error(PSOD_E_ARG,

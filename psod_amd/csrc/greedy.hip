@@ -943,6 +943,7 @@ extern "C" int psod_host_spherover(psod_ctx *ctx, int64_t npart,
                                    double *rec_f64, double *rad_bins,
                                    int32_t *mass_bins, uint8_t *alive,
                                    int64_t *structure) {
+  PSOD_TRY(psod_check_npart("spherover", npart));
   PSOD_TRY(psod_use_device(ctx));
   if (!pos || !isort || !p || !nrec || npart <= 0 || npart_new < 0)
     return psod_set_error(PSOD_E_ARG, "spherover: bad arguments");

@@ -55,6 +55,7 @@ extern "C" int psod_pass(psod_ctx *ctx, const psod_sod_params *p,
                          const int64_t *d_ids, const int32_t *d_labels,
                          int64_t nhalo, float *d_grid,
                          const psod_halo_out *out) {
+  PSOD_TRY(psod_check_npart("psod_pass", npart));
   PSOD_TRY(psod_use_device(ctx));
   if (!p || !out || !d_pos || !d_labels || npart <= 0 || nhalo < 0)
     return psod_set_error(PSOD_E_ARG, "psod_pass: bad arguments");
@@ -185,6 +186,7 @@ extern "C" int psod_pass_graph(psod_ctx *ctx, const psod_sod_params *p,
                                const int64_t *d_ids, const int32_t *d_labels,
                                int64_t nhalo, float *d_grid,
                                const psod_halo_out *out, int32_t *replayed) {
+  PSOD_TRY(psod_check_npart("psod_pass_graph", npart));
   PSOD_TRY(psod_use_device(ctx));
   if (replayed) *replayed = 0;
   if (!p || !out || !d_pos || !d_labels || npart <= 0 || nhalo < 0)

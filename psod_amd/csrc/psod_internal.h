@@ -28,6 +28,13 @@ int psod_set_error(int code, const char *fmt, ...);
 
 #define PSOD_LAUNCH_CHECK() PSOD_HIP(hipGetLastError())
 
+// Refuses counts beyond PSOD_NPART_MAX, before anything is allocated.
+inline int psod_check_npart(const char *who, int64_t npart) {
+  if (npart <= PSOD_NPART_MAX) return PSOD_OK;
+  return psod_set_error(PSOD_E_ARG, "%s: %lld particles, at most %lld", who,
+                        (long long)npart, (long long)PSOD_NPART_MAX);
+}
+
 // ---------------------------------------------------------------------------
 // context: one device, one stream, growable scratch slots
 // ---------------------------------------------------------------------------

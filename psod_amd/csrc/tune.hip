@@ -129,6 +129,7 @@ extern "C" int psod_autotune(psod_ctx *ctx, const psod_sod_params *p,
                              const int32_t *d_labels, int64_t nhalo,
                              int32_t reps, const char *cache_file,
                              psod_tunables *chosen, double *stage_ms) {
+  PSOD_TRY(psod_check_npart("psod_autotune", npart));
   PSOD_TRY(psod_use_device(ctx));
   if (!p || !d_pos || !d_labels || npart <= 0 || nhalo <= 0 || p->nx != nx)
     return psod_set_error(PSOD_E_ARG, "psod_autotune: bad arguments");
