@@ -413,7 +413,16 @@ k_cic_deposit(const int32_t *__restrict__ cell_start,
 // at 512^3 2.30 -> 0.87 ms, 1024^3 8.5 -> 6.9, 128^3 70 -> 21 us, with the
 // keys below (pieces of 2^14: 35 us at 128^3).
 constexpr int32_t INT_CH = 1 << 12;
-// below this the list costs more than an uneven launch (one more kernel)
+// From 2^21 particles on.  The list costs two short launches and the idle
+// workgroups of its capacity, 4-7 us; what it saves depends on the densest
+// block, which the host does not know.  Calls with seed keys, us without / with
+// it, at 128^3 cells: uniform 45.3 / 51.3 (1.0e6 particles), 50.7 / 57.4 (2.1e6);
+// clumps of at most 1% of the particles 47.4 / 50.7 (8e5), 50.7 / 54.2 (1.0e6),
+// 53.0 / 55.9 (1.6e6), 66.5 / 60.2 (2.1e6, 15643 records in the densest block);
+// 5% in one halo 52.2 / 54.7 (1.0e6), 59.1 / 56.8 (1.6e6), 67.5 / 60.0 (2.1e6).
+// Blocks above about 10^4 records pay for it at any count (30% in one halo:
+// 2.6e5 58.1 / 56.7, 1.0e6 102 / 71; half of 2.1e6 221 / 66): the line is where
+// ordinary catalogues have them.
 constexpr int64_t INT_SPLIT_MIN = 1 << 21;
 __global__ void __launch_bounds__(256)
 k_interp_split(const int32_t *__restrict__ cell_start, int32_t nblk,
