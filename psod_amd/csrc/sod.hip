@@ -124,6 +124,7 @@ k_plan(SodCfg c, int64_t nhalo, const int32_t *__restrict__ seed,
   const int l = threadIdx.x & 63;
   const int64_t h = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
   if (h >= nhalo) return;  // uniform per wave
+  if (h == 0 && l == 0) counters[38] = cell_start[(int64_t)c.nx * c.nx * c.nx];
   HaloPlan pl;
   pl.seed = seed[h];
   pl.nmem = nmem ? nmem[h] : 0;
@@ -4666,7 +4667,7 @@ static int32_t pilot_big() {
 // read the counts on the device.  counters[36] is set when that pass's
 // tasks exceed the capacity (the host then runs the pass without the
 // graph), counters[37] holds the large-halo count before the small path's
-// deferrals.
+// deferrals, counters[38] the records that cell_start counts.
 struct SodCounts {
   bool dev;         // counts on the device only (captured pass)
   int32_t nlarge1;  // large halos of the plan (eager)
@@ -4677,15 +4678,17 @@ struct SodCounts {
 // dn, the first *dn of at most nlarge): tasks of 64 candidates, their
 // bounds, pilots, groups, and each halo's centre in plan[].centre.  ntask,
 // task0 and ntot are scratch of nlarge + 16 entries (ntot: 16); hbest
-// holds 2 * nlarge + 4 entries.  after_setup() is called once the task
-// count is known, before the search's kernels are queued.
+// holds 2 * nlarge + 4 entries.  nrec: records that cell_start counts.
+// after_setup() is called once the task count is known, before the search's
+// kernels are queued.
 template <typename F>
 static int centre_search(psod_ctx *ctx, const SodCfg &c,
                          const psod_catalogue *cat, HaloPlan *plan,
                          const int32_t *large, int32_t nlarge,
                          const int32_t *dn, int32_t *overflow, int32_t *ntask,
                          int32_t *task0, int32_t *ntot,
-                         unsigned long long *hbest, F &&after_setup) {
+                         unsigned long long *hbest, int64_t nrec,
+                         F &&after_setup) {
   hipStream_t st = ctx->stream;
   k_task_count<<<grid_for(nlarge, 4), 256, 0, st>>>(c, cat->cell_start, plan,
                                                      large, nlarge, dn, ntask);
@@ -4758,9 +4761,9 @@ static int centre_search(psod_ctx *ctx, const SodCfg &c,
       nb = 4;
     return (unsigned)ctx->num_cus * (unsigned)nb;
   };
-  // 2 bytes per particle: the windows of 8 records
+  // 2 bytes per record: the windows of 8
   float4 *gwin = (float4 *)psod_scratch(
-      ctx, S_WIN, (size_t)(cat->npart / 8 + 2) * sizeof(float4));
+      ctx, S_WIN, (size_t)(nrec / 8 + 2) * sizeof(float4));
   if (!gwin) return PSOD_E_NOMEM;
   k_centre_windows<<<grid_for((int64_t)nlarge * WIN_WAVES, 4), 256, 0, st>>>(
       c, cat->cell_start, (const float4 *)cat->rec, plan, large, nlarge, dn,
@@ -4992,15 +4995,19 @@ static int sod_fof_queue(psod_ctx *ctx, const psod_sod_params *p,
   // ones it defers (their centre found) behind them
   int32_t nlarge1 = (int32_t)nhalo;  // a bound in the device-count mode
   const int32_t *dn1 = nullptr;
+  // records of the catalogue: what cell_start counts (a caller's npart may be
+  // another; the pass's own is the same, and nothing is read back there)
+  int64_t nrec = cat->npart;
   if (dev) {
     k_copy_i32<<<1, 64, 0, st>>>(counters + 1, counters + 37);
     PSOD_LAUNCH_CHECK();
     dn1 = counters + 37;
   } else {
-    int32_t hc[4];
-    PSOD_HIP(hipMemcpyAsync(hc, counters, 16, hipMemcpyDeviceToHost, st));
+    int32_t hc[40];
+    PSOD_HIP(hipMemcpyAsync(hc, counters, 160, hipMemcpyDeviceToHost, st));
     PSOD_HIP(hipStreamSynchronize(st));
     nlarge1 = hc[1];
+    nrec = hc[38];
   }
   // Small halos, persistent (a few workgroups per CU), on the side stream:
   // they overlap the centre search of the large halos, which touches other
@@ -5041,7 +5048,7 @@ static int sod_fof_queue(psod_ctx *ctx, const psod_sod_params *p,
     PSOD_TRY(size_order(nlarge1, dn1, 0));
     PSOD_TRY(centre_search(ctx, c, cat, plan, large, nlarge1, dn1,
                            counters + 36, S->ntask, S->task0, S->ntot,
-                           S->hbest, launch_small));
+                           S->hbest, nrec, launch_small));
   } else {
     PSOD_TRY(launch_small());
   }
