@@ -690,8 +690,6 @@ k_cs_big_place(const int32_t *__restrict__ gs, int g, int32_t nx,
   }
 }
 
-int psod_fill_i32(psod_ctx *c, int32_t *p, int64_t n, int32_t v);
-
 // ---------------------------------------------------------------------------
 // Dense cells (>= 64 particles) are reordered by the Morton key of the
 // particle's 1/8-cell sub-cell, so that any 64 consecutive particles of a

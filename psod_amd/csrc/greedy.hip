@@ -593,7 +593,6 @@ struct GrowLds {
   uint32_t ord[GS_CAP];
   int32_t hist[GS_BINS];
   int64_t red_l[GG_T / 64];
-  double red_d[GG_T / 64];
   int32_t n;
 };
 

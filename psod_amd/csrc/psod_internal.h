@@ -66,9 +66,10 @@ enum ScratchSlot {
   S_GREEDY2,
   S_GREEDY3,
   S_TILE,      // deposit tile counts and dispatch order
-  S_CS_A,      // cell sort: records, block ids, labels (two buffers)
-  S_CS_C,
-  S_CS_H,      // cell sort: bucket tables and tile histograms
+  S_CS_A,      // cell sort, first pass: raw positions with indices, labels,
+               // 16-bit block keys
+  S_CS_C,      // the same after the second pass, without keys
+  S_CS_H,      // cell sort: digit counts, starts, chunks of the buckets
   S_PASS_CS,   // psod_pass: cell offsets, records, labels, halo arrays, grid
   S_PASS_REC,
   S_PASS_LAB,
