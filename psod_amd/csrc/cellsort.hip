@@ -83,11 +83,11 @@ __device__ inline int32_t block_of(const float4 &v, int32_t nx) {
 // matter, so no per-tile counts are kept, and a digit's runs of successive
 // chunks are neighbours in memory.
 //
-// At 1024^3 the sort takes 34 ms (hist 2.4, scatter 10.4, hist 1.0, scatter
-// 8.9, final 7.0-8.4, large groups 3.7, subsort 1.7); three passes of 7 bits with
+// At 1024^3 the sort takes 37.0 ms (hist 2.4, scatter 10.6, hist 1.0, scatter
+// 9.0, final 8.4, large groups 3.8, subsort 1.7); three passes of 7 bits with
 // per-tile counts and a block sort took 55.  What bounds it is HBM: a pass
-// moves 40 bytes per particle (4.1-4.9 TB/s in the scatters, 5.3 in k_cs_final).  A chunk's run
-// of one digit is short (CH / 2^bits elements, 4 to 16), so its first and
+// moves 40 bytes per particle (4.1-5.2 TB/s in the scatters, 4.8 in
+// k_cs_final).  A chunk's run of one digit is short (CH / 2^bits elements, 4 to 16), so its first and
 // last 128-byte lines are partial, and so are most lines of the 4-byte
 // labels.  They reach memory whole when the neighbouring runs are written
 // through the same L2 soon after: each XCD has its own L2, and workgroups go

@@ -180,7 +180,8 @@ __device__ inline float clamp01(float x) {
 // (v_rndne) and an FP64 add onto 2^52: the low bits of the sum are the
 // integer sum, exact up to 2^16 unit weights, and leave the register by one
 // 64-bit subtraction.  Bound by VALU issue (85 %) and the LDS atomics
-// together, at 1.9 TB/s of records and nodes: 1024^3 8.66 -> 8.0 ms, zoom
+// together, at 2.1 TB/s of positions and nodes (12 bytes a particle, 4 a node;
+// 4.0 TB/s of what it moves): 1024^3 8.66 -> 8.1 ms, zoom
 // catalogue at 512^3 (with the pieces) 2.66 -> 1.10 ms, 256^3 on 512^3 nodes
 // 0.42 -> 0.40 ms.  Slower at 1024^3: a margin of nodes in LDS instead of the
 // bounds checks (9.2: fewer waves fit), 2, 3 or 8 particles per lane (9.0,

@@ -17,11 +17,16 @@
 // that each spread one step over the GPU: gather (one workgroup per seed),
 // centre search (64 candidates per workgroup), growth (one workgroup per
 // seed, keys sorted in LDS).  One workgroup per seed for everything took
-// 5.2 ms a round, 353 ms for the 66 rounds of the 128^3 catalogue: FP64
+// 5.2 ms a round, 290-350 ms for the 66 rounds of the 128^3 catalogue: FP64
 // square roots and divisions of every candidate pair on one CU, then a
 // bitonic sort of all gathered particles in global memory.  The staged
-// rounds take 7.8 ms with the transfers; what is left is the chain of six
-// short launches per round.
+// rounds, at most 24 there (smaller marking blocks let more seeds run side by
+// side), take 7.2 ms with the transfers: 3.3 of it kernels, the rest pageable
+// copies and the waits.
+//
+// A seed that fails ends the zone at its place in the order: the seeds
+// before it run on, and where seeds after it had run too, those before it
+// run a second time by themselves.
 #include <algorithm>
 #include <cmath>
 #include <cstring>

@@ -1743,8 +1743,8 @@ __constant__ int8_t kCellOrder[27] = {13, 4,  10, 12, 14, 16, 22, 1,  3,
 // candidate's exact sum so far plus that reaches the halo's best.  On
 // sampled halos (n5 5e3..8e4) an item needs 35% of its neighbours; checked
 // at the ends of the cells, against bounds kept per cell, 46%.  The pair
-// tests run at the issue rate of their 13 instructions, so fewer of them is
-// what helps.  Taking the neighbours in shells of distance (windows by
+// tests issue 1.00 VALU instructions per CU and cycle (the bound 1.25) with
+// an LDS read per 64 of them, 13 instructions a test.  Taking the neighbours in shells of distance (windows by
 // their centre, 3 or 5 shells) needs 23-30% of them, but its window tests
 // and its registers cost what that saves (1024^3 36.9 ms against 39.7, zoom
 // catalogue at 512^3 11.5 against 9.6, 256^3 1.00 against 0.86; bounds per
